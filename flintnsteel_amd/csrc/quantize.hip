@@ -106,8 +106,9 @@ __global__ __launch_bounds__(256) void k_amax_guard_q8_1(const float *__restrict
     }
 }
 
-// The same for rows of at most 256 C padded columns: each thread's C values are loaded once, all in flight together
-// (clamped, unconditional loads), and quantised from registers; same operations, same bits.
+// The same for rows of exactly 256 C padded columns (every column below 256 C is stored): each thread's C values are
+// loaded once, all in flight together (clamped, unconditional loads), and quantised from registers; same operations,
+// same bits.
 template <int C>
 __global__ __launch_bounds__(256) void k_amax_guard_q8_1_reg(const float *__restrict__ act, float *__restrict__ escale,
                                                              uint8_t *__restrict__ xq, int n, int64_t row_bytes) {
@@ -217,6 +218,8 @@ int amax_guard_q8_1(const float *act, float *escale, void *xq, int n, int rows, 
         hipLaunchKernelGGL(k_amax_guard_q8_1_reg<2>, dim3((unsigned) rows), dim3(256), 0, st, act, escale, (uint8_t *) xq, n, rb);
     else if (npad <= 1024)
         hipLaunchKernelGGL(k_amax_guard_q8_1_reg<4>, dim3((unsigned) rows), dim3(256), 0, st, act, escale, (uint8_t *) xq, n, rb);
+    else if (npad <= 1536)
+        hipLaunchKernelGGL(k_amax_guard_q8_1_reg<6>, dim3((unsigned) rows), dim3(256), 0, st, act, escale, (uint8_t *) xq, n, rb);
     else if (npad <= 2048)
         hipLaunchKernelGGL(k_amax_guard_q8_1_reg<8>, dim3((unsigned) rows), dim3(256), 0, st, act, escale, (uint8_t *) xq, n, rb);
     else

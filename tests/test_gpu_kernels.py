@@ -277,6 +277,24 @@ def test_amax_guard_q8_1(ops, n):
     assert np.array_equal(host(a2), (act / ref_e[:, None]).astype(np.float32))
 
 
+@pytest.mark.parametrize("n", [1056, 1280, 1536])
+def test_amax_guard_q8_1_stays_in_its_rows(ops, n):
+    """Rows of 1025 to 1536 columns (padded to 1536): every row's bytes are its own, and nothing is written past the
+    last row."""
+    rng = np.random.default_rng(40 + n)
+    rows = 5
+    act = gaussian(rng, (rows, n), 0.5)
+    ref = orc.quantize_q8_1(act)
+    buf = torch.full((ref.size + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    from flintnsteel_amd.ops import _p, _s, call
+    import ctypes
+    a, e = dev(act), torch.empty(rows, device="cuda")
+    call("fns_hip_amax_guard_q8_1", _p(a), _p(e), ctypes.c_void_p(buf.data_ptr()), n, rows, _s())
+    got = host(buf)
+    assert np.array_equal(got[: ref.size].reshape(ref.shape), ref)
+    assert (got[ref.size:] == 0x5A).all()
+
+
 def test_swiglu_epilogues(ops):
     rng = np.random.default_rng(2)
     g = gaussian(rng, (4, F), 3.0)
