@@ -64,6 +64,9 @@ size_t mmq_image_bytes(int64_t ncols);
 size_t mmq_q8_1_bytes(int64_t ncols, int64_t nrows);
 size_t mmq_bounds_bytes(int64_t n_expert);
 int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, void *xpack, hipStream_t st);
+bool mmq_rms_norm_image_fits(const float *x, const float *w, const float *out, int64_t n);
+int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, void *ximg,
+                       hipStream_t st);
 int mmq_quant_image_scaled(const float *x, const float *escale, int64_t ncols, int64_t rows, void *xpack, int64_t stride,
                            hipStream_t st);
 int mmq_compact(const int32_t *ids, int64_t n_tok, int64_t k, int64_t n_expert, int64_t x_rows_per_tok,

@@ -30,6 +30,7 @@
 #include "fns_host.hpp"
 #include "fns_internal.hpp"
 #include "fns_lanes.hpp"
+#include "fns_q8x8.hpp"
 #include "fns_quarter.hpp"
 #include "fns_router_gemm.hpp"
 
@@ -217,22 +218,14 @@ struct Q8Split {
     _Float16 hi[8], lo[8];  // in the stored order
     _Float16 shi, slo;      // the block's min-term sum (lane q = 0 of the block stores it)
 };
-template <bool EXACT>
-__device__ __forceinline__ Q8Split q8_split8_vals(const float (&v)[8]) {
+// the split of eight codes of a block with scale dh (an f16 value)
+__device__ __forceinline__ Q8Split q8_split_of(const int (&q)[8], float dh) {
     Q8Split r;
-    float amax = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[k]));
-    amax = lanes_max<4>(amax);
-    const float d = amax / 127.0f;
-    const float dh = half_to_float(float_to_half(d));
-    const float id = amax == 0.0f ? 0.0f : 1.0f / d;
     int qsum = 0;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        const int qk = amax == 0.0f ? 0 : (int) (int8_t) roundf(EXACT ? v[k] / d : v[k] * id);
-        qsum += qk;
-        const float x = (float) qk * dh;  // exact
+        qsum += q[k];
+        const float x = (float) q[k] * dh;  // exact
         const _Float16 h = (_Float16) x;
         r.hi[perm8(k)] = h;
         r.lo[perm8(k)] = (_Float16) (x - (float) h);
@@ -243,6 +236,20 @@ __device__ __forceinline__ Q8Split q8_split8_vals(const float (&v)[8]) {
     r.slo = (_Float16) (sv - (float) r.shi);
     return r;
 }
+template <bool EXACT>
+__device__ __forceinline__ Q8Split q8_split8_vals(const float (&v)[8]) {
+    float amax = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[k]));
+    amax = lanes_max<4>(amax);
+    const float d = amax / 127.0f;
+    const float dh = half_to_float(float_to_half(d));
+    const float id = amax == 0.0f ? 0.0f : 1.0f / d;
+    int q[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) q[k] = amax == 0.0f ? 0 : (int) (int8_t) roundf(EXACT ? v[k] / d : v[k] * id);
+    return q8_split_of(q, dh);
+}
 // byte offsets within an image row of the 8 columns at col (hi; lo at + 256) and of the block's min-term sums (hi;
 // lo at + 16)
 __device__ __forceinline__ uint32_t img_col_off(int col) {
@@ -251,10 +258,7 @@ __device__ __forceinline__ uint32_t img_col_off(int col) {
 __device__ __forceinline__ uint32_t img_sum_off(int ncols, int col) {
     return (uint32_t) ((ncols >> 8) * kSbMain + (col >> 8) * kSbMin + 2 * perm8((col >> 5) & 7));
 }
-template <bool EXACT>
-__device__ __forceinline__ void q8_split8(const float (&v)[8], uint8_t *row, int ncols, int col, bool store) {
-    const Q8Split r = q8_split8_vals<EXACT>(v);
-    if (!store) return;
+__device__ __forceinline__ void q8_split_store(const Q8Split &r, uint8_t *row, int ncols, int col) {
     uint8_t *o = row + img_col_off(col);
     *(uint4 *) o = __builtin_bit_cast(uint4, r.hi);
     *(uint4 *) (o + 256) = __builtin_bit_cast(uint4, r.lo);
@@ -263,6 +267,11 @@ __device__ __forceinline__ void q8_split8(const float (&v)[8], uint8_t *row, int
         m[0] = r.shi;
         m[8] = r.slo;
     }
+}
+template <bool EXACT>
+__device__ __forceinline__ void q8_split8(const float (&v)[8], uint8_t *row, int ncols, int col, bool store) {
+    const Q8Split r = q8_split8_vals<EXACT>(v);
+    if (store) q8_split_store(r, row, ncols, col);
 }
 
 // x [rows][ncols] f32 -> split image rows with the reference's Q8_1 arithmetic; grid (ceil(ncols / 2048), rows), 256
@@ -275,6 +284,21 @@ __global__ __launch_bounds__(256) void k_quant_image(const float *__restrict__ x
     const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
     const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
     q8_split8<true>(v, out + (size_t) row * img_row_bytes, ncols, col, true);
+}
+
+// RMSNorm of a row of at most 2048 C columns (fns_q8x8.hpp) with its Q8_1 blocks and its split image row, as
+// rms_norm_q8_1 and k_quant_image give them, in one pass over x.
+template <int C>
+__global__ __launch_bounds__(256) void k_rms_norm_image(const float *__restrict__ x, const float *__restrict__ w,
+                                                        float *__restrict__ out, uint8_t *__restrict__ xq, int n,
+                                                        float eps, int64_t row_bytes, uint8_t *__restrict__ img,
+                                                        int64_t img_row_bytes) {
+    __shared__ __align__(16) float xs[2048 * C];
+    const size_t r = blockIdx.x;
+    uint8_t *row = img + r * img_row_bytes;
+    rms_norm_row<C>(x + r * n, w, out + r * n, xq + r * row_bytes, n, eps, xs, [&](const Q8x8 &q, int col) {
+        q8_split_store(q8_split_of(q.q, half_to_float(float_to_half(q.d))), row, n, col);
+    });
 }
 
 // F16-guard form: only the rows whose guard scale is not 1 are re-quantised (the others already hold the image of
@@ -1364,6 +1388,26 @@ int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, void *xpack, hi
     return host::check_launch("mmq quantize");
 }
 
+// RMSNorm of x (f32 [rows][n]) into out, its Q8_1 blocks into xq (null: none) and its split image rows into ximg, for
+// rows that mmq_rms_norm_image_fits: at most 8192 columns, 16-byte aligned arrays.
+bool mmq_rms_norm_image_fits(const float *x, const float *w, const float *out, int64_t n) {
+    return n > 0 && n % 256 == 0 && n <= 8192 && (((uintptr_t) x | (uintptr_t) w | (uintptr_t) out) & 15) == 0;
+}
+int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, void *ximg,
+                       hipStream_t st) {
+    if (!x || !w || !out || !ximg || rows < 0 || !mmq_rms_norm_image_fits(x, w, out, n))
+        return host::set_error(host::ERR_SHAPE, "mmq rms_norm: bad arguments");
+    if (rows == 0) return host::OK;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned) rows), dim3(256), 0, st, x, w, out, (uint8_t *) xq, n, eps,
+                           host::q8_1_row_bytes(n), (uint8_t *) ximg, (int64_t) mmq_image_bytes(n));
+    };
+    if (n <= 2048) go(k_rms_norm_image<1>);
+    else if (n <= 4096) go(k_rms_norm_image<2>);
+    else go(k_rms_norm_image<4>);
+    return host::check_launch("mmq rms_norm");
+}
+
 int mmq_quant_image_scaled(const float *x, const float *escale, int64_t ncols, int64_t rows, void *xpack,
                            int64_t stride, hipStream_t st) {
     if (!x || !escale || !xpack || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
@@ -1671,11 +1715,17 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     const char *const *table = (const char *const *) L->table;
 
     // RMSNorm first when the layer has one: the router and the experts read h (reference src/engine.cu:331)
+    bool have_img = false;  // the RMSNorm kernel has built the activation image
     if (L->ffn_norm) {
-        FNS_TRY(rms_norm_q8_1(x, L->ffn_norm, (float *) sec[11], sec[12], (int) L->hidden, L->norm_eps, (int) n_tok, st));
-        x = (const float *) sec[11];
+        float *h = (float *) sec[11];
+        have_img = mmq_rms_norm_image_fits(x, L->ffn_norm, h, L->hidden);
+        if (have_img)
+            FNS_TRY(mmq_rms_norm_image(x, L->ffn_norm, h, sec[12], (int) L->hidden, L->norm_eps, (int) n_tok, sec[3], st));
+        else
+            FNS_TRY(rms_norm_q8_1(x, L->ffn_norm, h, sec[12], (int) L->hidden, L->norm_eps, (int) n_tok, st));
+        x = h;
     }
-    // the router GEMM and the activation image in one launch when the GEMM takes its unguarded path (whole 64-column
+    // the router GEMM and the activation image (unless the RMSNorm built it) in one launch when the GEMM takes its unguarded path (whole 64-column
     // chunks, aligned rows, 32-bit offsets), else as two launches
     const int H = (int) L->hidden, NE = (int) L->n_expert;
     const bool bf = L->router_dtype == T_BF16;
@@ -1684,7 +1734,7 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     if (one) {
         const int tiles_x = (int) ((n_tok + 15) / 16), n_rt = tiles_x * ((NE + 15) / 16);
         const int nxb = (H + 2047) / 2048;
-        const int64_t n_img = (nxb * n_tok + 1) / 2;
+        const int64_t n_img = have_img ? 0 : (nxb * n_tok + 1) / 2;
         if (n_rt + n_img > INT32_MAX) return host::set_error(host::ERR_SHAPE, "prefill: grid too large");
         const dim3 g((unsigned) (n_rt + n_img));
         if (bf)
@@ -1697,7 +1747,7 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     } else {
         FNS_TRY(gemm_router_bias(L->router_dtype, L->router_w, L->router_bias, x, logits, L->hidden, L->n_expert,
                                  (int) n_tok, st));
-        FNS_TRY(mmq_quant_image(x, L->hidden, n_tok, sec[3], st));
+        if (!have_img) FNS_TRY(mmq_quant_image(x, L->hidden, n_tok, sec[3], st));
     }
     FNS_TRY(route_topk(logits, ids, w, L->n_expert, L->k, (int) n_tok, L->gating, L->norm_w, st));
     // gate/up (SwiGLU and the Q8_1 of act fused) and down: act image rows padded to whole cache lines; one launch

@@ -11,6 +11,7 @@
 #include "fns_common.hpp"
 #include "fns_host.hpp"
 #include "fns_internal.hpp"
+#include "fns_q8x8.hpp"
 
 namespace fns {
 
@@ -32,6 +33,17 @@ __global__ __launch_bounds__(256) void k_quantize_q8_1(const float *__restrict__
     const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
     const float v = i < ncols ? x[r * ncols + i] : 0.0f;
     q8_1_store(v, xq + r * row_bytes, (int) (i / 32), (int) (i % 32));
+}
+
+// RMSNorm of a row of at most 2048 C columns, then its Q8_1 (fns_q8x8.hpp): one row per workgroup, every load issued at
+// the start. Latency-bound (one row is 16 KB); the form below waits for each of its n / 256 loads in turn.
+template <int C>
+__global__ __launch_bounds__(256) void k_rms_norm_q8_1_rows(const float *__restrict__ x, const float *__restrict__ w,
+                                                            float *__restrict__ out, uint8_t *__restrict__ xq, int n,
+                                                            float eps, int64_t row_bytes) {
+    __shared__ __align__(16) float xs[2048 * C];
+    const size_t r = blockIdx.x;
+    rms_norm_row<C>(x + r * n, w, out + r * n, xq + r * row_bytes, n, eps, xs, [](const Q8x8 &, int) {});
 }
 
 // RMSNorm of one row (any n that is a multiple of 32) then Q8_1 of the result; one workgroup per row.
@@ -197,8 +209,16 @@ int rms_norm_q8_1(const float *x, const float *w, float *out, void *xq, int n, f
     if (!x || !w || !out || !xq || n <= 0 || n % 32 || rows < 0)
         return host::set_error(host::ERR_SHAPE, "rms_norm_q8_1: n must be a positive multiple of 32");
     if (rows == 0) return host::OK;
-    hipLaunchKernelGGL(k_rms_norm_q8_1, dim3((unsigned) rows), dim3(256), 0, st, x, w, out, (uint8_t *) xq, n, eps,
-                       host::q8_1_row_bytes(n));
+    // the register form: rows of at most 8192 columns, 16-byte loads and stores (n % 32 == 0 keeps every row aligned)
+    const bool vec = n <= 8192 && (((uintptr_t) x | (uintptr_t) w | (uintptr_t) out) & 15) == 0 && ((uintptr_t) xq & 3) == 0;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned) rows), dim3(256), 0, st, x, w, out, (uint8_t *) xq, n, eps,
+                           host::q8_1_row_bytes(n));
+    };
+    if (!vec) go(k_rms_norm_q8_1);
+    else if (n <= 2048) go(k_rms_norm_q8_1_rows<1>);
+    else if (n <= 4096) go(k_rms_norm_q8_1_rows<2>);
+    else go(k_rms_norm_q8_1_rows<4>);
     return host::check_launch("rms_norm_q8_1");
 }
 

@@ -141,6 +141,24 @@ def test_flint_block_prefill(ops, layer, mats):
     assert_close_chain(out[toks], ref, "flint block prefill")
 
 
+def test_flint_block_prefill_norm_image(ops, layer):
+    """The prefill's RMSNorm output, its Q8_1 blocks and the activation image built in the same pass equal the
+    standalone kernel's output, blocks and the image those blocks define."""
+    from flintnsteel_amd import synth
+    from tests.helpers import split_image
+    T = 3
+    pre = ops.MoePrefill(layer)
+    x = synth.activations(T, H, SEED, layer=36)
+    ws = pre.workspace(T)
+    pre(x, ws=ws, x_resid=x)
+    h, xq = (host(t) for t in ops.rms_norm_q8_1(x, layer.ffn_norm, 1e-6))
+    o11, n11 = pre.section(T, 11)
+    o12, n12 = pre.section(T, 12)
+    assert np.array_equal(host(ws[o11:o11 + n11]).view(np.float32).reshape(T, H), h)
+    assert np.array_equal(host(ws[o12:o12 + n12]).reshape(T, -1), xq)
+    assert np.array_equal(host(pre.trace(ws, T)["xpack"]), split_image(xq, H))
+
+
 def test_flint_block_shared_types_differ(ops, layer, mats):
     """A shared expert whose types differ from the routed ones (Q6_K gate/up, Q4_K down) is not fused into the decode
     kernel: the dense-mode gate/up and down kernels compute it, at one token and at four."""

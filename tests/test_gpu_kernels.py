@@ -72,6 +72,24 @@ def test_rms_norm_q8_1(ops):
     assert np.array_equal(host(xq), orc.quantize_q8_1(out_h))
 
 
+@pytest.mark.parametrize("n", [32, 96, 544, 2048, 2080, 4096, 4128, 8192, 8224])
+def test_rms_norm_q8_1_row_widths(ops, n):
+    """The register form (up to 8192 columns, aligned) at the edges of its 2048-column chunks and the loop form beyond
+    give the same bits: an x that is not 16-byte aligned takes the loop form."""
+    rng = np.random.default_rng(70 + n)
+    rows = 3
+    x, w = gaussian(rng, (rows, n)), gaussian(rng, (n,), 1.0)
+    out, xq = ops.rms_norm_q8_1(dev(x), dev(w), 1e-6)
+    out_h = host(out)
+    ref = x.astype(np.float64) / np.sqrt((x.astype(np.float64) ** 2).mean(1, keepdims=True) + 1e-6) * w
+    assert_close(out_h, ref, "rms_norm", 1e-5, 1e-6)
+    assert np.array_equal(host(xq), orc.quantize_q8_1(out_h))
+    off = torch.empty(rows * n + 1, device="cuda")[1:].view(rows, n)
+    off.copy_(dev(x))
+    out2, xq2 = ops.rms_norm_q8_1(off, dev(w), 1e-6)
+    assert np.array_equal(host(out2), out_h) and np.array_equal(host(xq2), host(xq))
+
+
 # ---- expert GEMVs -----------------------------------------------------------------------------------------------
 
 @pytest.fixture(scope="module")
