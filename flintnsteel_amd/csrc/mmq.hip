@@ -368,6 +368,20 @@ struct MmqArgs {
     uint32_t *status;          // fused launch: sticky status word, kStatusTimeout once a wait gave up
 };
 
+// One dense matrix that rides in the expert launch (a layer's shared expert, of the routed experts' type): its groups
+// of 64 activation rows x row blocks take the first workgroups of the grid. n_rows = 0: none.
+struct MmqShared {
+    const uint8_t *w;
+    int64_t off_b;             // GLU: the up matrix from w (the gate)
+    int ncols, nrows, n_rows;
+    const uint8_t *xpack;      // activation image rows (x_img bytes each), row t of every group in order
+    int64_t x_img;
+    float *dst;                // non-GLU
+    uint8_t *out_pack;         // GLU
+    int64_t out_img;
+    int n_cb, items;           // launch: row blocks per group; workgroups of the grid it takes (a multiple of kXcds)
+};
+
 // Weight fragments of one 256-value block for one lane: the header (scales, d) and the codes of column groups
 // kg = 2 h and 2 h + 1 (h = lane / 32) of every sub-block - 16 contiguous bytes per code array, one load each.
 template <int T> struct WFrag;
@@ -1171,28 +1185,52 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
 // (SPX mode: one partition of all 8 XCDs. In a partitioned mode the mapping is a performance assumption only.)
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 template <int T, bool GLU>
-__global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mmq(const MmqArgs a) {
+__global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mmq(const MmqArgs m,
+                                                                                            const MmqShared sh) {
     __shared__ __align__(16) uint8_t sh_a0[kMmqTok * kRowA];
     __shared__ __align__(16) uint8_t sh_a1[kMmqTok * kRowA];
     __shared__ __align__(16) uint8_t sh_s[(T == T_Q4_K || T == T_Q5_K) ? kMmqTok * kRowS : 16];
     __shared__ __align__(16) uint32_t sh_grid[kGridWords<T> > 0 ? kGridWords<T> : 4];
     __shared__ int sh_src[kMmqTok], sh_dst[kMmqTok], sh_grp[4];
     const MmqLds L{sh_a0, sh_a1, *(uint8_t (*)[kMmqTok * kRowS]) sh_s, sh_src, sh_dst, sh_grp, sh_grid};
-    const int lid = blockIdx.x, r = lid / kXcds;
-    int j = (r / a.n_cb) * kXcds + lid % kXcds;
-    const int wb = r % a.n_cb;
-    if (a.bounds) {
+    MmqArgs a = m;
+    const bool shared = (int) blockIdx.x < sh.items;
+    const int lid = shared ? (int) blockIdx.x : (int) blockIdx.x - sh.items, r = lid / kXcds;
+    const int n_cb = shared ? sh.n_cb : m.n_cb;
+    const int j = (r / n_cb) * kXcds + lid % kXcds, wb = r % n_cb;
+    bool one = false;  // a group of at most 32 rows: one token tile
+    int g = j;
+    if (shared) {
+        a.table = nullptr;
+        a.w_dense = sh.w;
+        a.off_a = 0;
+        a.off_b = sh.off_b;
+        a.ncols = sh.ncols;
+        a.nrows = sh.nrows;
+        a.xpack = sh.xpack;
+        a.x_img = sh.x_img;
+        a.bounds = a.src = a.dst_rows = nullptr;
+        a.n_rows = sh.n_rows;
+        a.dst = sh.dst;
+        a.out_pack = sh.out_pack;
+        a.out_img = sh.out_img;
+        a.act_out = nullptr;
+        if (kMmqTok * j >= sh.n_rows) return;
+        one = sh.n_rows - kMmqTok * j <= kMmqTok / 2;
+        if (one) g = 2 * j;
+    } else if (m.bounds) {
         // expert path: the groups that exist in this call (the device-side counts of the 64-row list and of the
         // remainder list) take the first workgroups; the rest of the grid (sized for the upper bound) returns at once
-        const int nm = a.gprefix[a.n_expert], nr = a.gprefix[2 * (a.n_expert + 1) - 1];
+        const int nm = m.gprefix[m.n_expert], nr = m.gprefix[2 * (m.n_expert + 1) - 1];
         if (j >= nm + nr) return;
-        if (j < nm) mmq_group<T, GLU, 2, false>(a, j, wb, L);
-        else mmq_group<T, GLU, 1, false>(a, j - nm, wb, L);
-        return;
+        one = j >= nm;
+        if (one) g = j - nm;
+    } else {
+        if (j >= m.n_groups) return;
+        one = m.dense_small != 0;
     }
-    if (j >= a.n_groups) return;
-    if (a.dense_small) mmq_group<T, GLU, 1, false>(a, j, wb, L);
-    else mmq_group<T, GLU, 2, false>(a, j, wb, L);
+    if (one) mmq_group<T, GLU, 1, false>(a, g, wb, L);
+    else mmq_group<T, GLU, 2, false>(a, g, wb, L);
 }
 
 // Gate/up (with SwiGLU and the Q8_1 of act) and down of the expert path in one launch. The gate/up items come first,
@@ -1290,7 +1328,8 @@ template <bool GLU> const void *mmq_kernel(int type) {
 
 // groups: upper bound of the 64-row list; expert path: of the 64-row list and the <= 32-row remainders together (the
 // workgroups past the device-side counts return at once)
-int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st) {
+// sh: a dense matrix of the same type whose groups come first in the grid (expert path only)
+int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st, const MmqShared *sh = nullptr) {
     const void *fn = glu ? mmq_kernel<true>(type) : mmq_kernel<false>(type);
     if (!fn) return host::set_error(host::ERR_TYPE, "mmq: type %d not supported", type);
     if (groups <= 0) return host::OK;
@@ -1299,8 +1338,16 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st)
     // expert path: n_expert + ceil(pairs / 64) (the 64-row list's bound) bounds both lists together, as expert e
     // has ceil(n_e / 64) groups in all
     int total = groups;
-    void *args[] = {&arg};
+    MmqShared shared{};
+    void *args[] = {&arg, &shared};
     const int rows = glu ? 128 : 256;  // weight rows per workgroup
+    int64_t sh_items = 0;
+    if (sh && a.bounds) {
+        shared = *sh;
+        shared.n_cb = (sh->nrows + rows - 1) / rows;
+        const int sg = (sh->n_rows + kMmqTok - 1) / kMmqTok;
+        sh_items = (int64_t) shared.n_cb * kXcds * ((sg + kXcds - 1) / kXcds);
+    }
     arg.n_cb = (a.nrows + rows - 1) / rows;
     // dense: when even twice the workgroups of the 64-row groups fit one per CU, groups of 32 rows (one token tile:
     // more B decode per MFMA, but twice the workgroups; measured faster for 64 -> 128 workgroups, slower for
@@ -1314,8 +1361,9 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st)
         total = (a.n_rows + 31) / 32;
     }
     arg.n_groups = total;
-    const int64_t items = (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds);
+    const int64_t items = sh_items + (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds);
     if (items > INT32_MAX) return host::set_error(host::ERR_SHAPE, "mmq: grid too large");
+    shared.items = (int) sh_items;
     const hipError_t e = hipLaunchKernel(fn, dim3((unsigned) items, (unsigned) ks), dim3(kMmqThreads), args, 0, st);
     if (e != hipSuccess) return host::set_error(host::ERR_LAUNCH, "mmq: %s", hipGetErrorString(e));
     return host::check_launch("mmq");
@@ -1586,35 +1634,48 @@ int moe_prefill_workspace(const FnsMoeLayer *L, int64_t n_tok, size_t *offsets, 
     return host::OK;
 }
 
-// The shared expert over the n_tok split-image rows of h: one GLU launch (gate and up, SwiGLU, Q8_1 of act into
-// act_img) and the down launch into sh [n_tok][hidden]; both are the grouped GEMM over one dense matrix.
-int mmq_dense_shared(const FnsMoeLayer *L, const void *ximg, int64_t n_tok, void *act_img, float *sh, hipStream_t st) {
-    const int gt = L->shexp_gu_type ? L->shexp_gu_type : L->gu_type;
-    const int dt = L->shexp_down_type ? L->shexp_down_type : L->down_type;
-    FNS_TRY(check_mmq_shape(gt, L->hidden, L->shexp_inter));
-    FNS_TRY(check_mmq_shape(dt, L->shexp_inter, L->hidden));
-    const int groups = (int) ((n_tok + kMmqTok - 1) / kMmqTok);
-    MmqArgs g{};
-    g.w_dense = (const uint8_t *) L->shexp_gate;
-    g.off_a = 0;
+// The shared expert over the n_tok split-image rows of h: gate and up, SwiGLU and the Q8_1 of act into act_img (gu),
+// then down into sh [n_tok][hidden] (dn). Both are the grouped GEMM over one dense matrix; with the routed experts'
+// type they ride in the routed launch (its workgroups are few: 8 at 37 tokens of the reference model's block, 25.5 +
+// 15.9 us as launches of their own, against nothing beside the routed 149 experts'), otherwise mmq_dense_shared
+// launches them.
+MmqShared shared_gate_up(const FnsMoeLayer *L, const void *ximg, int64_t n_tok, void *act_img) {
+    MmqShared g{};
+    g.w = (const uint8_t *) L->shexp_gate;
     g.off_b = (const uint8_t *) L->shexp_up - (const uint8_t *) L->shexp_gate;
     g.ncols = L->hidden;
     g.nrows = L->shexp_inter;
+    g.n_rows = (int) n_tok;
     g.xpack = (const uint8_t *) ximg;
     g.x_img = (int64_t) mmq_image_bytes(L->hidden);
-    g.n_rows = (int) n_tok;
     g.out_pack = (uint8_t *) act_img;
     g.out_img = (int64_t) mmq_image_bytes(L->shexp_inter);
-    FNS_TRY(launch_mmq(gt, true, g, groups, st));
-    MmqArgs d{};
-    d.w_dense = (const uint8_t *) L->shexp_down;
+    return g;
+}
+MmqShared shared_down(const FnsMoeLayer *L, const void *act_img, int64_t n_tok, float *sh) {
+    MmqShared d{};
+    d.w = (const uint8_t *) L->shexp_down;
     d.ncols = L->shexp_inter;
     d.nrows = L->hidden;
+    d.n_rows = (int) n_tok;
     d.xpack = (const uint8_t *) act_img;
     d.x_img = (int64_t) mmq_image_bytes(L->shexp_inter);
-    d.n_rows = (int) n_tok;
     d.dst = sh;
-    return launch_mmq(dt, false, d, groups, st);
+    return d;
+}
+int mmq_dense_shared(int type, bool glu, const MmqShared &s, hipStream_t st) {
+    MmqArgs a{};
+    a.w_dense = s.w;
+    a.off_b = s.off_b;
+    a.ncols = s.ncols;
+    a.nrows = s.nrows;
+    a.xpack = s.xpack;
+    a.x_img = s.x_img;
+    a.n_rows = s.n_rows;
+    a.dst = s.dst;
+    a.out_pack = s.out_pack;
+    a.out_img = s.out_img;
+    return launch_mmq(type, glu, a, (s.n_rows + kMmqTok - 1) / kMmqTok, st);
 }
 
 // Dense GEMMs on activation images already built (the dense FFN block): gate/up in one GLU launch (SwiGLU and the
@@ -1767,6 +1828,20 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
                         astride));
     FNS_TRY(expert_args(L->down_type, table, L->down_off, 0, false, L->inter, L->hidden, L->n_expert, sec[4], dstr,
                         dstr, bounds, bounds + L->n_expert + 1, dexp, nullptr, nullptr, dn, astride));
+    // the shared expert (reference src/engine.cu:351-355): in the routed launches where the types agree
+    const bool has_sh = L->shexp_inter > 0;
+    const int sgt = has_sh && L->shexp_gu_type ? L->shexp_gu_type : L->gu_type;
+    const int sdt = has_sh && L->shexp_down_type ? L->shexp_down_type : L->down_type;
+    float *sh = has_sh ? (float *) sec[14] : nullptr;
+    MmqShared sgu{}, sdn{};
+    if (has_sh) {
+        FNS_TRY(check_mmq_shape(sgt, L->hidden, L->shexp_inter));
+        FNS_TRY(check_mmq_shape(sdt, L->shexp_inter, L->hidden));
+        sgu = shared_gate_up(L, sec[3], n_tok, sec[13]);
+        sdn = shared_down(L, sec[13], n_tok, sh);
+    }
+    const bool ride_gu = has_sh && !fused && sgt == L->gu_type, ride_dn = has_sh && !fused && sdt == L->down_type;
+    if (has_sh && !ride_gu) FNS_TRY(mmq_dense_shared(sgt, true, sgu, st));
     if (fused) {
         MoeArgs m{};
         m.table = table;
@@ -1791,18 +1866,14 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
         moe_test_hooks(&m.spin_limit, &m.gwait);  // withheld arrivals; + the gate/up row blocks per group
         FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, m, st));
     } else {
-        FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st));
+        FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st, ride_gu ? &sgu : nullptr));
         if (L->guard) {  // whole-row amax: a second pass over the f32 act rows (reference src/kernels.cu:534-552)
             FNS_TRY(amax_guard(act, escale, L->inter, (int) P, st));
             FNS_TRY(mmq_quant_image_scaled(act, escale, L->inter, P, sec[4], astride, st));
         }
-        FNS_TRY(launch_mmq(L->down_type, false, dn, groups, st));
+        FNS_TRY(launch_mmq(L->down_type, false, dn, groups, st, ride_dn ? &sdn : nullptr));
     }
-    float *sh = nullptr;
-    if (L->shexp_inter > 0) {  // shared expert (reference src/engine.cu:351-355): dense gate/up + SwiGLU, then down
-        sh = (float *) sec[14];
-        FNS_TRY(mmq_dense_shared(L, sec[3], n_tok, sec[13], sh, st));
-    }
+    if (has_sh && !ride_dn) FNS_TRY(mmq_dense_shared(sdt, false, sdn, st));
     return moe_combine(dexp, L->guard ? escale : nullptr, w, sh, x_resid, out, L->hidden, L->k, (int) n_tok, st);
 }
 

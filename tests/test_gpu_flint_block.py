@@ -141,6 +141,20 @@ def test_flint_block_prefill(ops, layer, mats):
     assert_close_chain(out[toks], ref, "flint block prefill")
 
 
+@pytest.mark.parametrize("T", [32, 33, 64, 65, 96, 97])
+def test_flint_block_prefill_shared_groups(ops, layer, T):
+    """The shared expert's groups inside the routed launches, at the edges of their 64-row groups and 32-row tiles:
+    every token equals the same token prefilled alone (one token tile), bit for bit."""
+    from flintnsteel_amd import synth
+    pre = ops.MoePrefill(layer)
+    x = synth.activations(T, H, SEED, layer=37)
+    out = host(pre(x, ws=pre.workspace(T), x_resid=x))
+    ws1 = pre.workspace(1)
+    for t in sorted({0, 31, 32, 63, 64, T - 1} & set(range(T))):
+        xt = x[t:t + 1].contiguous()
+        assert np.array_equal(out[t], host(pre(xt, ws=ws1, x_resid=xt))[0]), f"token {t} of {T}"
+
+
 def test_flint_block_prefill_norm_image(ops, layer):
     """The prefill's RMSNorm output, its Q8_1 blocks and the activation image built in the same pass equal the
     standalone kernel's output, blocks and the image those blocks define."""
