@@ -67,8 +67,7 @@ int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, void *xpack, hi
 bool mmq_rms_norm_image_fits(const float *x, const float *w, const float *out, int64_t n);
 int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, void *ximg,
                        hipStream_t st);
-int mmq_quant_image_scaled(const float *x, const float *escale, int64_t ncols, int64_t rows, void *xpack, int64_t stride,
-                           hipStream_t st);
+int mmq_guard_image(float *act, float *escale, int64_t ncols, int64_t rows, void *img, int64_t stride, hipStream_t st);
 int mmq_compact(const int32_t *ids, int64_t n_tok, int64_t k, int64_t n_expert, int64_t x_rows_per_tok,
                 int32_t *ids_src1, int32_t *ids_dst, int32_t *bounds, int32_t *gprefix, hipStream_t st,
                 int32_t *gdone = nullptr, int n_gdone = 0);

@@ -116,4 +116,17 @@ __device__ __forceinline__ Q8Lane q8_1_lane(float v) {
     return r;
 }
 
+// F16 guard scale of a row with the fp32 sequence of the reference (src/kernels.cu:544-551).
+__device__ __forceinline__ float guard_scale(float amax) {
+    // amax <= 1024 (the common case): the sequence below gives exactly 1 (log <= 0, ceil <= 0, clamped to 0, exp(0))
+    if (amax <= 1024.0f) return 1.0f;
+    float e = amax * (1.0f / 1024.0f);
+    e = logf(e);
+    e = e * 1.4426950408889634f;
+    e = ceilf(e);
+    e = fminf(fmaxf(e, 0.0f), 127.0f);
+    e = e * 0.6931471805599453f;
+    return expf(e);
+}
+
 }  // namespace fns::dev

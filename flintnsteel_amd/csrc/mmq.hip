@@ -58,17 +58,18 @@ inline size_t gprefix_bytes(int64_t n_expert) { return (size_t) 2 * (n_expert + 
 // ---- compaction (ggml mm_ids_helper semantics, stable) ------------------------------------------------------------
 // ids [n_tok][k] -> pairs p = t k + j sorted by expert, ties in p order: ids_dst[q] = p, ids_src1[q] = the activation
 // row of p (t when x_rows_per_tok = 1, p when x_rows_per_tok = k), bounds[e] = first sorted position of expert e.
-// One workgroup; wave w owns a contiguous chunk of the pairs (its first 8 ids per lane kept in registers): per-wave
-// histograms (LDS atomics), one prefix over (expert, wave) in that order, then each wave walks its chunk again in
-// order, ranking the lanes that share an expert by ballots on the expert id bits, and advances its own running
-// positions - two passes over the ids, four barriers.
+// Workgroup b owns the 1024-pair pieces [b per_wg, (b + 1) per_wg) and needs no other workgroup: each reads every id
+// (they sit in the L2) into two LDS histograms - the pairs before its own, and the rest - which give every expert's
+// first position and how many of its rows earlier workgroups place. Its own pieces are then ranked in order: the lanes
+// that share an expert by ballots on the id bits, the waves by a prefix of their counts. One workgroup walking all
+// pairs took 47 us at 32768 pairs and 7.8 us at 4096.
 // Workgroup barrier for LDS data only: no global memory is produced and consumed inside the compaction kernel, so its
 // barriers need not wait for the id loads and the output stores still in flight (__syncthreads' fence would).
 __device__ __forceinline__ void lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 // Exclusive prefix of the per-expert counts cnt[0..ne) (ne <= 256) by one wave (lane = its lane): cnt[e] becomes the
 // expert's first sorted position; bounds[0..ne], and the group prefixes gprefix[0..ne] of the 64-row groups
 // (n_e / 64 full ones, and the remainder if it is > 32 rows) and gprefix[ne + 1 .. 2 ne + 1] of the <= 32-row
-// remainders are written. 4 experts per lane, then a lane scan.
+// remainders are written (bounds null: none are). 4 experts per lane, then a lane scan.
 __device__ __forceinline__ void expert_prefix_wave(int lane, int *cnt, int ne, int32_t *bounds, int32_t *gprefix) {
     int v[4], g[4], g2[4], s = 0, sg = 0, sg2 = 0;
 #pragma unroll
@@ -97,15 +98,17 @@ __device__ __forceinline__ void expert_prefix_wave(int lane, int *cnt, int ne, i
         const int e = 4 * lane + j;
         if (e < ne) {
             cnt[e] = run;  // the expert's first sorted position (its count is no longer needed)
-            bounds[e] = run;
-            gprefix[e] = rung;
-            gprefix[ne + 1 + e] = rung2;
+            if (bounds) {
+                bounds[e] = run;
+                gprefix[e] = rung;
+                gprefix[ne + 1 + e] = rung2;
+            }
         }
         run += v[j];
         rung += g[j];
         rung2 += g2[j];
     }
-    if (lane == 63) {
+    if (lane == 63 && bounds) {
         bounds[ne] = incl;
         gprefix[ne] = inclg;
         gprefix[2 * ne + 1] = inclg2;
@@ -115,69 +118,40 @@ __device__ __forceinline__ void expert_prefix_wave(int lane, int *cnt, int ne, i
 __global__ __launch_bounds__(kCompactThreads) void k_mmq_compact(const int32_t *__restrict__ ids, int n, int k, int ne,
                                                                  int x_rows_per_tok, int32_t *__restrict__ ids_src1,
                                                                  int32_t *__restrict__ ids_dst, int32_t *bounds,
-                                                                 int32_t *gprefix, int32_t *gdone, int n_gdone) {
-    constexpr int NW = kCompactThreads / kWave;
-    __shared__ int cnt[256];
-    __shared__ int wpos[NW][256];  // per-wave counts, then each wave's next sorted position per expert
+                                                                 int32_t *gprefix, int32_t *gdone, int n_gdone,
+                                                                 int per_wg) {
+    constexpr int NW = kCompactThreads / kWave, NT = kCompactThreads;
+    __shared__ int pos[256], rest[256], cnt[256];
+    __shared__ int wpos[NW][256];  // a piece's per-wave counts, then each wave's first sorted position per expert
     PF_MARK(2, 0);
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-    for (int i = tid; i < NW * 256; i += kCompactThreads) (&wpos[0][0])[i] = 0;
-    for (int i = tid; i < n_gdone; i += kCompactThreads) gdone[i] = 0;  // the next fused GEMM launch's arrivals
+    const int n_it = (n + NT - 1) / NT, it0 = blockIdx.x * per_wg, it1 = min(n_it, it0 + per_wg);
+    for (int i = tid; i < NW * 256; i += NT) (&wpos[0][0])[i] = 0;
+    if (tid < 256) pos[tid] = rest[tid] = 0;
+    for (int i = blockIdx.x * NT + tid; i < n_gdone; i += gridDim.x * NT) gdone[i] = 0;  // the fused GEMM launch's arrivals
     lds_sync();
     PF_MARK(2, 2);
-    const int chunk = (n + NW * kWave - 1) / (NW * kWave) * kWave;  // pairs per wave, a multiple of 64
-    const int p0 = wave * chunk, p1 = min(n, p0 + chunk);
-    // the first kCache ids of each lane stay in registers for the second pass; their loads are clamped into the
-    // array and unconditional (under the uniform n > 0: an empty batch still writes the bounds), so they are all in
-    // flight together
-    constexpr int kCache = 8;
-    int ev[kCache];
+    // clamped, unconditional loads (under the uniform n > 0: an empty batch still writes the bounds), eight in flight
+    constexpr int U = 8;
+    for (int it = 0; it < n_it; it += U) {
+        int v[U];
 #pragma unroll
-    for (int it = 0; it < kCache; ++it) {
-        const int p = p0 + lane + kWave * it;
-        const int v = n > 0 ? ids[min(p, n - 1)] : -1;
-        ev[it] = kWave * it < chunk && p < p1 ? v : -1;
-    }
-    auto id_at = [&](int p) { return p < p1 ? ids[p] : -1; };
+        for (int u = 0; u < U; ++u) v[u] = ids[min((it + u) * NT + tid, n - 1)];
 #pragma unroll
-    for (int it = 0; it < kCache; ++it) {
-        const int e = ev[it];
-        if (e >= 0 && e < ne) atomicAdd(&wpos[wave][e], 1);
-    }
-    for (int p = p0 + lane + kWave * kCache; p < p0 + chunk; p += kWave) {  // wave-uniform trip count
-        const int e = id_at(p);
-        if (e >= 0 && e < ne) atomicAdd(&wpos[wave][e], 1);
+        for (int u = 0; u < U; ++u)
+            if ((it + u) * NT + tid < n && v[u] >= 0 && v[u] < ne) atomicAdd(it + u < it0 ? &pos[v[u]] : &rest[v[u]], 1);
     }
     lds_sync();
     PF_MARK(2, 3);
-    if (tid < ne) {
-        int c = 0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) c += wpos[w][tid];
-        cnt[tid] = c;
-    }
+    if (tid < ne) cnt[tid] = pos[tid] + rest[tid];
     lds_sync();
-    PF_MARK(2, 4);
-    if (wave == 0) expert_prefix_wave(lane, cnt, ne, bounds, gprefix);
+    if (wave == 0) expert_prefix_wave(lane, cnt, ne, blockIdx.x == 0 ? bounds : nullptr, gprefix);
     lds_sync();
     PF_MARK(2, 5);
-    if (tid < ne) {  // the expert's sorted positions, split over the waves in wave order
-        int pos = cnt[tid];
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const int c = wpos[w][tid];
-            wpos[w][tid] = pos;
-            pos += c;
-        }
-    }
-    lds_sync();
-    PF_MARK(2, 6);
-    for (int it = 0, p = p0 + lane; p < p0 + chunk; ++it, p += kWave) {
-        int e = -1;
-#pragma unroll
-        for (int c = 0; c < kCache; ++c)
-            if (it == c) e = ev[c];
-        if (it >= kCache) e = id_at(p);
+    if (tid < ne) pos[tid] += cnt[tid];  // where this workgroup's first row of the expert goes
+    for (int it = it0; it < it1; ++it) {
+        const int p = it * NT + tid;
+        const int e = p < n ? ids[p] : -1;
         const bool live = e >= 0 && e < ne;
         // lanes with the same expert id: intersect the ballots of each id bit (and of liveness)
         uint64_t same = __ballot(live);
@@ -186,15 +160,30 @@ __global__ __launch_bounds__(kCompactThreads) void k_mmq_compact(const int32_t *
             const uint64_t m = __ballot(live && ((e >> b) & 1));
             same &= ((e >> b) & 1) ? m : ~m;
         }
-        if (!live) same = 0;
         const int rank = __popcll(same & ((1ull << lane) - 1ull));
-        if (live) {
-            const int pos = wpos[wave][e] + rank;
-            ids_dst[pos] = p;
-            ids_src1[pos] = x_rows_per_tok == 1 ? p / k : p;
+        if (live && rank == 0) wpos[wave][e] = __popcll(same);
+        lds_sync();
+        if (tid < ne) {  // the piece's rows of the expert, split over the waves in wave order
+            int q = pos[tid];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const int c = wpos[w][tid];
+                wpos[w][tid] = q;
+                q += c;
+            }
+            pos[tid] = q;
         }
-        // (this wave's reads above complete before its write below: one wave, LDS accesses in order)
-        if (live && rank == 0) wpos[wave][e] += __popcll(same);
+        lds_sync();
+        if (live) {
+            const int q = wpos[wave][e] + rank;
+            ids_dst[q] = p;
+            ids_src1[q] = x_rows_per_tok == 1 ? p / k : p;
+        }
+        if (it + 1 < it1) {
+            lds_sync();
+            for (int i = tid; i < NW * 256; i += NT) (&wpos[0][0])[i] = 0;
+            lds_sync();
+        }
     }
     PF_MARK(2, 1);
 }
@@ -301,16 +290,31 @@ __global__ __launch_bounds__(256) void k_rms_norm_image(const float *__restrict_
     });
 }
 
-// F16-guard form: only the rows whose guard scale is not 1 are re-quantised (the others already hold the image of
-// the same values, written by the GEMM epilogue); grid as k_quant_image.
-__global__ __launch_bounds__(256) void k_quant_image_scaled(const float *__restrict__ x, const float *__restrict__ escale,
-                                                            int ncols, uint8_t *__restrict__ out, int64_t img_row_bytes) {
-    const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * 8;
-    if (escale[row] == 1.0f || col >= ncols) return;
-    const float *src = x + (size_t) row * ncols + col;
-    const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
-    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    q8_split8<true>(v, out + (size_t) row * img_row_bytes, ncols, col, true);
+// F16 guard of the act rows (reference src/kernels.cu:534-577), one wave per row of n columns (n % 256 == 0): the scale
+// from the row's maximum, and only where it is not 1 the division in place and the row's image again (the GEMM epilogue
+// has written the image of the undivided values, which is the same when it is 1). Bound by reading the rows once; the
+// scale and the image were two launches (9.9 + 5.2 us at 6126 rows of 512).
+__global__ __launch_bounds__(256) void k_guard_image(float *__restrict__ act, float *__restrict__ escale, int n, int rows,
+                                                     uint8_t *__restrict__ out, int64_t img_row_bytes) {
+    const int row = blockIdx.x * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (row >= rows) return;
+    float *r = act + (size_t) row * n;
+    float m = 0.0f;
+#pragma unroll 2
+    for (int i = 4 * lane; i < n; i += 4 * kWave) {
+        const float4 v = *(const float4 *) (r + i);
+        m = fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+    }
+    const float e = guard_scale(lanes_max<64>(m));
+    if (lane == 0) escale[row] = e;
+    if (e == 1.0f) return;  // (the whole wave)
+    for (int i = 8 * lane; i < n; i += 8 * kWave) {  // a block's four lanes are all in or all out
+        const float4 x0 = *(const float4 *) (r + i), x1 = *(const float4 *) (r + i + 4);
+        const float v[8] = {x0.x / e, x0.y / e, x0.z / e, x0.w / e, x1.x / e, x1.y / e, x1.z / e, x1.w / e};
+        *(float4 *) (r + i) = make_float4(v[0], v[1], v[2], v[3]);
+        *(float4 *) (r + i + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        q8_split8<true>(v, out + (size_t) row * img_row_bytes, n, i, true);
+    }
 }
 
 // Router GEMM tiles and the split activation image of the same rows in one launch (the two only read x): workgroups
@@ -1456,14 +1460,13 @@ int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int
     return host::check_launch("mmq rms_norm");
 }
 
-int mmq_quant_image_scaled(const float *x, const float *escale, int64_t ncols, int64_t rows, void *xpack,
-                           int64_t stride, hipStream_t st) {
-    if (!x || !escale || !xpack || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
-        return host::set_error(host::ERR_SHAPE, "mmq quantize: bad arguments");
+int mmq_guard_image(float *act, float *escale, int64_t ncols, int64_t rows, void *img, int64_t stride, hipStream_t st) {
+    if (!act || !escale || !img || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
+        return host::set_error(host::ERR_SHAPE, "mmq guard: bad arguments");
     if (rows == 0) return host::OK;
-    hipLaunchKernelGGL(k_quant_image_scaled, dim3((unsigned) ((ncols + 2047) / 2048), (unsigned) rows), dim3(256), 0, st,
-                       x, escale, (int) ncols, (uint8_t *) xpack, stride);
-    return host::check_launch("mmq quantize (guarded rows)");
+    hipLaunchKernelGGL(k_guard_image, dim3((unsigned) ((rows + 3) / 4)), dim3(256), 0, st, act, escale, (int) ncols,
+                       (int) rows, (uint8_t *) img, stride);
+    return host::check_launch("mmq guard");
 }
 
 int mmq_compact(const int32_t *ids, int64_t n_tok, int64_t k, int64_t n_expert, int64_t x_rows_per_tok,
@@ -1474,8 +1477,13 @@ int mmq_compact(const int32_t *ids, int64_t n_tok, int64_t k, int64_t n_expert, 
     if ((any && (!ids || !ids_src1 || !ids_dst)) || !bounds || !gprefix || n_tok < 0 || k < 1 || n_expert < 1 || n_expert > 256 ||
         n_tok * k > (1 << 20) || (x_rows_per_tok != 1 && x_rows_per_tok != k))
         return host::set_error(host::ERR_SHAPE, "mmq compaction: bad arguments");
-    hipLaunchKernelGGL(k_mmq_compact, dim3(1), dim3(kCompactThreads), 0, st, ids, (int) (n_tok * k), (int) k,
-                       (int) n_expert, (int) x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, gdone, gdone ? n_gdone : 0);
+    // at most 64 workgroups (every one reads all ids), one 1024-pair piece each up to 65536 pairs
+    const int64_t pieces = (n_tok * k + kCompactThreads - 1) / kCompactThreads;
+    const int per_wg = (int) std::max<int64_t>(1, (pieces + 63) / 64);
+    const unsigned wgs = (unsigned) std::max<int64_t>(1, (pieces + per_wg - 1) / per_wg);
+    hipLaunchKernelGGL(k_mmq_compact, dim3(wgs), dim3(kCompactThreads), 0, st, ids, (int) (n_tok * k), (int) k,
+                       (int) n_expert, (int) x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, gdone, gdone ? n_gdone : 0,
+                       per_wg);
     return host::check_launch("mmq compaction");
 }
 
@@ -1867,10 +1875,8 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
         FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, m, st));
     } else {
         FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st, ride_gu ? &sgu : nullptr));
-        if (L->guard) {  // whole-row amax: a second pass over the f32 act rows (reference src/kernels.cu:534-552)
-            FNS_TRY(amax_guard(act, escale, L->inter, (int) P, st));
-            FNS_TRY(mmq_quant_image_scaled(act, escale, L->inter, P, sec[4], astride, st));
-        }
+        // whole-row amax: a second pass over the f32 act rows (reference src/kernels.cu:534-552)
+        if (L->guard) FNS_TRY(mmq_guard_image(act, escale, L->inter, P, sec[4], astride, st));
         FNS_TRY(launch_mmq(L->down_type, false, dn, groups, st, ride_dn ? &sdn : nullptr));
     }
     if (has_sh && !ride_dn) FNS_TRY(mmq_dense_shared(sdt, false, sdn, st));

@@ -551,18 +551,6 @@ __global__ __launch_bounds__(NTH) void k_gate_up_q(const LayerArgs a) {
 }
 
 // ---- K3: (guard) + down GEMV + combine -------------------------------------------------------------------------------
-__device__ __forceinline__ float guard_scale(float amax) {
-    // amax <= 1024 (the common case): the sequence below gives exactly 1 (log <= 0, ceil <= 0, clamped to 0, exp(0))
-    if (amax <= 1024.0f) return 1.0f;
-    float e = amax * (1.0f / 1024.0f);
-    e = logf(e);
-    e = e * 1.4426950408889634f;
-    e = ceilf(e);
-    e = fminf(fmaxf(e, 0.0f), 127.0f);
-    e = e * 0.6931471805599453f;
-    return expf(e);
-}
-
 // Quarter-block form of the down projection + combine: 1024 threads; the work is 2 * n_chan groups of (channel, four
 // of the workgroup's eight rows), group g taken by wave g % 16. Each wave copies its channel's act image and its four
 // rows into a private LDS area, waits only for its own copies and computes its four rows with 16 lanes per row.

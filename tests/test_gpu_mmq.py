@@ -46,6 +46,23 @@ def table_of(mats_dev):
                         dtype=torch.int64, device="cuda")
 
 
+@pytest.mark.parametrize("n_pairs", [1024, 1025, 2047, 65536, 65537, 70001])
+def test_compaction_pieces(ops, n_pairs):
+    """One id per token at the edges of the 1024-pair pieces and of one piece per workgroup (65536 pairs), two thirds
+    of them one expert's and some of no expert at all (ids outside 0 .. n_expert - 1 are left out)."""
+    rng = np.random.default_rng(n_pairs)
+    ne = 60
+    ids = rng.integers(0, ne, n_pairs).astype(np.int32)
+    ids[rng.random(n_pairs) < 0.66] = 17
+    ids[rng.random(n_pairs) < 0.01] = ne
+    ids[rng.random(n_pairs) < 0.01] = -1
+    bounds, src, dst = (host(t) for t in ops.mmq_compact(dev(ids[:, None]), ne, 1))
+    live = np.flatnonzero((ids >= 0) & (ids < ne))
+    want = live[np.argsort(ids[live], kind="stable")]
+    assert np.array_equal(bounds, np.concatenate([[0], np.cumsum(np.bincount(ids[live], minlength=ne))]))
+    assert np.array_equal(dst[:want.size], want) and np.array_equal(src[:want.size], want)
+
+
 @pytest.mark.parametrize("n_tok,k,n_expert,xr", [(0, 8, 16, 1), (77, 8, 16, 1), (77, 8, 16, 8), (1, 1, 1, 1), (600, 8, 128, 1),
                                                  (5, 6, 256, 6), (1100, 4, 8, 1), (4096, 8, 128, 1),
                                                  (1024, 8, 128, 1), (1023, 8, 64, 8)])
