@@ -1,0 +1,403 @@
+// fns_mmq_i8.hpp - the grouped GEMM on int8 MFMA, for the types whose scales change every 32 columns (Q8_0, Q4_K, Q5_K,
+// IQ4_XS, IQ3_XXS, IQ3_S: a sub-block is exactly one v_mfma_i32_32x32x32_i8). Included by mmq.hip, whose group lists,
+// epilogues and weight fragments it shares.
+//
+// Per sub-block s the MFMA gives the exact integer dot I of 32 codes; the output takes I * (d8[token] * dw[row]) with
+// dw = the row's sub-block scale (block d times the integer scale, exact in fp32 for a 6-bit scale): convert, scale
+// product and fma, 48 VALU instructions per 32x32x32 step against one 32-cycle MFMA, so the kernel is bound by VALU
+// issue, 192 cycles a step. The f16 form spends four MFMAs (128 cycles; eight for Q8_0 and IQ4_XS, whose operands are
+// split in two) plus the B decode on the same step, and its activations are 4.125 bytes a value against 1.25 here: half
+// the LDS-DMA traffic remains in every superblock, one barrier instead of two, and no f16 decode of the codes.
+#pragma once
+
+namespace fns {
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// ---- activation image ---------------------------------------------------------------------------------------------
+// Row layout, per 256-column superblock kb at kb * 320: the 256 int8 codes, the 8 block scales d8 (f32, f16 values),
+// the min-term sums [S_hi 8 f16][S_lo 8 f16] of the split image (same order).
+constexpr int kI8Sb = 320, kI8Scale = 256, kI8Sum = 288;
+__host__ __device__ constexpr int64_t i8_row_bytes(int64_t ncols) { return ncols / 256 * kI8Sb; }
+
+// the lane's part of a quantised block (8 codes at column col, a multiple of 8; scale dh): the block's first lane also
+// stores the scale and the sums
+__device__ __forceinline__ void i8_store(const Q8x8 &r, uint8_t *row, int col) {
+    uint8_t *sb = row + (size_t) (col >> 8) * kI8Sb;
+    uint32_t w[2] = {0, 0};
+    int qsum = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        w[k / 4] |= (uint32_t) (uint8_t) (int8_t) r.q[k] << (8 * (k % 4));
+        qsum += r.q[k];
+    }
+    *(uint2 *) (sb + (col & 255)) = make_uint2(w[0], w[1]);
+    qsum = lanes_sum_i<4>(qsum);
+    if ((col & 31) == 0) {
+        const int s = (col >> 5) & 7;
+        const float dh = half_to_float(float_to_half(r.d)), sv = dh * (float) qsum;  // exact in fp32
+        const _Float16 hi = (_Float16) sv;
+        *(float *) (sb + kI8Scale + 4 * s) = dh;
+        _Float16 *m = (_Float16 *) (sb + kI8Sum + 2 * perm8(s));
+        m[0] = hi;
+        m[8] = (_Float16) (sv - (float) hi);
+    }
+}
+
+// x [rows][ncols] f32 -> image rows; grid (ceil(ncols / 2048), rows), 256 threads of 8 columns each
+__global__ __launch_bounds__(256) void k_quant_i8(const float *__restrict__ x, int ncols, uint8_t *__restrict__ out,
+                                                  int64_t img_row_bytes) {
+    const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (col >= ncols) return;
+    const float *src = x + (size_t) row * ncols + col;
+    const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
+    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    i8_store(q8_1_x8(v), out + (size_t) row * img_row_bytes, col);
+}
+
+// RMSNorm of a row of at most 2048 C columns (fns_q8x8.hpp), out as f32 and as an image row.
+template <int C>
+__global__ __launch_bounds__(256) void k_rms_norm_i8(const float *__restrict__ x, const float *__restrict__ w,
+                                                     float *__restrict__ out, int n, float eps, uint8_t *__restrict__ img,
+                                                     int64_t img_row_bytes) {
+    __shared__ __align__(16) float xs[2048 * C];
+    const size_t r = blockIdx.x;
+    uint8_t *row = img + r * img_row_bytes;
+    rms_norm_row<C>(x + r * n, w, out + r * n, nullptr, n, eps, xs, [&](const Q8x8 &q, int col) { i8_store(q, row, col); });
+}
+
+// ---- weight fragments ---------------------------------------------------------------------------------------------
+// The types of the f16 form keep their fragments (WFrag). Q8_0 (blocks of 34 bytes, f16 d then 32 codes): blocks e = 2 p
+// and e + 1 start at 68 p, a multiple of four; lane half h reads the even block's 16 codes as the 20 aligned bytes at
+// 68 p + 16 h (they start two bytes in) and the odd block's 16 at 68 p + 36 + 16 h. The two d lie in those bytes, the
+// even block's in the first dword of half 0, the odd block's in the last of half 1: one exchange between the halves.
+// (16 bytes at 2-byte addresses and a 2-byte load per d, as the f16 form had, were half of that kernel's time.)
+template <int T> struct I8Frag { WFrag<T> f; };
+template <> struct I8Frag<T_Q8_0> { uint4 e[4], o[4]; uint32_t x[4]; };
+template <int T, int P>
+__device__ __forceinline__ void i8frag_load(Rsrc r, uint32_t vo, uint32_t vc, uint32_t so, I8Frag<T> &f) {
+    if constexpr (T == T_Q8_0) {
+#pragma unroll
+        for (int p = 2 * P; p < 2 * P + 2; ++p) {
+            f.e[p] = bload16(r, vc, so + 68 * p);
+            f.x[p] = bload4(r, vc, so + 68 * p + 16);
+            f.o[p] = bload16(r, vc, so + 68 * p + 36);
+        }
+    } else {
+        wfrag_load<T, P>(r, vo, vc, so, f.f);
+    }
+}
+// Sub-block s (compile time): the lane's 16 codes as signed bytes (columns 16 h .. 16 h + 15 of the sub-block; IQ4_XS:
+// 8 h .. 8 h + 7 and 16 + 8 h ..) and the row's scale of the sub-block.
+template <int T>
+__device__ __forceinline__ v4i i8_codes(const I8Frag<T> &f, int s, int h, const uint32_t *grid) {
+    if constexpr (T == T_Q8_0) {
+        const int p = s >> 1;
+        if (s & 1) return v4i{(int) f.o[p].x, (int) f.o[p].y, (int) f.o[p].z, (int) f.o[p].w};
+        return v4i{(int) __builtin_amdgcn_alignbit(f.e[p].y, f.e[p].x, 16),
+                   (int) __builtin_amdgcn_alignbit(f.e[p].z, f.e[p].y, 16),
+                   (int) __builtin_amdgcn_alignbit(f.e[p].w, f.e[p].z, 16),
+                   (int) __builtin_amdgcn_alignbit(f.x[p], f.e[p].w, 16)};
+    } else if constexpr (T == T_Q4_K || T == T_Q5_K) {
+        const uint4 q = f.f.q[s >> 1];
+        const int sh = 4 * (s & 1);
+        uint32_t w[4] = {(q.x >> sh) & kLo4, (q.y >> sh) & kLo4, (q.z >> sh) & kLo4, (q.w >> sh) & kLo4};
+        if constexpr (T == T_Q5_K) {
+            const uint4 qh = f.f.qh;
+            w[0] |= ((qh.x >> s) & 0x01010101u) << 4;
+            w[1] |= ((qh.y >> s) & 0x01010101u) << 4;
+            w[2] |= ((qh.z >> s) & 0x01010101u) << 4;
+            w[3] |= ((qh.w >> s) & 0x01010101u) << 4;
+        }
+        return v4i{(int) w[0], (int) w[1], (int) w[2], (int) w[3]};
+    } else if constexpr (T == T_IQ4_XS) {
+        const uint2 q = f.f.q[s];
+        return v4i{(int) iq4nl_values(q.x & kLo4), (int) iq4nl_values(q.y & kLo4), (int) iq4nl_values((q.x >> 4) & kLo4),
+                   (int) iq4nl_values((q.y >> 4) & kLo4)};
+    } else if constexpr (T == T_IQ3_XXS) {
+        const uint32_t aux = word(f.f.aux[s >> 2], s & 3), idx = f.f.idx[s];
+        v4i r;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const uint32_t sg = ksigns((aux >> (7 * (2 * h + p))) & 127u);
+            r[2 * p] = signed_grid(grid[(idx >> (16 * p)) & 0xffu], spread4(sg & 0xfu));
+            r[2 * p + 1] = signed_grid(grid[(idx >> (16 * p + 8)) & 0xffu], spread4(sg >> 4));
+        }
+        return r;
+    } else {
+        static_assert(T == T_IQ3_S, "a type of the int8 form");
+        const uint32_t qh = (s < 4 ? f.f.qh.x : f.f.qh.y) >> (8 * (s & 3)), idx = f.f.idx[s];
+        v4i r;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int g = 2 * h + p;
+            const uint32_t sb = (f.f.sg[s] >> (8 * p)) & 0xffu;
+            r[2 * p] = signed_grid(grid[((idx >> (16 * p)) & 0xffu) | (((qh >> (2 * g)) & 1u) << 8)], spread4(sb & 0xfu));
+            r[2 * p + 1] =
+                signed_grid(grid[((idx >> (16 * p + 8)) & 0xffu) | (((qh >> (2 * g + 1)) & 1u) << 8)], spread4(sb >> 4));
+        }
+        return r;
+    }
+}
+template <int T> __device__ __forceinline__ float i8_scale(const I8Frag<T> &f, int s, int h) {
+    if constexpr (T == T_Q8_0) {
+        const int p = s >> 1;
+        const uint32_t own = h ? f.x[p] >> 16 : f.e[p].x & 0xffffu;  // half 0: the even block's d, half 1: the odd one's
+        const uint32_t other = (uint32_t) xor_lane_i<32>((int) own);
+        return half_to_float((s & 1) == h ? own : other);
+    } else if constexpr (T == T_Q4_K || T == T_Q5_K) {
+        const uint4 hd = f.f.h;
+        const uint32_t w = s < 4 ? (hd.y & 0x3F3F3F3Fu) : ((hd.w & kLo4) | ((hd.y >> 2) & 0x30303030u));
+        return half_to_float(hd.x & 0xffffu) * (float) ((w >> (8 * (s & 3))) & 0xffu);
+    } else if constexpr (T == T_IQ4_XS) {
+        const int ls = (int) (((f.f.h.y >> (4 * s)) & 0xfu) | (((f.f.h.x >> (16 + 2 * s)) & 3u) << 4)) - 32;
+        return half_to_float(f.f.h.x & 0xffffu) * (float) ls;
+    } else if constexpr (T == T_IQ3_XXS) {
+        return 0.25f * half_to_float(f.f.d & 0xffffu) * (float) (2 * (int) (word(f.f.aux[s >> 2], s & 3) >> 28) + 1);
+    } else {
+        return half_to_float(f.f.d & 0xffffu) * (float) (2 * (int) ((f.f.sc >> (4 * s)) & 0xfu) + 1);
+    }
+}
+
+// ---- one group ----------------------------------------------------------------------------------------------------
+// LDS: the superblock's codes [rows][256] and scales [8][rows], double-buffered (the 16-byte pieces of row r at piece
+// p ^ (r % 16), so an operand read touches distinct banks), and its min-term sums. 40 KB for 64 rows.
+constexpr int kI8Buf = kMmqTok * kActRow * 4;  // a code buffer, sized for the GLU epilogue's act tile (17 KB)
+struct MmqI8Lds {
+    uint8_t (&q0)[kI8Buf];
+    uint8_t (&q1)[kI8Buf];
+    float (&d)[2][8][kMmqTok];
+    uint8_t (&s)[2][kMmqTok * kRowS];
+    int (&src)[kMmqTok];
+    int (&dst)[kMmqTok];
+    int (&grp)[4];
+    uint32_t *grid;
+};
+
+// Group g, weight row block wb: as mmq_group (4 waves, two 32-row weight streams each, 32 NT activation rows).
+template <int T, bool GLU, int NT>
+__device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, const MmqI8Lds &L) {
+    constexpr int ROWS = 32 * NT, WROWS = GLU ? 128 : 256, BB = Traits<T>::bytes;
+    constexpr bool MIN = T == T_Q4_K || T == T_Q5_K;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+    const int hh = lane / 32, jl = lane % 32;
+    if constexpr (kGridWords<T> > 0) {  // the codebook into LDS (visible after the barriers below)
+        const uint4 *src = (const uint4 *) (T == T_IQ3_XXS ? (const void *) g_iq_grids.iq3xxs : (const void *) g_iq_grids.iq3s);
+        for (int i = tid; i < kGridWords<T> / 4; i += kMmqThreads) ((uint4 *) L.grid)[i] = src[i];
+    }
+    int e, seg, cnt;
+    if (!group_rows<NT>(a, g, L.grp, e, seg, cnt)) return;
+    int *const sh_src = L.src, *const sh_dst = L.dst;
+    for (int i = tid; i < ROWS; i += kMmqThreads) {
+        const int q = seg + min(i, cnt - 1);
+        sh_src[i] = a.src ? a.src[q] : q;
+        sh_dst[i] = a.dst_rows ? a.dst_rows[q] : q;
+    }
+    const uint8_t *wbase = expert_base(a, e);
+    const int nb = a.ncols / 256;
+    const int64_t row_bytes = (int64_t) nb * BB;
+    // weight rows past nrows (nrows % WROWS != 0) are computed from the last row and not stored
+    const int row0 = wb * WROWS + wave * 32 + jl;
+    const int ra = min(row0, a.nrows - 1), rb = GLU ? ra : min(row0 + 128, a.nrows - 1);
+    const Rsrc r0 = rsrc_of(wbase + a.off_a), r1 = rsrc_of(wbase + (GLU ? a.off_b : a.off_a)), rx = rsrc_of(a.xpack);
+    const uint32_t v0 = (uint32_t) (ra * row_bytes), v1 = (uint32_t) (rb * row_bytes);
+    const uint32_t c0 = v0 + 16 * hh, c1 = v1 + 16 * hh;
+    __syncthreads();  // sh_src / sh_dst
+
+    // LDS-DMA of a superblock's codes: instruction u of wave w takes rows 16 u + 4 w .. + 3, 16 lanes per row
+    constexpr int NU = ROWS / 16;
+    uint32_t qo[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        const int r = 16 * u + 4 * wave + lane / 16;
+        qo[u] = (uint32_t) ((size_t) sh_src[r] * a.x_img + 16 * ((lane % 16) ^ (r % 16)));
+    }
+    const int srow = 32 * (wave % NT);
+    const uint32_t so = (uint32_t) ((size_t) sh_src[srow + lane / 2] * a.x_img + kI8Sum + 16 * (lane & 1));
+    // scales: thread t < 2 ROWS reads four of row t / 2 and stores them transposed
+    const bool dthr = tid < 2 * ROWS;
+    const uint32_t dof = (uint32_t) ((size_t) sh_src[(tid / 2) % ROWS] * a.x_img + kI8Scale + 16 * (tid & 1));
+    auto dma_sb = [&](uint8_t *buf, int sb, int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < NU; ++u) dma16(rx, buf + (16 * u + 4 * wave) * 256, qo[u], (uint32_t) (kb * kI8Sb));
+        if constexpr (MIN) dma16(rx, L.s[sb] + srow * kRowS, so, (uint32_t) (kb * kI8Sb));
+    };
+    auto store_d = [&](int sb, const uint4 &v) __attribute__((always_inline)) {
+        if (dthr) {
+            const int r = tid / 2, s = 4 * (tid & 1);
+            L.d[sb][s][r] = __builtin_bit_cast(float, v.x);
+            L.d[sb][s + 1][r] = __builtin_bit_cast(float, v.y);
+            L.d[sb][s + 2][r] = __builtin_bit_cast(float, v.z);
+            L.d[sb][s + 3][r] = __builtin_bit_cast(float, v.w);
+        }
+    };
+    // the superblocks [kb0, kb_end) of this item: all of them, or part blockIdx.y of a split K range
+    int kb0 = 0, kb_end = nb, part = 0;
+    if constexpr (!GLU) {
+        if (a.ksplit > 1) {
+            part = (int) blockIdx.y;
+            kb0 = part * nb / a.ksplit;
+            kb_end = (part + 1) * nb / a.ksplit;
+        }
+    }
+    I8Frag<T> f0, f1, n0, n1;
+    dma_sb(L.q0, 0, kb0);
+    uint4 dv = bload16(rx, dof, (uint32_t) (kb0 * kI8Sb));
+    i8frag_load<T, 0>(r0, v0, c0, (uint32_t) (kb0 * BB), f0);
+    i8frag_load<T, 0>(r1, v1, c1, (uint32_t) (kb0 * BB), f1);
+    store_d(0, dv);
+    dma_wait();
+    lds_barrier();
+
+    v16f acc[NT][2];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][0][r] = acc[t][1][r] = 0.0f;
+
+    // Operands of step i (sub-block i / NT, token tile i % NT) of the superblock in LDS buffer (buf, sb): the tile's codes
+    // and the scales d8 of the 16 tokens this lane holds.
+    struct Step {
+        v4i a;
+        float d[16];
+    };
+    auto load_step = [&](const uint8_t *buf, int sb, int i, Step &o) __attribute__((always_inline)) {
+        const int s = i / NT, t = i % NT, r = t * 32 + jl;
+        if constexpr (T == T_IQ4_XS) {
+            const uint8_t *p0 = buf + r * 256 + 8 * hh;
+            const uint2 lo = *(const uint2 *) (p0 + 16 * ((2 * s) ^ (r & 15)));
+            const uint2 hi = *(const uint2 *) (p0 + 16 * ((2 * s + 1) ^ (r & 15)));
+            o.a = v4i{(int) lo.x, (int) lo.y, (int) hi.x, (int) hi.y};
+        } else {
+            o.a = *(const v4i *) (buf + r * 256 + 16 * ((2 * s + hh) ^ (r & 15)));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 v = *(const float4 *) &L.d[sb][s][t * 32 + 8 * q + 4 * hh];
+            o.d[4 * q] = v.x, o.d[4 * q + 1] = v.y, o.d[4 * q + 2] = v.z, o.d[4 * q + 3] = v.w;
+        }
+    };
+    // Four sub-blocks 4 P .. 4 P + 3, one step at a time (the scheduling barrier keeps the compiler from hoisting the
+    // operands of many steps, which spills); a step's LDS reads are issued during the step before it.
+    auto half_pass = [&](const uint8_t *buf, int sb, auto pc, const I8Frag<T> &f0, const I8Frag<T> &f1) __attribute__((always_inline)) {
+        constexpr int P = decltype(pc)::value;
+        Step cur, nxt;
+        load_step(buf, sb, 4 * P * NT, cur);
+        v4i b0, b1;
+        float w0, w1;
+#pragma unroll
+        for (int i = 4 * P * NT; i < (4 * P + 4) * NT; ++i) {
+            const int s = i / NT, t = i % NT;
+            __builtin_amdgcn_sched_barrier(0);
+            if (t == 0) {
+                b0 = i8_codes<T>(f0, s, hh, L.grid), b1 = i8_codes<T>(f1, s, hh, L.grid);
+                w0 = i8_scale<T>(f0, s, hh), w1 = i8_scale<T>(f1, s, hh);
+            }
+            if (i + 1 < (4 * P + 4) * NT) load_step(buf, sb, i + 1, nxt);
+            const v16i z = {};
+            const v16i i0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a, b0, z, 0, 0, 0);
+            const v16i i1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a, b1, z, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                acc[t][0][q] = fmaf_((float) i0[q], cur.d[q] * w0, acc[t][0][q]);
+                acc[t][1][q] = fmaf_((float) i1[q], cur.d[q] * w1, acc[t][1][q]);
+            }
+            // (pins this step's sums here: instruction selection is free to sink them past the scheduling barriers)
+            asm volatile("" : "+v"(acc[t][0]), "+v"(acc[t][1]));
+            cur = nxt;
+        }
+    };
+    auto superblock = [&](int kb, int sb, uint8_t *buf, uint8_t *nbuf, I8Frag<T> &f0, I8Frag<T> &f1, I8Frag<T> &n0,
+                          I8Frag<T> &n1) __attribute__((always_inline)) {
+        const int kn = kb + 1 < kb_end ? kb + 1 : kb;  // the last superblock reloads itself: the same loads every time
+        dma_sb(nbuf, sb ^ 1, kn);
+        const uint4 dn = bload16(rx, dof, (uint32_t) (kn * kI8Sb));
+        i8frag_load<T, 1>(r0, v0, c0, (uint32_t) (kb * BB), f0);
+        i8frag_load<T, 1>(r1, v1, c1, (uint32_t) (kb * BB), f1);
+        __builtin_amdgcn_sched_barrier(0);
+        half_pass(buf, sb, std::integral_constant<int, 0>{}, f0, f1);
+        __builtin_amdgcn_sched_barrier(0);
+        i8frag_load<T, 0>(r0, v0, c0, (uint32_t) (kn * BB), n0);
+        i8frag_load<T, 0>(r1, v1, c1, (uint32_t) (kn * BB), n1);
+        __builtin_amdgcn_sched_barrier(0);
+        half_pass(buf, sb, std::integral_constant<int, 1>{}, f0, f1);
+        if constexpr (MIN) {  // the min term: acc -= dmin (m . S)
+            const float m0 = -half_to_float(f0.f.h.x >> 16), m1 = -half_to_float(f1.f.h.x >> 16);
+            const v8h bm0 = min_b<T>(f0.f), bm1 = min_b<T>(f1.f);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                v16f z;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) z[r] = 0.0f;
+                const v8h am = *(const v8h *) (L.s[sb] + (t * 32 + jl) * kRowS + 16 * hh);
+                const v16f t0 = mfma32(am, bm0, z), t1 = mfma32(am, bm1, z);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    acc[t][0][r] = fmaf_(m0, t0[r], acc[t][0][r]);
+                    acc[t][1][r] = fmaf_(m1, t1[r], acc[t][1][r]);
+                }
+            }
+        }
+        store_d(sb ^ 1, dn);
+        __builtin_amdgcn_sched_barrier(0);
+        dma_wait();     // the next superblock's codes and sums (and the next weights)
+        lds_barrier();  // visible to every wave; this superblock's buffers are free
+    };
+    for (int kb = kb0; kb < kb_end; kb += 2) {
+        superblock(kb, 0, L.q0, L.q1, f0, f1, n0, n1);
+        if (kb + 1 < kb_end) superblock(kb + 1, 1, L.q1, L.q0, n0, n1, f0, f1);
+    }
+    if constexpr (!GLU) {
+        store_group<NT>(a, acc, sh_dst, cnt, row0, hh, part, false);
+    } else {
+        float *t0 = (float *) L.q0, *t1 = (float *) L.q1;
+        act_to_lds<NT>(acc, t0, t1, wave, jl, hh);
+        __syncthreads();
+        act_blocks(a, t0, t1, sh_dst, cnt, wb, wave, lane, [&](int i, int col, bool live, const float (&v)[8]) {
+            const Q8x8 q = q8_1_x8(v);
+            if (!live) return;
+            uint8_t *row = a.out_pack + (size_t) sh_dst[i] * a.out_img;
+            if (a.out_i8) i8_store(q, row, col);
+            else q8_split_store(q8_split_of(q.q, half_to_float(float_to_half(q.d))), row, a.nrows, col);
+        });
+    }
+}
+
+// Grid as k_mmq's for the expert lists and the shared expert. Dense: the row blocks go to the XCDs in turn and an XCD
+// takes every row group of one block before the next, so each weight byte enters one XCD's L2 and the (small) activation
+// images all eight; with few row blocks (rows_first = 0) the groups go to the XCDs instead, as in k_mmq.
+template <int T, bool GLU>
+__global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mmq_i8(const MmqArgs m,
+                                                                                               const MmqShared sh) {
+    __shared__ __align__(16) uint8_t sh_q0[kI8Buf];
+    __shared__ __align__(16) uint8_t sh_q1[kI8Buf];
+    __shared__ __align__(16) float sh_d[2][8][kMmqTok];
+    __shared__ __align__(16) uint8_t sh_s[2][(T == T_Q4_K || T == T_Q5_K) ? kMmqTok * kRowS : 16];
+    __shared__ __align__(16) uint32_t sh_grid[kGridWords<T> > 0 ? kGridWords<T> : 4];
+    __shared__ int sh_src[kMmqTok], sh_dst[kMmqTok], sh_grp[4];
+    const MmqI8Lds L{sh_q0, sh_q1, sh_d, *(uint8_t (*)[2][kMmqTok * kRowS]) sh_s, sh_src, sh_dst, sh_grp, sh_grid};
+    MmqArgs a;
+    int g, wb;
+    bool one;
+    if (!mmq_item(m, sh, a, g, wb, one)) return;
+    if (one) mmq_group_i8<T, GLU, 1>(a, g, wb, L);
+    else mmq_group_i8<T, GLU, 2>(a, g, wb, L);
+}
+
+template <bool GLU> const void *mmq_i8_kernel(int type) {
+    switch (type) {
+        case T_Q8_0: return (const void *) k_mmq_i8<T_Q8_0, GLU>;
+        case T_Q4_K: return (const void *) k_mmq_i8<T_Q4_K, GLU>;
+        case T_Q5_K: return (const void *) k_mmq_i8<T_Q5_K, GLU>;
+        case T_IQ4_XS: return (const void *) k_mmq_i8<T_IQ4_XS, GLU>;
+        case T_IQ3_XXS: return (const void *) k_mmq_i8<T_IQ3_XXS, GLU>;
+        case T_IQ3_S: return (const void *) k_mmq_i8<T_IQ3_S, GLU>;
+    }
+    return nullptr;
+}
+inline bool mmq_i8_type(int type) { return mmq_i8_kernel<false>(type) != nullptr; }
+
+}  // namespace
+}  // namespace fns

@@ -360,11 +360,13 @@ struct MmqArgs {
     const int32_t *dst_rows;   // sorted position -> output row (null: identity)
     int n_rows;                // dense: number of activation rows
     int dense_small;           // dense: 1 = groups of 32 activation rows (one tile), 0 = of 64
+    int rows_first;            // dense: 1 = row blocks over the XCDs, all groups of a block in turn; 0 = groups over them
     int ksplit;                // dense, non-GLU: > 1 = the K range split into ksplit parts (blockIdx.y), part p's
     int64_t part_stride;       //   partial sums written at dst + p * part_stride floats
     float *dst;                // [out row][nrows] f32 (non-GLU)
     uint8_t *out_pack;         // GLU: act split image rows (by output row)
     int64_t out_img;
+    int out_i8;                // GLU, int8 form: 1 = int8 image rows, 0 = split image rows
     float *act_out;            // GLU: optional f32 act [out row][nrows]
     int *gdone;                // fused launch: per-group arrival counts (zeroed by the compaction kernel)
     int gwait;                 // fused launch: arrivals a down item waits for (its group's gate/up items)
@@ -805,6 +807,105 @@ struct MmqLds {
     uint32_t *grid;  // IQ3_XXS / IQ3_S / IQ2_S: the codebook (kGridWords words)
 };
 
+// Expert e, first sorted row seg and row count cnt (1 .. 32 NT) of group g; false: the group does not exist.
+template <int NT>
+__device__ __forceinline__ bool group_rows(const MmqArgs &a, int g, int (&grp)[4], int &e, int &seg, int &cnt) {
+    const int tid = threadIdx.x;
+    // which expert / rows of activations: thread t < n_expert tests whether group g is expert t's (gp[t] <= g <
+    // gp[t + 1]); all the prefix loads are independent, one round trip, and the one match publishes through LDS
+    e = seg = cnt = 0;
+    if (a.bounds) {
+        const int32_t *gp = NT == 2 ? a.gprefix : a.gprefix + a.n_expert + 1;
+        if (g >= gp[a.n_expert]) return false;
+        if (tid < a.n_expert) {
+            const int g0 = gp[tid], g1 = gp[tid + 1], b0 = a.bounds[tid], b1 = a.bounds[tid + 1];
+            if (g0 <= g && g < g1) {
+                int c, sg;
+                if constexpr (NT == 1) {  // the expert's last rows: n_e % 64 of them
+                    c = (b1 - b0) % kMmqTok;
+                    sg = b1 - c;
+                } else {
+                    sg = b0 + (g - g0) * kMmqTok;
+                    c = min(kMmqTok, b1 - sg);
+                }
+                grp[0] = tid;
+                grp[1] = sg;
+                grp[2] = c;
+            }
+        }
+        __syncthreads();
+        e = __builtin_amdgcn_readfirstlane(grp[0]);
+        seg = __builtin_amdgcn_readfirstlane(grp[1]);
+        cnt = __builtin_amdgcn_readfirstlane(grp[2]);
+    } else {
+        seg = g * 32 * NT;
+        cnt = min(32 * NT, a.n_rows - seg);
+    }
+    return cnt > 0;
+}
+
+// The matrix of expert e (or the dense one), as a scalar, so the weight buffer resources stay in SGPRs.
+__device__ __forceinline__ const uint8_t *expert_base(const MmqArgs &a, int e) {
+    const uint64_t w = (uint64_t) (a.table ? (const uint8_t *) gload<const char *>((const uint8_t *) (a.table + e)) : a.w_dense);
+    return (const uint8_t *) (((uint64_t) __builtin_amdgcn_readfirstlane((uint32_t) (w >> 32)) << 32) |
+                              (uint32_t) __builtin_amdgcn_readfirstlane((uint32_t) w));
+}
+
+// Output rows of a finished group: (token i, weight row row0 and row0 + 128) of acc[t][m][r], i = 32 t + 8 (r / 4) + 4 hh + r % 4
+template <int NT>
+__device__ __forceinline__ void store_group(const MmqArgs &a, const v16f (&acc)[NT][2], const int *dst, int cnt, int row0,
+                                            int hh, int part, bool failed) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = t * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
+            if (i < cnt) {
+                float *o = a.dst + (size_t) part * a.part_stride + (size_t) dst[i] * a.nrows;
+                if (row0 < a.nrows) o[row0] = failed ? __builtin_nanf("") : acc[t][0][r];
+                if (row0 + 128 < a.nrows) o[row0 + 128] = failed ? __builtin_nanf("") : acc[t][1][r];
+            }
+        }
+}
+
+// act = up * silu(gate) of a finished GLU group (reference src/ggml/ggml_mmvq.cu:240-247 epilogue with zero biases;
+// silu(g) = g / (1 + e^-g) from the hardware exp2 and reciprocal, about 2 ulp) into LDS as [token][64 rows] f32 per wave
+// pair: waves 0-1 in t0, waves 2-3 in t1, row stride kActRow floats (16-byte aligned rows).
+constexpr int kActRow = 68;
+template <int NT>
+__device__ __forceinline__ void act_to_lds(const v16f (&acc)[NT][2], float *t0, float *t1, int wave, int jl, int hh) {
+    float *act = wave < 2 ? t0 : t1;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = t * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
+            const float g = acc[t][0][r] + 0.0f;
+            act[i * kActRow + (wave & 1) * 32 + jl] = (acc[t][1][r] + 0.0f) * (g * silu_rcp(g));
+        }
+}
+// Then the Q8_1 blocks (token, 32 rows), 4 lanes per block and 8 values per lane: sink(i, col, live, v) for token i and
+// act column col; the 4 lanes of a block are live together. The f32 act rows too when act_out asks for them.
+template <class Sink>
+__device__ __forceinline__ void act_blocks(const MmqArgs &a, const float *t0, const float *t1, const int *dst, int cnt, int wb,
+                                           int wave, int lane, Sink sink) {
+    for (int p0 = wave * 16; p0 < 4 * cnt; p0 += 16 * kMmqWaves) {  // wave-uniform trip count
+        const int p = p0 + lane / 4, q = lane % 4;
+        const int i = p < 4 * cnt ? p / 4 : 0, blk = p % 4;
+        const int col = wb * 128 + 32 * blk + 8 * q;
+        const bool live = p < 4 * cnt && col < a.nrows;  // the same for the 4 lanes of a block
+        const float *src = (blk < 2 ? t0 : t1) + i * kActRow + 32 * (blk & 1) + 8 * q;
+        const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
+        const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        sink(i, col, live, v);
+        if (live && a.act_out) {
+            float *ao = a.act_out + (size_t) dst[i] * a.nrows + col;
+            *(float4 *) ao = x0;
+            *(float4 *) (ao + 4) = x1;
+        }
+    }
+}
+
 // Group g of the launch's list (NT = 2: the 64-row groups and remainders > 32 rows; NT = 1: the expert's <= 32-row
 // remainder), weight row block wb. DEV: an item of the fused launch (gate/up items count their arrival, down items
 // wait for their group's).
@@ -829,37 +930,8 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
                                                            : (const void *) g_iq_grids.iq2s);
         for (int i = tid; i < kGridWords<T> / 4; i += kMmqThreads) ((uint4 *) L.grid)[i] = src[i];
     }
-    // which expert / rows of activations: thread t < n_expert tests whether group g is expert t's (gp[t] <= g <
-    // gp[t + 1]); all the prefix loads are independent, one round trip, and the one match publishes through LDS
-    int e = 0, seg = 0, cnt = 0;
-    if (a.bounds) {
-        const int32_t *gp = NT == 2 ? a.gprefix : a.gprefix + a.n_expert + 1;
-        if (g >= gp[a.n_expert]) return;
-        if (tid < a.n_expert) {
-            const int g0 = gp[tid], g1 = gp[tid + 1], b0 = a.bounds[tid], b1 = a.bounds[tid + 1];
-            if (g0 <= g && g < g1) {
-                int c, sg;
-                if constexpr (NT == 1) {  // the expert's last rows: n_e % 64 of them
-                    c = (b1 - b0) % kMmqTok;
-                    sg = b1 - c;
-                } else {
-                    sg = b0 + (g - g0) * kMmqTok;
-                    c = min(kMmqTok, b1 - sg);
-                }
-                L.grp[0] = tid;
-                L.grp[1] = sg;
-                L.grp[2] = c;
-            }
-        }
-        __syncthreads();
-        e = __builtin_amdgcn_readfirstlane(L.grp[0]);
-        seg = __builtin_amdgcn_readfirstlane(L.grp[1]);
-        cnt = __builtin_amdgcn_readfirstlane(L.grp[2]);
-    } else {
-        seg = g * ROWS;
-        cnt = min(ROWS, a.n_rows - seg);
-    }
-    if (cnt <= 0) return;
+    int e, seg, cnt;
+    if (!group_rows<NT>(a, g, L.grp, e, seg, cnt)) return;
     MMQ_MARK(0);
     MMQ_NOTE(NT * 1000 + cnt);
     for (int i = tid; i < ROWS; i += kMmqThreads) {
@@ -868,13 +940,7 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
         sh_dst[i] = a.dst_rows ? a.dst_rows[q] : q;
     }
 
-    // (the expert's base as a scalar, so the weight buffer resources stay in SGPRs)
-    const uint8_t *wbase = a.table ? (const uint8_t *) gload<const char *>((const uint8_t *) (a.table + e)) : a.w_dense;
-    {
-        const uint64_t wb64 = (uint64_t) wbase;
-        wbase = (const uint8_t *) (((uint64_t) __builtin_amdgcn_readfirstlane((uint32_t) (wb64 >> 32)) << 32) |
-                                   (uint32_t) __builtin_amdgcn_readfirstlane((uint32_t) wb64));
-    }
+    const uint8_t *wbase = expert_base(a, e);
     const int nb = a.ncols / 256;
     const int64_t row_bytes = (int64_t) nb * BB;
     // weight rows past nrows (nrows % WROWS != 0) are computed from the last row and not stored
@@ -1120,56 +1186,22 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
     }
 
     dma_wait();  // the last (unused) sums load
-    // output (token i, weight row row0) of acc[t][m][r]: i = 32 t + 8 (r / 4) + 4 hh + r % 4
     if constexpr (!GLU) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int i = t * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                if (i < cnt) {
-                    float *o = a.dst + (size_t) part * a.part_stride + (size_t) sh_dst[i] * a.nrows;
-                    if (row0 < a.nrows) o[row0] = failed ? __builtin_nanf("") : acc[t][0][r];
-                    if (row0 + 128 < a.nrows) o[row0 + 128] = failed ? __builtin_nanf("") : acc[t][1][r];
-                }
-            }
+        store_group<NT>(a, acc, sh_dst, cnt, row0, hh, part, failed);
     } else {
-        // act = up * silu(gate) (reference src/ggml/ggml_mmvq.cu:240-247 epilogue with zero biases; silu(g) =
-        // g / (1 + e^-g) from the hardware exp2 and reciprocal, about 2 ulp), staged as [token][64 rows] f32 per wave
-        // pair (waves 0-1 in chunk buffer 0, waves 2-3 in buffer 1; row stride 68 floats: 16-byte aligned rows),
-        // then the Q8_1 blocks (token, 32 rows) into the act split image rows: 4 lanes per block, 8 values per lane
-        constexpr int kAct = 68;
-        static_assert(ROWS * kAct * 4 <= ROWS * kRowA, "act tile fits a chunk buffer");
-        float *act = (float *) (wave < 2 ? sh_a0 : sh_a1);
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int i = t * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                const float g = acc[t][0][r] + 0.0f;
-                act[i * kAct + (wave & 1) * 32 + jl] = (acc[t][1][r] + 0.0f) * (g * silu_rcp(g));
-            }
+        static_assert(ROWS * kActRow * 4 <= ROWS * kRowA, "act tile fits a chunk buffer");
+        act_to_lds<NT>(acc, (float *) sh_a0, (float *) sh_a1, wave, jl, hh);
         __syncthreads();
-        for (int p0 = wave * 16; p0 < 4 * cnt; p0 += 16 * kMmqWaves) {  // wave-uniform trip count
-            const int p = p0 + lane / 4, q = lane % 4;
-            const int i = p < 4 * cnt ? p / 4 : 0, blk = p % 4;
-            const int col = wb * WROWS + 32 * blk + 8 * q;
-            const bool live = p < 4 * cnt && col < a.nrows;  // the same for the 4 lanes of a block
-            const float *src = (const float *) (blk < 2 ? sh_a0 : sh_a1) + i * kAct + 32 * (blk & 1) + 8 * q;
-            const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
-            const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-            // the reference's Q8_1 arithmetic (q = roundf(v / d), IEEE division): the same codes as the quantiser of
-            // the f32 act rows would give
-            if constexpr (DEV)
-                q8_split8_dev(v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img), a.nrows, col, live);
-            else
-                q8_split8<true>(v, a.out_pack + (size_t) sh_dst[i] * a.out_img, a.nrows, col, live);
-            if (live && a.act_out) {
-                float *ao = a.act_out + (size_t) sh_dst[i] * a.nrows + col;
-                *(float4 *) ao = x0;
-                *(float4 *) (ao + 4) = x1;
-            }
-        }
+        // the reference's Q8_1 arithmetic (q = roundf(v / d), IEEE division): the same codes as the quantiser of the f32
+        // act rows would give, written straight into the act split image rows
+        act_blocks(a, (const float *) sh_a0, (const float *) sh_a1, sh_dst, cnt, wb, wave, lane,
+                   [&](int i, int col, bool live, const float (&v)[8]) {
+                       if constexpr (DEV)
+                           q8_split8_dev(v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img), a.nrows, col,
+                                         live);
+                       else
+                           q8_split8<true>(v, a.out_pack + (size_t) sh_dst[i] * a.out_img, a.nrows, col, live);
+                   });
         if constexpr (DEV) {  // every act store of the workgroup has completed: count the arrival
             dma_wait();
             __syncthreads();
@@ -1188,22 +1220,17 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
 // row block; groups go to the XCDs in turn (group u on XCD u % 8) in increasing order.
 // (SPX mode: one partition of all 8 XCDs. In a partitioned mode the mapping is a performance assumption only.)
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
-template <int T, bool GLU>
-__global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mmq(const MmqArgs m,
-                                                                                            const MmqShared sh) {
-    __shared__ __align__(16) uint8_t sh_a0[kMmqTok * kRowA];
-    __shared__ __align__(16) uint8_t sh_a1[kMmqTok * kRowA];
-    __shared__ __align__(16) uint8_t sh_s[(T == T_Q4_K || T == T_Q5_K) ? kMmqTok * kRowS : 16];
-    __shared__ __align__(16) uint32_t sh_grid[kGridWords<T> > 0 ? kGridWords<T> : 4];
-    __shared__ int sh_src[kMmqTok], sh_dst[kMmqTok], sh_grp[4];
-    const MmqLds L{sh_a0, sh_a1, *(uint8_t (*)[kMmqTok * kRowS]) sh_s, sh_src, sh_dst, sh_grp, sh_grid};
-    MmqArgs a = m;
+// Workgroup -> its arguments, group g, weight row block wb and whether the group is one token tile (at most 32 rows);
+// false: nothing to do.
+__device__ __forceinline__ bool mmq_item(const MmqArgs &m, const MmqShared &sh, MmqArgs &a, int &g, int &wb, bool &one) {
+    a = m;
     const bool shared = (int) blockIdx.x < sh.items;
     const int lid = shared ? (int) blockIdx.x : (int) blockIdx.x - sh.items, r = lid / kXcds;
     const int n_cb = shared ? sh.n_cb : m.n_cb;
-    const int j = (r / n_cb) * kXcds + lid % kXcds, wb = r % n_cb;
-    bool one = false;  // a group of at most 32 rows: one token tile
-    int g = j;
+    const int j = (r / n_cb) * kXcds + lid % kXcds, wbj = r % n_cb;
+    one = false;
+    g = j;
+    wb = wbj;
     if (shared) {
         a.table = nullptr;
         a.w_dense = sh.w;
@@ -1219,23 +1246,51 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
         a.out_pack = sh.out_pack;
         a.out_img = sh.out_img;
         a.act_out = nullptr;
-        if (kMmqTok * j >= sh.n_rows) return;
+        if (kMmqTok * j >= sh.n_rows) return false;
         one = sh.n_rows - kMmqTok * j <= kMmqTok / 2;
         if (one) g = 2 * j;
     } else if (m.bounds) {
         // expert path: the groups that exist in this call (the device-side counts of the 64-row list and of the
         // remainder list) take the first workgroups; the rest of the grid (sized for the upper bound) returns at once
         const int nm = m.gprefix[m.n_expert], nr = m.gprefix[2 * (m.n_expert + 1) - 1];
-        if (j >= nm + nr) return;
+        if (j >= nm + nr) return false;
         one = j >= nm;
         if (one) g = j - nm;
     } else {
-        if (j >= m.n_groups) return;
+        if (m.rows_first) {
+            wb = (r / m.n_groups) * kXcds + lid % kXcds;
+            g = r % m.n_groups;
+            if (wb >= n_cb) return false;
+        } else if (j >= m.n_groups) {
+            return false;
+        }
         one = m.dense_small != 0;
     }
+    return true;
+}
+
+template <int T, bool GLU>
+__global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mmq(const MmqArgs m,
+                                                                                            const MmqShared sh) {
+    __shared__ __align__(16) uint8_t sh_a0[kMmqTok * kRowA];
+    __shared__ __align__(16) uint8_t sh_a1[kMmqTok * kRowA];
+    __shared__ __align__(16) uint8_t sh_s[(T == T_Q4_K || T == T_Q5_K) ? kMmqTok * kRowS : 16];
+    __shared__ __align__(16) uint32_t sh_grid[kGridWords<T> > 0 ? kGridWords<T> : 4];
+    __shared__ int sh_src[kMmqTok], sh_dst[kMmqTok], sh_grp[4];
+    const MmqLds L{sh_a0, sh_a1, *(uint8_t (*)[kMmqTok * kRowS]) sh_s, sh_src, sh_dst, sh_grp, sh_grid};
+    MmqArgs a;
+    int g, wb;
+    bool one;
+    if (!mmq_item(m, sh, a, g, wb, one)) return;
     if (one) mmq_group<T, GLU, 1, false>(a, g, wb, L);
     else mmq_group<T, GLU, 2, false>(a, g, wb, L);
 }
+
+}  // namespace
+}  // namespace fns
+#include "fns_mmq_i8.hpp"
+namespace fns {
+namespace {
 
 // Gate/up (with SwiGLU and the Q8_1 of act) and down of the expert path in one launch. The gate/up items come first,
 // in the order and XCD mapping of k_mmq (group g's weight row blocks on XCD g % 8), then the down items with the same
@@ -1332,9 +1387,11 @@ template <bool GLU> const void *mmq_kernel(int type) {
 
 // groups: upper bound of the 64-row list; expert path: of the 64-row list and the <= 32-row remainders together (the
 // workgroups past the device-side counts return at once)
-// sh: a dense matrix of the same type whose groups come first in the grid (expert path only)
-int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st, const MmqShared *sh = nullptr) {
-    const void *fn = glu ? mmq_kernel<true>(type) : mmq_kernel<false>(type);
+// sh: a dense matrix of the same type whose groups come first in the grid (expert path only); i8: the int8 form
+int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st, const MmqShared *sh = nullptr,
+               bool i8 = false) {
+    const void *fn = i8 ? (glu ? mmq_i8_kernel<true>(type) : mmq_i8_kernel<false>(type))
+                        : (glu ? mmq_kernel<true>(type) : mmq_kernel<false>(type));
     if (!fn) return host::set_error(host::ERR_TYPE, "mmq: type %d not supported", type);
     if (groups <= 0) return host::OK;
     MmqArgs arg = a;
@@ -1365,7 +1422,9 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
         total = (a.n_rows + 31) / 32;
     }
     arg.n_groups = total;
-    const int64_t items = sh_items + (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds);
+    arg.rows_first = i8 && !a.bounds && (arg.n_cb % kXcds == 0 || arg.n_cb >= 4 * kXcds);
+    const int64_t items = sh_items + (arg.rows_first ? (int64_t) total * kXcds * ((arg.n_cb + kXcds - 1) / kXcds)
+                                                     : (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds));
     if (items > INT32_MAX) return host::set_error(host::ERR_SHAPE, "mmq: grid too large");
     shared.items = (int) sh_items;
     const hipError_t e = hipLaunchKernel(fn, dim3((unsigned) items, (unsigned) ks), dim3(kMmqThreads), args, 0, st);
@@ -1438,6 +1497,30 @@ int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, void *xpack, hi
     hipLaunchKernelGGL(k_quant_image, dim3((unsigned) ((ncols + 2047) / 2048), (unsigned) rows), dim3(256), 0, st, x, (int) ncols,
                        (uint8_t *) xpack, (int64_t) mmq_image_bytes(ncols));
     return host::check_launch("mmq quantize");
+}
+
+// The int8 form's image rows of x, and of RMSNorm(x) (out as f32 too; the shapes of mmq_rms_norm_image_fits).
+size_t mmq_i8_image_bytes(int64_t ncols) { return (size_t) i8_row_bytes(ncols); }
+int mmq_quant_i8(const float *x, int64_t ncols, int64_t rows, void *ximg, hipStream_t st) {
+    if (!x || !ximg || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
+        return host::set_error(host::ERR_SHAPE, "mmq quantize: bad arguments");
+    if (rows == 0) return host::OK;
+    hipLaunchKernelGGL(k_quant_i8, dim3((unsigned) ((ncols + 2047) / 2048), (unsigned) rows), dim3(256), 0, st, x, (int) ncols,
+                       (uint8_t *) ximg, (int64_t) mmq_i8_image_bytes(ncols));
+    return host::check_launch("mmq quantize (int8)");
+}
+int mmq_rms_norm_i8(const float *x, const float *w, float *out, int n, float eps, int rows, void *ximg, hipStream_t st) {
+    if (!x || !w || !out || !ximg || rows < 0 || !mmq_rms_norm_image_fits(x, w, out, n))
+        return host::set_error(host::ERR_SHAPE, "mmq rms_norm: bad arguments");
+    if (rows == 0) return host::OK;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned) rows), dim3(256), 0, st, x, w, out, n, eps, (uint8_t *) ximg,
+                           (int64_t) mmq_i8_image_bytes(n));
+    };
+    if (n <= 2048) go(k_rms_norm_i8<1>);
+    else if (n <= 4096) go(k_rms_norm_i8<2>);
+    else go(k_rms_norm_i8<4>);
+    return host::check_launch("mmq rms_norm (int8)");
 }
 
 // RMSNorm of x (f32 [rows][n]) into out, its Q8_1 blocks into xq (null: none) and its split image rows into ximg, for
@@ -1523,20 +1606,9 @@ int expert_args(int type, const char *const *table, size_t off_a, size_t off_b, 
     return host::OK;
 }
 
-int mmq_gemm_experts(int type, const char *const *table, size_t off_a, size_t off_b, bool glu, int64_t ncols,
-                     int64_t nrows, int64_t n_expert, const void *xpack, int64_t n_pairs, const int32_t *ids_src1,
-                     const int32_t *ids_dst, const int32_t *bounds, const int32_t *gprefix, float *dst, void *out_pack,
-                     float *act_out, hipStream_t st) {
-    MmqArgs a;
-    FNS_TRY(expert_args(type, table, off_a, off_b, glu, ncols, nrows, n_expert, xpack, ids_src1, ids_dst, bounds,
-                        gprefix, dst, out_pack, act_out, a));
-    return launch_mmq(type, glu, a, (int) main_groups(n_expert, n_pairs), st);
-}
-
-// Q8_0 (the reference's dense and output-head type, src/ggml/ggml_mmq.cu:59) takes the GEMV kernels, a few token
-// columns per weight pass: each 32-value block is d_w * d8 * (integer dot) in both, so the results are those of a
-// GEMM over the same Q8_1 activations; the bytes are re-read per column group (the tiled GEMM covers the expert
-// K-quant and IQ formats, whose sub-block scales fold into exact f16 operands; Q8_0's float block scale does not).
+// Q8_0 (the reference's dense and output-head type, src/ggml/ggml_mmq.cu:59) takes the int8 form of the GEMM, and for
+// row counts that are not a multiple of 64 the GEMV kernels, a few token columns per weight pass. The K-quants and IQ
+// types keep the split image in the caller's scratch.
 int mmq(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, int64_t n_tok, void *xq, float *dst,
         hipStream_t st) {
     if (type == T_Q8_0 && nrows % kMmqRows) {  // the GEMV kernels (any row count), a few token columns per pass
@@ -1549,16 +1621,17 @@ int mmq(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, i
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
     if (!w || !x || !xq || !dst || n_tok < 0) return host::set_error(host::ERR_SHAPE, "mmq: bad arguments");
     if (n_tok == 0) return host::OK;
-    FNS_TRY(mmq_quant_image(x, ncols, n_tok, xq, st));
+    const bool i8 = type == T_Q8_0;
+    FNS_TRY(i8 ? mmq_quant_i8(x, ncols, n_tok, xq, st) : mmq_quant_image(x, ncols, n_tok, xq, st));
     MmqArgs a{};
     a.w_dense = (const uint8_t *) w;
     a.ncols = (int) ncols;
     a.nrows = (int) nrows;
     a.xpack = (const uint8_t *) xq;
-    a.x_img = (int64_t) mmq_image_bytes(ncols);
+    a.x_img = (int64_t) (i8 ? mmq_i8_image_bytes(ncols) : mmq_image_bytes(ncols));
     a.n_rows = (int) n_tok;
     a.dst = dst;
-    return launch_mmq(type, false, a, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st);
+    return launch_mmq(type, false, a, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, i8);
 }
 
 int mmq_experts(int type, const char *const *table, size_t off, int64_t ncols, int64_t nrows, int64_t n_expert,
@@ -1584,9 +1657,12 @@ int mmq_experts(int type, const char *const *table, size_t off, int64_t ncols, i
     const int64_t rows = n_tok * x_rows_per_tok;
     int32_t *gprefix = (int32_t *) ((uint8_t *) xq + (size_t) rows * mmq_image_bytes(ncols));
     FNS_TRY(mmq_compact(ids, n_tok, n_used, n_expert, x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, st));
-    FNS_TRY(mmq_quant_image(x, ncols, rows, xq, st));
-    return mmq_gemm_experts(type, table, off, 0, false, ncols, nrows, n_expert, xq, n_tok * n_used, ids_src1, ids_dst,
-                            bounds, gprefix, dst, nullptr, nullptr, st);
+    const bool i8 = type == T_Q8_0;
+    FNS_TRY(i8 ? mmq_quant_i8(x, ncols, rows, xq, st) : mmq_quant_image(x, ncols, rows, xq, st));
+    MmqArgs a;
+    FNS_TRY(expert_args(type, table, off, 0, false, ncols, nrows, n_expert, xq, ids_src1, ids_dst, bounds, gprefix, dst,
+                        nullptr, nullptr, a, i8 ? mmq_i8_image_bytes(ncols) : 0));
+    return launch_mmq(type, false, a, (int) main_groups(n_expert, n_tok * n_used), st, nullptr, i8);
 }
 
 // ---- prefill MoE layer ----------------------------------------------------------------------------------------
@@ -1688,15 +1764,18 @@ int mmq_dense_shared(int type, bool glu, const MmqShared &s, hipStream_t st) {
 
 // Dense GEMMs on activation images already built (the dense FFN block): gate/up in one GLU launch (SwiGLU and the
 // Q8_1 of act in the epilogue, act images out), and a plain launch whose K range may be split into ksplit parts
-// (dst then holds ksplit partial sums, part_stride floats apart).
+// (dst then holds ksplit partial sums, part_stride floats apart). x_i8: the activations are int8 image rows and the
+// launch the int8 form; act_i8: so are the act rows written.
 bool mmq_tiled(int type, int64_t ncols, int64_t nrows) {
     const bool t = host::is_kquant(type) || type == T_Q8_0 || (host::is_iq(type) && (!host::iq_needs_grid(type) ||
                                                                                       host::iq_grids_ready()));
     return t && ncols > 0 && ncols % 256 == 0 && ncols <= 65536 && nrows > 0 && nrows % kMmqRows == 0;
 }
 
+bool mmq_i8(int type) { return mmq_i8_type(type); }
+
 int mmq_dense_glu(int type, const void *gate, const void *up, int64_t ncols, int64_t nrows, const void *ximg,
-                  int64_t n_tok, void *act_img, hipStream_t st) {
+                  int64_t n_tok, void *act_img, bool x_i8, bool act_i8, hipStream_t st) {
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
     MmqArgs g{};
     g.w_dense = (const uint8_t *) gate;
@@ -1705,27 +1784,28 @@ int mmq_dense_glu(int type, const void *gate, const void *up, int64_t ncols, int
     g.ncols = (int) ncols;
     g.nrows = (int) nrows;
     g.xpack = (const uint8_t *) ximg;
-    g.x_img = (int64_t) mmq_image_bytes(ncols);
+    g.x_img = (int64_t) (x_i8 ? mmq_i8_image_bytes(ncols) : mmq_image_bytes(ncols));
     g.n_rows = (int) n_tok;
     g.out_pack = (uint8_t *) act_img;
-    g.out_img = (int64_t) mmq_image_bytes(nrows);
-    return launch_mmq(type, true, g, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st);
+    g.out_img = (int64_t) (act_i8 ? mmq_i8_image_bytes(nrows) : mmq_image_bytes(nrows));
+    g.out_i8 = act_i8;
+    return launch_mmq(type, true, g, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, x_i8);
 }
 
 int mmq_dense_parts(int type, const void *w, int64_t ncols, int64_t nrows, const void *ximg, int64_t n_tok, float *dst,
-                    int ksplit, hipStream_t st) {
+                    int ksplit, bool x_i8, hipStream_t st) {
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
     MmqArgs d{};
     d.w_dense = (const uint8_t *) w;
     d.ncols = (int) ncols;
     d.nrows = (int) nrows;
     d.xpack = (const uint8_t *) ximg;
-    d.x_img = (int64_t) mmq_image_bytes(ncols);
+    d.x_img = (int64_t) (x_i8 ? mmq_i8_image_bytes(ncols) : mmq_image_bytes(ncols));
     d.n_rows = (int) n_tok;
     d.dst = dst;
     d.ksplit = ksplit;
     d.part_stride = n_tok * nrows;
-    return launch_mmq(type, false, d, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st);
+    return launch_mmq(type, false, d, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, x_i8);
 }
 
 namespace {

@@ -1,0 +1,64 @@
+"""The grouped GEMM's int8 form (types whose scales change every 32 columns) through the dense FFN block's prefill:
+every type, at the edges of its 32-row tiles and 64-row groups, both grid orders (few and many weight row blocks) and a
+split K range, against the float64 chain of dequantised weights and activations.
+
+Bars: act is re-quantised to 8 bits inside the block, so a code whose quotient lies on a rounding boundary may move one
+step where two fp32 sums differ in their last bits (about one code in 10^4, so at most two in a row of 1024). One step
+moves an output by at most max|act| / 127 * max|w_down|: two such steps plus 1e-5 of the largest output (32-bit sums, and
+the residual's rounding) bound every element; the relative L2 bound is that of the independent chains in
+tests/helpers.py."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from tests.helpers import CHAIN_L2_TOL, gaussian, rel_l2
+from tests.iq_data import random_blocks, register_grids, register_grids_in_library
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [orc.Q8_0, orc.Q4_K, orc.Q5_K, orc.IQ4_XS, orc.IQ3_XXS, orc.IQ3_S]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from flintnsteel_amd import ops as o
+    register_grids_in_library(register_grids())
+    return o
+
+
+def weights(qtype: int, nrows: int, ncols: int, seed: int) -> np.ndarray:
+    if qtype in (orc.IQ4_XS, orc.IQ3_XXS, orc.IQ3_S):
+        return random_blocks(qtype, nrows, ncols, seed)
+    w = gaussian(np.random.default_rng(seed), (nrows, ncols), 0.02)
+    w[:, 256:512] *= 3e-4   # small sub-block scales
+    w[1, :256] = 0.0        # a block with d = 0
+    return orc.quantize(qtype, w)
+
+
+def dequant(qtype: int, w: np.ndarray, nrows: int, ncols: int) -> np.ndarray:
+    return np.asarray(orc.dequantize(qtype, w.reshape(nrows, -1), ncols), np.float64).reshape(nrows, ncols)
+
+
+@pytest.mark.parametrize("T,H,F", [(1, 512, 768), (33, 512, 768), (65, 512, 768), (130, 2048, 1024)])
+@pytest.mark.parametrize("qtype", TYPES)
+def test_dense_prefill_int8(ops, qtype, T, H, F):
+    rng = np.random.default_rng(T + H)
+    g, u, d = weights(qtype, F, H, 1), weights(qtype, F, H, 2), weights(qtype, H, F, 3)
+    x = gaussian(rng, (T, H))
+    x[0, :64] = 0.0  # blocks with amax = 0
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    ffn = ops.DenseFfn(dev(g), dev(u), dev(d), qtype, qtype, qtype, H, F)
+    got = ffn(dev(x), prefill=True)
+    torch.cuda.synchronize()
+    xq = orc.dequantize_q8_1(orc.quantize_q8_1(x), H)
+    gate, up = xq @ dequant(qtype, g, F, H).T, xq @ dequant(qtype, u, F, H).T
+    act = (up * gate / (1 + np.exp(-gate))).astype(np.float32)
+    down = dequant(qtype, d, H, F)
+    ref = orc.dequantize_q8_1(orc.quantize_q8_1(act), F) @ down.T
+    err = np.abs(got.cpu().numpy().astype(np.float64) - x - ref)
+    bound = 2 * np.abs(act).max() / 127 * np.abs(down).max() + 1e-5 * np.abs(ref).max()
+    l2 = rel_l2(got.cpu().numpy().astype(np.float64) - x, ref)
+    assert err.max() <= bound and l2 <= CHAIN_L2_TOL, f"max err {err.max():.3e} (bound {bound:.3e}), rel L2 {l2:.3e}"
