@@ -81,23 +81,22 @@ int dense_ffn(const FnsDenseFfn *D, const float *x, float *out, int64_t n_tok, v
         // the tiled GEMMs on images built once: x image, gate + up in one launch (SwiGLU and the Q8_1 of act in its
         // epilogue, the act images land in the gate/act region), down with its K range split so that the launch
         // fills the GPU, then out = x + (sum of the parts)
-        const bool x_i8 = mmq_i8(D->gate_type), act_i8 = x_i8 && mmq_i8(D->down_type);
+        const int x_form = mmq_form(D->gate_type), act_form = mmq_form(D->down_type);
         if (D->ffn_norm && mmq_rms_norm_image_fits(x, D->ffn_norm, w.h, H)) {
-            FNS_TRY(x_i8 ? mmq_rms_norm_i8(x, D->ffn_norm, w.h, H, D->norm_eps, n, w.xq, st)
-                         : mmq_rms_norm_image(x, D->ffn_norm, w.h, nullptr, H, D->norm_eps, n, w.xq, st));
+            FNS_TRY(mmq_rms_norm_image(x, D->ffn_norm, w.h, nullptr, H, D->norm_eps, n, x_form, w.xq, st));
         } else {
             if (D->ffn_norm) {
                 FNS_TRY(rms_norm_q8_1(x, D->ffn_norm, w.h, w.xq, H, D->norm_eps, n, st));
                 h = w.h;
             }
-            FNS_TRY(x_i8 ? mmq_quant_i8(h, H, n_tok, w.xq, st) : mmq_quant_image(h, H, n_tok, w.xq, st));
+            FNS_TRY(mmq_quant_image(h, H, n_tok, x_form, w.xq, st));
         }
         void *act_img = w.gate;  // n x F image bytes (at most 4.125 per value) fit the gate and act regions together
-        FNS_TRY(mmq_dense_glu(D->gate_type, D->gate, D->up, H, F, w.xq, n_tok, act_img, x_i8, act_i8, st));
+        FNS_TRY(mmq_dense_glu(D->gate_type, D->gate, D->up, H, F, w.xq, n_tok, act_img, x_form, act_form, st));
         const int64_t items = (n_tok + 63) / 64 * ((H + 255) / 256);
         int parts = 1;
         while (parts < kMaxParts && items * parts * 2 <= 512 && F / 256 >= parts * 2) parts *= 2;
-        FNS_TRY(mmq_dense_parts(D->down_type, D->down, F, H, act_img, n_tok, w.parts, parts, act_i8, st));
+        FNS_TRY(mmq_dense_parts(D->down_type, D->down, F, H, act_img, n_tok, w.parts, parts, act_form, st));
         return add_parts(x, w.parts, parts, out, (int64_t) n * H, st);
     }
     if (prefill) {

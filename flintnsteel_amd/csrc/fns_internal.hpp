@@ -63,24 +63,22 @@ int moe_layer_stage(const FnsMoeLayer *L, int stage, const float *x, const float
 size_t mmq_image_bytes(int64_t ncols);
 size_t mmq_q8_1_bytes(int64_t ncols, int64_t nrows);
 size_t mmq_bounds_bytes(int64_t n_expert);
-int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, void *xpack, hipStream_t st);
+int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, int form, void *ximg, hipStream_t st);
 bool mmq_rms_norm_image_fits(const float *x, const float *w, const float *out, int64_t n);
-int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, void *ximg,
-                       hipStream_t st);
-int mmq_guard_image(float *act, float *escale, int64_t ncols, int64_t rows, void *img, int64_t stride, hipStream_t st);
+int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, int form,
+                       void *ximg, hipStream_t st);
+int mmq_guard_image(float *act, float *escale, int64_t ncols, int64_t rows, int form, void *img, int64_t stride,
+                    hipStream_t st);
 int mmq_compact(const int32_t *ids, int64_t n_tok, int64_t k, int64_t n_expert, int64_t x_rows_per_tok,
                 int32_t *ids_src1, int32_t *ids_dst, int32_t *bounds, int32_t *gprefix, hipStream_t st,
                 int32_t *gdone = nullptr, int n_gdone = 0);
-bool mmq_i8(int type);  // a type of the GEMM's int8 form
-size_t mmq_i8_image_bytes(int64_t ncols);
-int mmq_quant_i8(const float *x, int64_t ncols, int64_t rows, void *ximg, hipStream_t st);
-int mmq_rms_norm_i8(const float *x, const float *w, float *out, int n, float eps, int rows, void *ximg, hipStream_t st);
+int mmq_form(int type);  // the form of the activation image that a type's GEMM prefers
 int mmq(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, int64_t n_tok, void *xq, float *dst,
         hipStream_t st);
 int mmq_dense_glu(int type, const void *gate, const void *up, int64_t ncols, int64_t nrows, const void *ximg,
-                  int64_t n_tok, void *act_img, bool x_i8, bool act_i8, hipStream_t st);
+                  int64_t n_tok, void *act_img, int x_form, int act_form, hipStream_t st);
 int mmq_dense_parts(int type, const void *w, int64_t ncols, int64_t nrows, const void *ximg, int64_t n_tok, float *dst,
-                    int ksplit, bool x_i8, hipStream_t st);
+                    int ksplit, int x_form, hipStream_t st);
 bool mmq_tiled(int type, int64_t ncols, int64_t nrows);  // the tiled GEMM takes this type and shape
 int add_parts(const float *x, const float *parts, int n_parts, float *out, int64_t n, hipStream_t st);
 int mmq_experts(int type, const char *const *table, size_t off, int64_t ncols, int64_t nrows, int64_t n_expert,

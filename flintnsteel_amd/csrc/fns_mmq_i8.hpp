@@ -16,58 +16,6 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-// ---- activation image ---------------------------------------------------------------------------------------------
-// Row layout, per 256-column superblock kb at kb * 320: the 256 int8 codes, the 8 block scales d8 (f32, f16 values),
-// the min-term sums [S_hi 8 f16][S_lo 8 f16] of the split image (same order).
-constexpr int kI8Sb = 320, kI8Scale = 256, kI8Sum = 288;
-__host__ __device__ constexpr int64_t i8_row_bytes(int64_t ncols) { return ncols / 256 * kI8Sb; }
-
-// the lane's part of a quantised block (8 codes at column col, a multiple of 8; scale dh): the block's first lane also
-// stores the scale and the sums
-__device__ __forceinline__ void i8_store(const Q8x8 &r, uint8_t *row, int col) {
-    uint8_t *sb = row + (size_t) (col >> 8) * kI8Sb;
-    uint32_t w[2] = {0, 0};
-    int qsum = 0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        w[k / 4] |= (uint32_t) (uint8_t) (int8_t) r.q[k] << (8 * (k % 4));
-        qsum += r.q[k];
-    }
-    *(uint2 *) (sb + (col & 255)) = make_uint2(w[0], w[1]);
-    qsum = lanes_sum_i<4>(qsum);
-    if ((col & 31) == 0) {
-        const int s = (col >> 5) & 7;
-        const float dh = half_to_float(float_to_half(r.d)), sv = dh * (float) qsum;  // exact in fp32
-        const _Float16 hi = (_Float16) sv;
-        *(float *) (sb + kI8Scale + 4 * s) = dh;
-        _Float16 *m = (_Float16 *) (sb + kI8Sum + 2 * perm8(s));
-        m[0] = hi;
-        m[8] = (_Float16) (sv - (float) hi);
-    }
-}
-
-// x [rows][ncols] f32 -> image rows; grid (ceil(ncols / 2048), rows), 256 threads of 8 columns each
-__global__ __launch_bounds__(256) void k_quant_i8(const float *__restrict__ x, int ncols, uint8_t *__restrict__ out,
-                                                  int64_t img_row_bytes) {
-    const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * 8;
-    if (col >= ncols) return;
-    const float *src = x + (size_t) row * ncols + col;
-    const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
-    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    i8_store(q8_1_x8(v), out + (size_t) row * img_row_bytes, col);
-}
-
-// RMSNorm of a row of at most 2048 C columns (fns_q8x8.hpp), out as f32 and as an image row.
-template <int C>
-__global__ __launch_bounds__(256) void k_rms_norm_i8(const float *__restrict__ x, const float *__restrict__ w,
-                                                     float *__restrict__ out, int n, float eps, uint8_t *__restrict__ img,
-                                                     int64_t img_row_bytes) {
-    __shared__ __align__(16) float xs[2048 * C];
-    const size_t r = blockIdx.x;
-    uint8_t *row = img + r * img_row_bytes;
-    rms_norm_row<C>(x + r * n, w, out + r * n, nullptr, n, eps, xs, [&](const Q8x8 &q, int col) { i8_store(q, row, col); });
-}
-
 // ---- weight fragments ---------------------------------------------------------------------------------------------
 // The types of the f16 form keep their fragments (WFrag). Q8_0 (blocks of 34 bytes, f16 d then 32 codes): blocks e = 2 p
 // and e + 1 start at 68 p, a multiple of four; lane half h reads the even block's 16 codes as the 20 aligned bytes at
@@ -176,17 +124,22 @@ struct MmqI8Lds {
     uint32_t *grid;
 };
 
-// Group g, weight row block wb: as mmq_group (4 waves, two 32-row weight streams each, 32 NT activation rows).
-template <int T, bool GLU, int NT>
+// the type's codebook into LDS (visible after the barriers that follow)
+template <int T> __device__ __forceinline__ void grid_to_lds(const MmqI8Lds &L) {
+    if constexpr (kGridWords<T> > 0) {
+        const uint4 *src = (const uint4 *) (T == T_IQ3_XXS ? (const void *) g_iq_grids.iq3xxs : (const void *) g_iq_grids.iq3s);
+        for (int i = threadIdx.x; i < kGridWords<T> / 4; i += kMmqThreads) ((uint4 *) L.grid)[i] = src[i];
+    }
+}
+// Group g, weight row block wb: as mmq_group (4 waves, two 32-row weight streams each, 32 NT activation rows; DEV: an item
+// of the fused launch).
+template <int T, bool GLU, int NT, bool DEV>
 __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, const MmqI8Lds &L) {
     constexpr int ROWS = 32 * NT, WROWS = GLU ? 128 : 256, BB = Traits<T>::bytes;
     constexpr bool MIN = T == T_Q4_K || T == T_Q5_K;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
     const int hh = lane / 32, jl = lane % 32;
-    if constexpr (kGridWords<T> > 0) {  // the codebook into LDS (visible after the barriers below)
-        const uint4 *src = (const uint4 *) (T == T_IQ3_XXS ? (const void *) g_iq_grids.iq3xxs : (const void *) g_iq_grids.iq3s);
-        for (int i = tid; i < kGridWords<T> / 4; i += kMmqThreads) ((uint4 *) L.grid)[i] = src[i];
-    }
+    grid_to_lds<T>(L);
     int e, seg, cnt;
     if (!group_rows<NT>(a, g, L.grp, e, seg, cnt)) return;
     int *const sh_src = L.src, *const sh_dst = L.dst;
@@ -207,6 +160,7 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
     __syncthreads();  // sh_src / sh_dst
 
     // LDS-DMA of a superblock's codes: instruction u of wave w takes rows 16 u + 4 w .. + 3, 16 lanes per row
+    constexpr int CPOL = DEV && !GLU ? kCpolDevice : 0;  // the fused down items read this launch's act rows
     constexpr int NU = ROWS / 16;
     uint32_t qo[NU];
 #pragma unroll
@@ -221,8 +175,12 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
     const uint32_t dof = (uint32_t) ((size_t) sh_src[(tid / 2) % ROWS] * a.x_img + kI8Scale + 16 * (tid & 1));
     auto dma_sb = [&](uint8_t *buf, int sb, int kb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < NU; ++u) dma16(rx, buf + (16 * u + 4 * wave) * 256, qo[u], (uint32_t) (kb * kI8Sb));
-        if constexpr (MIN) dma16(rx, L.s[sb] + srow * kRowS, so, (uint32_t) (kb * kI8Sb));
+        for (int u = 0; u < NU; ++u) dma16<CPOL>(rx, buf + (16 * u + 4 * wave) * 256, qo[u], (uint32_t) (kb * kI8Sb));
+        if constexpr (MIN) dma16<CPOL>(rx, L.s[sb] + srow * kRowS, so, (uint32_t) (kb * kI8Sb));
+    };
+    auto load_d = [&](int kb) __attribute__((always_inline)) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rx, dof, (uint32_t) (kb * kI8Sb), CPOL);
+        return make_uint4(v[0], v[1], v[2], v[3]);
     };
     auto store_d = [&](int sb, const uint4 &v) __attribute__((always_inline)) {
         if (dthr) {
@@ -235,7 +193,7 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
     };
     // the superblocks [kb0, kb_end) of this item: all of them, or part blockIdx.y of a split K range
     int kb0 = 0, kb_end = nb, part = 0;
-    if constexpr (!GLU) {
+    if constexpr (!GLU && !DEV) {
         if (a.ksplit > 1) {
             part = (int) blockIdx.y;
             kb0 = part * nb / a.ksplit;
@@ -243,11 +201,20 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
         }
     }
     I8Frag<T> f0, f1, n0, n1;
-    dma_sb(L.q0, 0, kb0);
-    uint4 dv = bload16(rx, dof, (uint32_t) (kb0 * kI8Sb));
-    i8frag_load<T, 0>(r0, v0, c0, (uint32_t) (kb0 * BB), f0);
-    i8frag_load<T, 0>(r1, v1, c1, (uint32_t) (kb0 * BB), f1);
-    store_d(0, dv);
+    bool failed = false;
+    if constexpr (DEV && !GLU) {  // the first weights in flight, then the wait for the group's act rows
+        i8frag_load<T, 0>(r0, v0, c0, 0, f0);
+        i8frag_load<T, 0>(r1, v1, c1, 0, f1);
+        failed = wait_group(a, NT == 2 ? g : a.n_main + g, &L.grp[3]);
+        dma_sb(L.q0, 0, 0);
+        store_d(0, load_d(0));
+    } else {
+        dma_sb(L.q0, 0, kb0);
+        const uint4 dv = load_d(kb0);
+        i8frag_load<T, 0>(r0, v0, c0, (uint32_t) (kb0 * BB), f0);
+        i8frag_load<T, 0>(r1, v1, c1, (uint32_t) (kb0 * BB), f1);
+        store_d(0, dv);
+    }
     dma_wait();
     lds_barrier();
 
@@ -257,34 +224,32 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][0][r] = acc[t][1][r] = 0.0f;
 
-    // Operands of step i (sub-block i / NT, token tile i % NT) of the superblock in LDS buffer (buf, sb): the tile's codes
-    // and the scales d8 of the 16 tokens this lane holds.
-    struct Step {
-        v4i a;
-        float d[16];
-    };
-    auto load_step = [&](const uint8_t *buf, int sb, int i, Step &o) __attribute__((always_inline)) {
+    // The codes of step i (sub-block i / NT, token tile i % NT) of the superblock in LDS buffer buf, and the scales d8 of
+    // the 16 tokens of the tile that this lane holds.
+    auto load_step = [&](const uint8_t *buf, int i) __attribute__((always_inline)) {
         const int s = i / NT, t = i % NT, r = t * 32 + jl;
+        const uint8_t *row = buf + r * 256;
         if constexpr (T == T_IQ4_XS) {
-            const uint8_t *p0 = buf + r * 256 + 8 * hh;
-            const uint2 lo = *(const uint2 *) (p0 + 16 * ((2 * s) ^ (r & 15)));
-            const uint2 hi = *(const uint2 *) (p0 + 16 * ((2 * s + 1) ^ (r & 15)));
-            o.a = v4i{(int) lo.x, (int) lo.y, (int) hi.x, (int) hi.y};
+            const uint2 lo = *(const uint2 *) (row + 8 * hh + 16 * ((2 * s) ^ (r & 15)));
+            const uint2 hi = *(const uint2 *) (row + 8 * hh + 16 * ((2 * s + 1) ^ (r & 15)));
+            return v4i{(int) lo.x, (int) lo.y, (int) hi.x, (int) hi.y};
         } else {
-            o.a = *(const v4i *) (buf + r * 256 + 16 * ((2 * s + hh) ^ (r & 15)));
+            return *(const v4i *) (row + 16 * ((2 * s + hh) ^ (r & 15)));
         }
+    };
+    auto load_scales = [&](int sb, int i, float (&d)[16]) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const float4 v = *(const float4 *) &L.d[sb][s][t * 32 + 8 * q + 4 * hh];
-            o.d[4 * q] = v.x, o.d[4 * q + 1] = v.y, o.d[4 * q + 2] = v.z, o.d[4 * q + 3] = v.w;
+            const float4 v = *(const float4 *) &L.d[sb][i / NT][(i % NT) * 32 + 8 * q + 4 * hh];
+            d[4 * q] = v.x, d[4 * q + 1] = v.y, d[4 * q + 2] = v.z, d[4 * q + 3] = v.w;
         }
     };
     // Four sub-blocks 4 P .. 4 P + 3, one step at a time (the scheduling barrier keeps the compiler from hoisting the
-    // operands of many steps, which spills); a step's LDS reads are issued during the step before it.
+    // operands of many steps, which spills); a step's codes are read during the step before it. (The scales too: 16 more
+    // registers, and 465 us against 384 for a 2048-token Q8_0 dense FFN block.)
     auto half_pass = [&](const uint8_t *buf, int sb, auto pc, const I8Frag<T> &f0, const I8Frag<T> &f1) __attribute__((always_inline)) {
         constexpr int P = decltype(pc)::value;
-        Step cur, nxt;
-        load_step(buf, sb, 4 * P * NT, cur);
+        v4i cur = load_step(buf, 4 * P * NT), nxt;
         v4i b0, b1;
         float w0, w1;
 #pragma unroll
@@ -295,14 +260,16 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
                 b0 = i8_codes<T>(f0, s, hh, L.grid), b1 = i8_codes<T>(f1, s, hh, L.grid);
                 w0 = i8_scale<T>(f0, s, hh), w1 = i8_scale<T>(f1, s, hh);
             }
-            if (i + 1 < (4 * P + 4) * NT) load_step(buf, sb, i + 1, nxt);
+            float d8[16];
+            load_scales(sb, i, d8);
+            if (i + 1 < (4 * P + 4) * NT) nxt = load_step(buf, i + 1);
             const v16i z = {};
-            const v16i i0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a, b0, z, 0, 0, 0);
-            const v16i i1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a, b1, z, 0, 0, 0);
+            const v16i i0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur, b0, z, 0, 0, 0);
+            const v16i i1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur, b1, z, 0, 0, 0);
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                acc[t][0][q] = fmaf_((float) i0[q], cur.d[q] * w0, acc[t][0][q]);
-                acc[t][1][q] = fmaf_((float) i1[q], cur.d[q] * w1, acc[t][1][q]);
+                acc[t][0][q] = fmaf_((float) i0[q], d8[q] * w0, acc[t][0][q]);
+                acc[t][1][q] = fmaf_((float) i1[q], d8[q] * w1, acc[t][1][q]);
             }
             // (pins this step's sums here: instruction selection is free to sink them past the scheduling barriers)
             asm volatile("" : "+v"(acc[t][0]), "+v"(acc[t][1]));
@@ -313,7 +280,7 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
                           I8Frag<T> &n1) __attribute__((always_inline)) {
         const int kn = kb + 1 < kb_end ? kb + 1 : kb;  // the last superblock reloads itself: the same loads every time
         dma_sb(nbuf, sb ^ 1, kn);
-        const uint4 dn = bload16(rx, dof, (uint32_t) (kn * kI8Sb));
+        const uint4 dn = load_d(kn);
         i8frag_load<T, 1>(r0, v0, c0, (uint32_t) (kb * BB), f0);
         i8frag_load<T, 1>(r1, v1, c1, (uint32_t) (kb * BB), f1);
         __builtin_amdgcn_sched_barrier(0);
@@ -350,18 +317,24 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
         if (kb + 1 < kb_end) superblock(kb + 1, 1, L.q1, L.q0, n0, n1, f0, f1);
     }
     if constexpr (!GLU) {
-        store_group<NT>(a, acc, sh_dst, cnt, row0, hh, part, false);
+        store_group<NT>(a, acc, sh_dst, cnt, row0, hh, part, failed);
     } else {
         float *t0 = (float *) L.q0, *t1 = (float *) L.q1;
         act_to_lds<NT>(acc, t0, t1, wave, jl, hh);
         __syncthreads();
         act_blocks(a, t0, t1, sh_dst, cnt, wb, wave, lane, [&](int i, int col, bool live, const float (&v)[8]) {
-            const Q8x8 q = q8_1_x8(v);
-            if (!live) return;
-            uint8_t *row = a.out_pack + (size_t) sh_dst[i] * a.out_img;
-            if (a.out_i8) i8_store(q, row, col);
-            else q8_split_store(q8_split_of(q.q, half_to_float(float_to_half(q.d))), row, a.nrows, col);
+            if constexpr (DEV)
+                image_store_dev(kImgI8, v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img), a.nrows, col, live);
+            else if (const Q8x8 q = q8_1_x8(v); live)
+                image_store(a.out_form, q, a.out_pack + (size_t) sh_dst[i] * a.out_img, a.nrows, col);
         });
+        if constexpr (DEV) {  // every act store of the workgroup has completed: count the arrival
+            dma_wait();
+            __syncthreads();
+            if (tid == 0)
+                __hip_atomic_fetch_add(a.gdone + (NT == 2 ? g : a.n_main + g), 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
@@ -382,8 +355,8 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
     int g, wb;
     bool one;
     if (!mmq_item(m, sh, a, g, wb, one)) return;
-    if (one) mmq_group_i8<T, GLU, 1>(a, g, wb, L);
-    else mmq_group_i8<T, GLU, 2>(a, g, wb, L);
+    if (one) mmq_group_i8<T, GLU, 1, false>(a, g, wb, L);
+    else mmq_group_i8<T, GLU, 2, false>(a, g, wb, L);
 }
 
 template <bool GLU> const void *mmq_i8_kernel(int type) {
@@ -397,7 +370,5 @@ template <bool GLU> const void *mmq_i8_kernel(int type) {
     }
     return nullptr;
 }
-inline bool mmq_i8_type(int type) { return mmq_i8_kernel<false>(type) != nullptr; }
-
 }  // namespace
 }  // namespace fns

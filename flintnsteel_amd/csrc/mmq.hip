@@ -126,34 +126,16 @@ __global__ __launch_bounds__(kCompactThreads) void k_mmq_compact(const int32_t *
     PF_MARK(2, 0);
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const int n_it = (n + NT - 1) / NT, it0 = blockIdx.x * per_wg, it1 = min(n_it, it0 + per_wg);
+    // this workgroup's first piece, in flight beside the histogram's loads
+    const int own = n > 0 ? ids[min(it0 * NT + tid, n - 1)] : -1;
     for (int i = tid; i < NW * 256; i += NT) (&wpos[0][0])[i] = 0;
     if (tid < 256) pos[tid] = rest[tid] = 0;
     for (int i = blockIdx.x * NT + tid; i < n_gdone; i += gridDim.x * NT) gdone[i] = 0;  // the fused GEMM launch's arrivals
     lds_sync();
     PF_MARK(2, 2);
-    // clamped, unconditional loads (under the uniform n > 0: an empty batch still writes the bounds), eight in flight
-    constexpr int U = 8;
-    for (int it = 0; it < n_it; it += U) {
-        int v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = ids[min((it + u) * NT + tid, n - 1)];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if ((it + u) * NT + tid < n && v[u] >= 0 && v[u] < ne) atomicAdd(it + u < it0 ? &pos[v[u]] : &rest[v[u]], 1);
-    }
-    lds_sync();
-    PF_MARK(2, 3);
-    if (tid < ne) cnt[tid] = pos[tid] + rest[tid];
-    lds_sync();
-    if (wave == 0) expert_prefix_wave(lane, cnt, ne, blockIdx.x == 0 ? bounds : nullptr, gprefix);
-    lds_sync();
-    PF_MARK(2, 5);
-    if (tid < ne) pos[tid] += cnt[tid];  // where this workgroup's first row of the expert goes
-    for (int it = it0; it < it1; ++it) {
-        const int p = it * NT + tid;
-        const int e = p < n ? ids[p] : -1;
-        const bool live = e >= 0 && e < ne;
-        // lanes with the same expert id: intersect the ballots of each id bit (and of liveness)
+    // a piece's lanes with the same expert id: intersect the ballots of each id bit (and of liveness); the lane's rank
+    // among them, and the wave's count of the expert
+    auto rank_piece = [&](int e, bool live) __attribute__((always_inline)) {
         uint64_t same = __ballot(live);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -162,7 +144,46 @@ __global__ __launch_bounds__(kCompactThreads) void k_mmq_compact(const int32_t *
         }
         const int rank = __popcll(same & ((1ull << lane) - 1ull));
         if (live && rank == 0) wpos[wave][e] = __popcll(same);
-        lds_sync();
+        return rank;
+    };
+    int e = it0 * NT + tid < n ? own : -1;
+    bool live = e >= 0 && e < ne;
+    int rank = rank_piece(e, live);
+    if (n_it > 1) {
+        // clamped, unconditional loads, eight in flight
+        constexpr int U = 8;
+        for (int it = 0; it < n_it; it += U) {
+            int v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = ids[min((it + u) * NT + tid, n - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if ((it + u) * NT + tid < n && v[u] >= 0 && v[u] < ne) atomicAdd(it + u < it0 ? &pos[v[u]] : &rest[v[u]], 1);
+        }
+    }
+    lds_sync();
+    PF_MARK(2, 3);
+    if (tid < ne) {
+        int c = pos[tid] + rest[tid];
+        if (n_it <= 1)  // one piece: its counts are the waves'
+            for (int w = 0; w < NW; ++w) c += wpos[w][tid];
+        cnt[tid] = c;
+    }
+    lds_sync();
+    if (wave == 0) expert_prefix_wave(lane, cnt, ne, blockIdx.x == 0 ? bounds : nullptr, gprefix);
+    lds_sync();
+    PF_MARK(2, 5);
+    if (tid < ne) pos[tid] += cnt[tid];  // where this workgroup's first row of the expert goes
+    for (int it = it0; it < it1; ++it) {
+        if (it > it0) {
+            lds_sync();
+            for (int i = tid; i < NW * 256; i += NT) (&wpos[0][0])[i] = 0;
+            lds_sync();
+            e = it * NT + tid < n ? ids[it * NT + tid] : -1;
+            live = e >= 0 && e < ne;
+            rank = rank_piece(e, live);
+            lds_sync();
+        }
         if (tid < ne) {  // the piece's rows of the expert, split over the waves in wave order
             int q = pos[tid];
 #pragma unroll
@@ -175,14 +196,9 @@ __global__ __launch_bounds__(kCompactThreads) void k_mmq_compact(const int32_t *
         }
         lds_sync();
         if (live) {
-            const int q = wpos[wave][e] + rank;
+            const int p = it * NT + tid, q = wpos[wave][e] + rank;
             ids_dst[q] = p;
             ids_src1[q] = x_rows_per_tok == 1 ? p / k : p;
-        }
-        if (it + 1 < it1) {
-            lds_sync();
-            for (int i = tid; i < NW * 256; i += NT) (&wpos[0][0])[i] = 0;
-            lds_sync();
         }
     }
     PF_MARK(2, 1);
@@ -199,15 +215,12 @@ constexpr int kSbMain = 1024, kSbMin = 32;
 __host__ __device__ constexpr int64_t split_row_bytes(int64_t ncols) { return ncols / 256 * (kSbMain + kSbMin); }
 __device__ __forceinline__ int perm8(int k) { return (k & ~3) | ((k & 1) << 1) | ((k >> 1) & 1); }
 
-// Q8_1 of 8 consecutive values per lane, 4 lanes per 32-value block (lanes 4j .. 4j + 3 of a quad, all active), into
-// the split image row `row` at column col (a multiple of 8): d = amax / 127, q = roundf(v / d) - with an IEEE
-// division per value (EXACT: the reference's arithmetic, bit for bit) or v * (1 / d). The max and the integer sum are
-// exact in any order. Returns nothing; lane q = 0 of the block also stores its min-term sums.
+// The split of eight codes of a block (four lanes per 32-value block, all active) with scale dh (an f16 value): lane
+// q = 0 of the block also stores its min-term sums.
 struct Q8Split {
     _Float16 hi[8], lo[8];  // in the stored order
     _Float16 shi, slo;      // the block's min-term sum (lane q = 0 of the block stores it)
 };
-// the split of eight codes of a block with scale dh (an f16 value)
 __device__ __forceinline__ Q8Split q8_split_of(const int (&q)[8], float dh) {
     Q8Split r;
     int qsum = 0;
@@ -225,20 +238,6 @@ __device__ __forceinline__ Q8Split q8_split_of(const int (&q)[8], float dh) {
     r.slo = (_Float16) (sv - (float) r.shi);
     return r;
 }
-template <bool EXACT>
-__device__ __forceinline__ Q8Split q8_split8_vals(const float (&v)[8]) {
-    float amax = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[k]));
-    amax = lanes_max<4>(amax);
-    const float d = amax / 127.0f;
-    const float dh = half_to_float(float_to_half(d));
-    const float id = amax == 0.0f ? 0.0f : 1.0f / d;
-    int q[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) q[k] = amax == 0.0f ? 0 : (int) (int8_t) roundf(EXACT ? v[k] / d : v[k] * id);
-    return q8_split_of(q, dh);
-}
 // byte offsets within an image row of the 8 columns at col (hi; lo at + 256) and of the block's min-term sums (hi;
 // lo at + 16)
 __device__ __forceinline__ uint32_t img_col_off(int col) {
@@ -247,47 +246,81 @@ __device__ __forceinline__ uint32_t img_col_off(int col) {
 __device__ __forceinline__ uint32_t img_sum_off(int ncols, int col) {
     return (uint32_t) ((ncols >> 8) * kSbMain + (col >> 8) * kSbMin + 2 * perm8((col >> 5) & 7));
 }
-__device__ __forceinline__ void q8_split_store(const Q8Split &r, uint8_t *row, int ncols, int col) {
-    uint8_t *o = row + img_col_off(col);
-    *(uint4 *) o = __builtin_bit_cast(uint4, r.hi);
-    *(uint4 *) (o + 256) = __builtin_bit_cast(uint4, r.lo);
+
+// ---- int8 images (the int8 form of the GEMM, fns_mmq_i8.hpp) ---------------------------------------------------------
+// Row layout, per 256-column superblock kb at kb * 320: the 256 int8 codes, the 8 block scales d8 (f32, f16 values), the
+// min-term sums of the split image (same order). A row's codes, scales and sums define its split row and the other way
+// round.
+enum : int { kImgSplit = 0, kImgI8 = 1 };
+constexpr int kI8Sb = 320, kI8Scale = 256, kI8Sum = 288;
+__host__ __device__ constexpr int img_sb_bytes(int form) { return form == kImgI8 ? kI8Sb : kSbMain + kSbMin; }
+
+// The lane's part of a quantised block (8 codes at column col, a multiple of 8; all four lanes of the block active):
+// put(byte offset within the row, value); the block's first lane also stores the scale and the sums.
+template <class Put> __device__ __forceinline__ void i8_put(const Q8x8 &r, int col, Put put) {
+    const uint32_t sb = (uint32_t) (col >> 8) * kI8Sb;
+    uint32_t w[2] = {0, 0};
+    int qsum = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        w[k / 4] |= (uint32_t) (uint8_t) (int8_t) r.q[k] << (8 * (k % 4));
+        qsum += r.q[k];
+    }
+    put(sb + (col & 255), make_uint2(w[0], w[1]));
+    qsum = lanes_sum_i<4>(qsum);
     if ((col & 31) == 0) {
-        _Float16 *m = (_Float16 *) (row + img_sum_off(ncols, col));
-        m[0] = r.shi;
-        m[8] = r.slo;
+        const int s = (col >> 5) & 7;
+        const float dh = half_to_float(float_to_half(r.d)), sv = dh * (float) qsum;  // exact in fp32
+        const _Float16 hi = (_Float16) sv, lo = (_Float16) (sv - (float) hi);
+        put(sb + kI8Scale + 4 * s, __builtin_bit_cast(uint32_t, dh));
+        put(sb + kI8Sum + 2 * perm8(s), __builtin_bit_cast(uint16_t, hi));
+        put(sb + kI8Sum + 16 + 2 * perm8(s), __builtin_bit_cast(uint16_t, lo));
     }
 }
-template <bool EXACT>
-__device__ __forceinline__ void q8_split8(const float (&v)[8], uint8_t *row, int ncols, int col, bool store) {
-    const Q8Split r = q8_split8_vals<EXACT>(v);
-    if (store) q8_split_store(r, row, ncols, col);
+template <class Put> __device__ __forceinline__ void split_put(const Q8x8 &q, int ncols, int col, Put put) {
+    const Q8Split r = q8_split_of(q.q, half_to_float(float_to_half(q.d)));
+    const uint32_t o = img_col_off(col);
+    put(o, __builtin_bit_cast(uint4, r.hi));
+    put(o + 256, __builtin_bit_cast(uint4, r.lo));
+    if ((col & 31) == 0) {
+        const uint32_t m = img_sum_off(ncols, col);
+        put(m, __builtin_bit_cast(uint16_t, r.shi));
+        put(m + 16, __builtin_bit_cast(uint16_t, r.slo));
+    }
+}
+__device__ __forceinline__ void image_store(int form, const Q8x8 &q, uint8_t *row, int ncols, int col) {
+    auto put = [&](uint32_t o, auto v) __attribute__((always_inline)) { *(decltype(v) *) (row + o) = v; };
+    if (form == kImgI8) i8_put(q, col, put);
+    else split_put(q, ncols, col, put);
 }
 
-// x [rows][ncols] f32 -> split image rows with the reference's Q8_1 arithmetic; grid (ceil(ncols / 2048), rows), 256
-// threads of 8 columns each (ncols % 256 == 0, so a block's 4 lanes are all in or all out).
-__global__ __launch_bounds__(256) void k_quant_image(const float *__restrict__ x, int ncols, uint8_t *__restrict__ out,
-                                                     int64_t img_row_bytes) {
-    const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * 8;
-    if (col >= ncols) return;
+// x [rows][ncols] f32 -> image rows with the reference's Q8_1 arithmetic; grid (ceil(ncols / 2048), rows), 256 threads
+// of 8 columns each (ncols % 256 == 0, so a block's 4 lanes are all in or all out).
+__device__ __forceinline__ void quant_image8(const float *__restrict__ x, int ncols, int row, int col, int form,
+                                             uint8_t *__restrict__ out, int64_t img_row_bytes) {
     const float *src = x + (size_t) row * ncols + col;
     const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
     const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    q8_split8<true>(v, out + (size_t) row * img_row_bytes, ncols, col, true);
+    image_store(form, q8_1_x8(v), out + (size_t) row * img_row_bytes, ncols, col);
+}
+__global__ __launch_bounds__(256) void k_quant_image(const float *__restrict__ x, int ncols, int form,
+                                                     uint8_t *__restrict__ out, int64_t img_row_bytes) {
+    const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (col < ncols) quant_image8(x, ncols, row, col, form, out, img_row_bytes);
 }
 
-// RMSNorm of a row of at most 2048 C columns (fns_q8x8.hpp) with its Q8_1 blocks and its split image row, as
+// RMSNorm of a row of at most 2048 C columns (fns_q8x8.hpp) with its Q8_1 blocks (xq null: none) and its image row, as
 // rms_norm_q8_1 and k_quant_image give them, in one pass over x.
 template <int C>
 __global__ __launch_bounds__(256) void k_rms_norm_image(const float *__restrict__ x, const float *__restrict__ w,
                                                         float *__restrict__ out, uint8_t *__restrict__ xq, int n,
-                                                        float eps, int64_t row_bytes, uint8_t *__restrict__ img,
+                                                        float eps, int64_t row_bytes, int form, uint8_t *__restrict__ img,
                                                         int64_t img_row_bytes) {
     __shared__ __align__(16) float xs[2048 * C];
     const size_t r = blockIdx.x;
     uint8_t *row = img + r * img_row_bytes;
-    rms_norm_row<C>(x + r * n, w, out + r * n, xq + r * row_bytes, n, eps, xs, [&](const Q8x8 &q, int col) {
-        q8_split_store(q8_split_of(q.q, half_to_float(float_to_half(q.d))), row, n, col);
-    });
+    rms_norm_row<C>(x + r * n, w, out + r * n, xq ? xq + r * row_bytes : nullptr, n, eps, xs,
+                    [&](const Q8x8 &q, int col) { image_store(form, q, row, n, col); });
 }
 
 // F16 guard of the act rows (reference src/kernels.cu:534-577), one wave per row of n columns (n % 256 == 0): the scale
@@ -295,7 +328,7 @@ __global__ __launch_bounds__(256) void k_rms_norm_image(const float *__restrict_
 // has written the image of the undivided values, which is the same when it is 1). Bound by reading the rows once; the
 // scale and the image were two launches (9.9 + 5.2 us at 6126 rows of 512).
 __global__ __launch_bounds__(256) void k_guard_image(float *__restrict__ act, float *__restrict__ escale, int n, int rows,
-                                                     uint8_t *__restrict__ out, int64_t img_row_bytes) {
+                                                     int form, uint8_t *__restrict__ out, int64_t img_row_bytes) {
     const int row = blockIdx.x * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
     if (row >= rows) return;
     float *r = act + (size_t) row * n;
@@ -313,7 +346,7 @@ __global__ __launch_bounds__(256) void k_guard_image(float *__restrict__ act, fl
         const float v[8] = {x0.x / e, x0.y / e, x0.z / e, x0.w / e, x1.x / e, x1.y / e, x1.z / e, x1.w / e};
         *(float4 *) (r + i) = make_float4(v[0], v[1], v[2], v[3]);
         *(float4 *) (r + i + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        q8_split8<true>(v, out + (size_t) row * img_row_bytes, n, i, true);
+        image_store(form, q8_1_x8(v), out + (size_t) row * img_row_bytes, n, i);
     }
 }
 
@@ -324,7 +357,8 @@ template <bool BF16>
 __global__ __launch_bounds__(512) void k_router_image(const void *__restrict__ w, const float *__restrict__ bias,
                                                       const float *__restrict__ x, float *__restrict__ y, int ncols,
                                                       int nrows, int n_tok, int tiles_x, int n_rt,
-                                                      uint8_t *__restrict__ img, int64_t img_row_bytes, int nxb) {
+                                                      int form, uint8_t *__restrict__ img, int64_t img_row_bytes,
+                                                      int nxb) {
     PF_MARK(0, 0);
     const int id = blockIdx.x;
     if (id < n_rt) {
@@ -334,12 +368,7 @@ __global__ __launch_bounds__(512) void k_router_image(const void *__restrict__ w
     }
     const int item = 2 * (id - n_rt) + (int) threadIdx.x / 256;
     const int row = item / nxb, col = ((item % nxb) * 256 + (int) threadIdx.x % 256) * 8;
-    if (item < nxb * n_tok && col < ncols) {
-        const float *src = x + (size_t) row * ncols + col;
-        const float4 x0 = *(const float4 *) src, x1 = *(const float4 *) (src + 4);
-        const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-        q8_split8<true>(v, img + (size_t) row * img_row_bytes, ncols, col, true);
-    }
+    if (item < nxb * n_tok && col < ncols) quant_image8(x, ncols, row, col, form, img, img_row_bytes);
     PF_MARK(0, 1);
 }
 
@@ -366,7 +395,7 @@ struct MmqArgs {
     float *dst;                // [out row][nrows] f32 (non-GLU)
     uint8_t *out_pack;         // GLU: act split image rows (by output row)
     int64_t out_img;
-    int out_i8;                // GLU, int8 form: 1 = int8 image rows, 0 = split image rows
+    int out_form;              // GLU: the form of the act image rows (kImg*)
     float *act_out;            // GLU: optional f32 act [out row][nrows]
     int *gdone;                // fused launch: per-group arrival counts (zeroed by the compaction kernel)
     int gwait;                 // fused launch: arrivals a down item waits for (its group's gate/up items)
@@ -385,6 +414,7 @@ struct MmqShared {
     float *dst;                // non-GLU
     uint8_t *out_pack;         // GLU
     int64_t out_img;
+    int out_form;
     int n_cb, items;           // launch: row blocks per group; workgroups of the grid it takes (a multiple of kXcds)
 };
 
@@ -757,20 +787,21 @@ __device__ __forceinline__ void dma16(Rsrc r, void *dst, uint32_t vo, uint32_t s
 // before the arrival, as in the decode layer's exchange.
 constexpr int kCpolDevice = 16;           // sc1
 constexpr uint32_t kStatusTimeout = 1u;   // FNS_STATUS_EXCHANGE_TIMEOUT
-__device__ __forceinline__ void q8_split8_dev(const float (&v)[8], Rsrc r, uint32_t row_off, int ncols, int col,
-                                              bool store) {
-    const Q8Split q = q8_split8_vals<true>(v);
+__device__ __forceinline__ void image_store_dev(int form, const float (&v)[8], Rsrc r, uint32_t row_off, int ncols, int col,
+                                                bool store) {
+    const Q8x8 q = q8_1_x8(v);
     if (!store) return;
-    const uint32_t o = row_off + img_col_off(col);
-    const uint4 hi = __builtin_bit_cast(uint4, q.hi), lo = __builtin_bit_cast(uint4, q.lo);
+    typedef uint32_t v2u __attribute__((ext_vector_type(2)));
     typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(v4u{hi.x, hi.y, hi.z, hi.w}, r, o, 0, kCpolDevice);
-    __builtin_amdgcn_raw_buffer_store_b128(v4u{lo.x, lo.y, lo.z, lo.w}, r, o + 256, 0, kCpolDevice);
-    if ((col & 31) == 0) {
-        const uint32_t m = row_off + img_sum_off(ncols, col);
-        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, q.shi), r, m, 0, kCpolDevice);
-        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, q.slo), r, m + 16, 0, kCpolDevice);
-    }
+    auto put = [&](uint32_t o, auto w) __attribute__((always_inline)) {
+        const uint32_t at = row_off + o;
+        if constexpr (sizeof w == 16) __builtin_amdgcn_raw_buffer_store_b128(v4u{w.x, w.y, w.z, w.w}, r, at, 0, kCpolDevice);
+        else if constexpr (sizeof w == 8) __builtin_amdgcn_raw_buffer_store_b64(v2u{w.x, w.y}, r, at, 0, kCpolDevice);
+        else if constexpr (sizeof w == 4) __builtin_amdgcn_raw_buffer_store_b32(w, r, at, 0, kCpolDevice);
+        else __builtin_amdgcn_raw_buffer_store_b16(w, r, at, 0, kCpolDevice);
+    };
+    if (form == kImgI8) i8_put(q, col, put);
+    else split_put(q, ncols, col, put);
 }
 // thread 0 polls the group's arrival count (bounded); true for every thread when the wait gave up
 __device__ __forceinline__ bool wait_group(const MmqArgs &a, int slot, int *flag) {
@@ -1197,10 +1228,10 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
         act_blocks(a, (const float *) sh_a0, (const float *) sh_a1, sh_dst, cnt, wb, wave, lane,
                    [&](int i, int col, bool live, const float (&v)[8]) {
                        if constexpr (DEV)
-                           q8_split8_dev(v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img), a.nrows, col,
-                                         live);
-                       else
-                           q8_split8<true>(v, a.out_pack + (size_t) sh_dst[i] * a.out_img, a.nrows, col, live);
+                           image_store_dev(kImgSplit, v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img),
+                                           a.nrows, col, live);
+                       else if (const Q8x8 q = q8_1_x8(v); live)
+                           image_store(a.out_form, q, a.out_pack + (size_t) sh_dst[i] * a.out_img, a.nrows, col);
                    });
         if constexpr (DEV) {  // every act store of the workgroup has completed: count the arrival
             dma_wait();
@@ -1245,6 +1276,7 @@ __device__ __forceinline__ bool mmq_item(const MmqArgs &m, const MmqShared &sh, 
         a.dst = sh.dst;
         a.out_pack = sh.out_pack;
         a.out_img = sh.out_img;
+        a.out_form = sh.out_form;
         a.act_out = nullptr;
         if (kMmqTok * j >= sh.n_rows) return false;
         one = sh.n_rows - kMmqTok * j <= kMmqTok / 2;
@@ -1312,14 +1344,13 @@ struct MoeArgs {
     int *gdone;
     uint32_t *status;
 };
-template <int TGU, int TDN>
+template <int T, bool I8>
 __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mmq_moe(const MoeArgs m) {
-    constexpr bool MIN = TGU == T_Q4_K || TGU == T_Q5_K || TDN == T_Q4_K || TDN == T_Q5_K;
-    __shared__ __align__(16) uint8_t sh_a0[kMmqTok * kRowA];
-    __shared__ __align__(16) uint8_t sh_a1[kMmqTok * kRowA];
-    __shared__ __align__(16) uint8_t sh_s[MIN ? kMmqTok * kRowS : 16];
+    __shared__ __align__(16) uint8_t sh_a0[I8 ? kI8Buf : kMmqTok * kRowA];
+    __shared__ __align__(16) uint8_t sh_a1[I8 ? kI8Buf : kMmqTok * kRowA];
+    __shared__ __align__(16) float sh_d[2][8][I8 ? kMmqTok : 4];
+    __shared__ __align__(16) uint8_t sh_s[2][kMmqTok * kRowS];
     __shared__ int sh_src[kMmqTok], sh_dst[kMmqTok], sh_grp[4];
-    const MmqLds L{sh_a0, sh_a1, *(uint8_t (*)[kMmqTok * kRowS]) sh_s, sh_src, sh_dst, sh_grp, nullptr};
     PF_MARK(3, 0);
     // The groups that exist in this call (the device-side counts of the two lists: the 64-row groups, then the <= 32-row
     // remainders) are numbered j = 0 .. R - 1 and take the first workgroups of the grid; the workgroups past them (the
@@ -1334,6 +1365,18 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
     if (j >= R) return;
     const int g = j < nm ? j : m.n_main + (j - nm);
     MmqArgs a{};
+    auto run = [&](auto glu) __attribute__((always_inline)) {
+        constexpr bool GLU = decltype(glu)::value;
+        if constexpr (I8) {
+            const MmqI8Lds L{sh_a0, sh_a1, sh_d, sh_s, sh_src, sh_dst, sh_grp, nullptr};
+            if (g < m.n_main) mmq_group_i8<T, GLU, 2, true>(a, g, wb, L);
+            else mmq_group_i8<T, GLU, 1, true>(a, g - m.n_main, wb, L);
+        } else {
+            const MmqLds L{sh_a0, sh_a1, sh_s[0], sh_src, sh_dst, sh_grp, nullptr};
+            if (g < m.n_main) mmq_group<T, GLU, 2, true>(a, g, wb, L);
+            else mmq_group<T, GLU, 1, true>(a, g - m.n_main, wb, L);
+        }
+    };
     a.table = m.table;
     a.n_expert = m.n_expert;
     a.bounds = m.bounds;
@@ -1351,8 +1394,7 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
         a.src = m.src1;
         a.out_pack = m.aimg;
         a.out_img = m.a_img;
-        if (g < m.n_main) mmq_group<TGU, true, 2, true>(a, g, wb, L);
-        else mmq_group<TGU, true, 1, true>(a, g - m.n_main, wb, L);
+        run(std::true_type{});
     } else {
         a.off_a = m.down_off;
         a.ncols = m.inter;
@@ -1364,34 +1406,34 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
         a.gwait = m.gwait;
         a.spin_limit = m.spin_limit;
         a.status = m.status;
-        if (g < m.n_main) mmq_group<TDN, false, 2, true>(a, g, wb, L);
-        else mmq_group<TDN, false, 1, true>(a, g - m.n_main, wb, L);
+        run(std::false_type{});
     }
     PF_MARK(3, 1);
 }
 
-template <bool GLU> const void *mmq_kernel(int type) {
+// the split form: mmq and mmq_experts over the caller's split image (Q8_0 takes the int8 form there), the types without an
+// int8 form, and calls of few workgroups
+const void *mmq_kernel(int type, bool glu) {
     switch (type) {
-        case T_Q8_0: return (const void *) k_mmq<T_Q8_0, GLU>;
-        case T_Q3_K: return (const void *) k_mmq<T_Q3_K, GLU>;
-        case T_Q4_K: return (const void *) k_mmq<T_Q4_K, GLU>;
-        case T_Q5_K: return (const void *) k_mmq<T_Q5_K, GLU>;
-        case T_Q6_K: return (const void *) k_mmq<T_Q6_K, GLU>;
-        case T_IQ4_XS: return (const void *) k_mmq<T_IQ4_XS, GLU>;
-        case T_IQ3_XXS: return (const void *) k_mmq<T_IQ3_XXS, GLU>;
-        case T_IQ3_S: return (const void *) k_mmq<T_IQ3_S, GLU>;
-        case T_IQ2_S: return (const void *) k_mmq<T_IQ2_S, GLU>;
+        case T_Q3_K: return glu ? (const void *) k_mmq<T_Q3_K, true> : (const void *) k_mmq<T_Q3_K, false>;
+        case T_Q6_K: return glu ? (const void *) k_mmq<T_Q6_K, true> : (const void *) k_mmq<T_Q6_K, false>;
+        case T_IQ2_S: return glu ? (const void *) k_mmq<T_IQ2_S, true> : (const void *) k_mmq<T_IQ2_S, false>;
+        case T_Q4_K: return glu ? (const void *) k_mmq<T_Q4_K, true> : (const void *) k_mmq<T_Q4_K, false>;
+        case T_Q5_K: return glu ? (const void *) k_mmq<T_Q5_K, true> : (const void *) k_mmq<T_Q5_K, false>;
+        case T_IQ4_XS: return glu ? (const void *) k_mmq<T_IQ4_XS, true> : (const void *) k_mmq<T_IQ4_XS, false>;
+        case T_IQ3_XXS: return glu ? (const void *) k_mmq<T_IQ3_XXS, true> : (const void *) k_mmq<T_IQ3_XXS, false>;
+        case T_IQ3_S: return glu ? (const void *) k_mmq<T_IQ3_S, true> : (const void *) k_mmq<T_IQ3_S, false>;
+        case T_Q8_0: return glu ? (const void *) k_mmq<T_Q8_0, true> : (const void *) k_mmq<T_Q8_0, false>;
     }
     return nullptr;
 }
 
 // groups: upper bound of the 64-row list; expert path: of the 64-row list and the <= 32-row remainders together (the
 // workgroups past the device-side counts return at once)
-// sh: a dense matrix of the same type whose groups come first in the grid (expert path only); i8: the int8 form
+// sh: a dense matrix of the same type whose groups come first in the grid (expert path only); form: of the activations
 int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st, const MmqShared *sh = nullptr,
-               bool i8 = false) {
-    const void *fn = i8 ? (glu ? mmq_i8_kernel<true>(type) : mmq_i8_kernel<false>(type))
-                        : (glu ? mmq_kernel<true>(type) : mmq_kernel<false>(type));
+               int form = kImgSplit) {
+    const void *fn = form == kImgI8 ? (glu ? mmq_i8_kernel<true>(type) : mmq_i8_kernel<false>(type)) : mmq_kernel(type, glu);
     if (!fn) return host::set_error(host::ERR_TYPE, "mmq: type %d not supported", type);
     if (groups <= 0) return host::OK;
     MmqArgs arg = a;
@@ -1417,12 +1459,12 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
     const int ks = !glu && !a.bounds && a.ksplit > 1 ? a.ksplit : 1;
     if (ks > 1 && (a.ncols / 256 < ks || ks > 8)) return host::set_error(host::ERR_SHAPE, "mmq: bad K split");
     arg.ksplit = ks;
-    if (!a.bounds && a.n_rows > 32 && (int64_t) 2 * groups * arg.n_cb * ks <= 256) {
+    if (!a.bounds && (a.n_rows <= 32 || (int64_t) 2 * groups * arg.n_cb * ks <= 256)) {
         arg.dense_small = 1;
         total = (a.n_rows + 31) / 32;
     }
     arg.n_groups = total;
-    arg.rows_first = i8 && !a.bounds && (arg.n_cb % kXcds == 0 || arg.n_cb >= 4 * kXcds);
+    arg.rows_first = form != kImgSplit && !a.bounds && (arg.n_cb % kXcds == 0 || arg.n_cb >= 4 * kXcds);
     const int64_t items = sh_items + (arg.rows_first ? (int64_t) total * kXcds * ((arg.n_cb + kXcds - 1) / kXcds)
                                                      : (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds));
     if (items > INT32_MAX) return host::set_error(host::ERR_SHAPE, "mmq: grid too large");
@@ -1432,26 +1474,18 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
     return host::check_launch("mmq");
 }
 
-// The fused kernel for the type pairs whose register allocation does not spill (the Q5_K and Q6_K decoders push the
-// combined kernel past 256 registers); the other pairs take two launches.
-template <int TGU> const void *mmq_moe_kernel_dn(int tdn) {
-    switch (tdn) {
-        case T_Q3_K: return (const void *) k_mmq_moe<TGU, T_Q3_K>;
-        case T_Q4_K: return (const void *) k_mmq_moe<TGU, T_Q4_K>;
-    }
-    return nullptr;
-}
-const void *mmq_moe_kernel(int tgu, int tdn) {
-    switch (tgu) {
-        case T_Q3_K: return mmq_moe_kernel_dn<T_Q3_K>(tdn);
-        case T_Q4_K: return mmq_moe_kernel_dn<T_Q4_K>(tdn);
-    }
+// The fused kernel: one type for gate/up and down (Q4_K in either form, Q3_K in the split one); the other pairs take two
+// launches (the Q5_K and Q6_K decoders push the combined kernel past 256 registers).
+const void *mmq_moe_kernel(int tgu, int tdn, int form) {
+    if (tgu == T_Q4_K && tdn == T_Q4_K)
+        return form == kImgI8 ? (const void *) k_mmq_moe<T_Q4_K, true> : (const void *) k_mmq_moe<T_Q4_K, false>;
+    if (tgu == T_Q3_K && tdn == T_Q3_K && form == kImgSplit) return (const void *) k_mmq_moe<T_Q3_K, false>;
     return nullptr;
 }
 
 // The fused launch (the arrival counters zero: the compaction kernel clears them).
-int launch_mmq_moe(int tgu, int tdn, MoeArgs m, hipStream_t st) {
-    const void *fn = mmq_moe_kernel(tgu, tdn);
+int launch_mmq_moe(int tgu, int tdn, int form, MoeArgs m, hipStream_t st) {
+    const void *fn = mmq_moe_kernel(tgu, tdn, form);
     if (!fn) return host::set_error(host::ERR_TYPE, "mmq: types %d / %d not supported", tgu, tdn);
     if (m.n_main <= 0) return host::OK;
     m.n_cb_gu = (m.inter + 127) / 128;
@@ -1490,52 +1524,31 @@ size_t mmq_image_bytes(int64_t ncols) { return (size_t) split_row_bytes(ncols); 
 size_t mmq_q8_1_bytes(int64_t ncols, int64_t nrows) { return (size_t) nrows * mmq_image_bytes(ncols) + 4096; }
 size_t mmq_bounds_bytes(int64_t n_expert) { return bounds_bytes(n_expert); }
 
-int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, void *xpack, hipStream_t st) {
-    if (!x || !xpack || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
-        return host::set_error(host::ERR_SHAPE, "mmq quantize: bad arguments");
-    if (rows == 0) return host::OK;
-    hipLaunchKernelGGL(k_quant_image, dim3((unsigned) ((ncols + 2047) / 2048), (unsigned) rows), dim3(256), 0, st, x, (int) ncols,
-                       (uint8_t *) xpack, (int64_t) mmq_image_bytes(ncols));
-    return host::check_launch("mmq quantize");
-}
+size_t mmq_form_bytes(int form, int64_t ncols) { return (size_t) (ncols / 256) * img_sb_bytes(form); }
+int mmq_form(int type) { return mmq_i8_kernel<false>(type) ? kImgI8 : kImgSplit; }
 
-// The int8 form's image rows of x, and of RMSNorm(x) (out as f32 too; the shapes of mmq_rms_norm_image_fits).
-size_t mmq_i8_image_bytes(int64_t ncols) { return (size_t) i8_row_bytes(ncols); }
-int mmq_quant_i8(const float *x, int64_t ncols, int64_t rows, void *ximg, hipStream_t st) {
+int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, int form, void *ximg, hipStream_t st) {
     if (!x || !ximg || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
         return host::set_error(host::ERR_SHAPE, "mmq quantize: bad arguments");
     if (rows == 0) return host::OK;
-    hipLaunchKernelGGL(k_quant_i8, dim3((unsigned) ((ncols + 2047) / 2048), (unsigned) rows), dim3(256), 0, st, x, (int) ncols,
-                       (uint8_t *) ximg, (int64_t) mmq_i8_image_bytes(ncols));
-    return host::check_launch("mmq quantize (int8)");
-}
-int mmq_rms_norm_i8(const float *x, const float *w, float *out, int n, float eps, int rows, void *ximg, hipStream_t st) {
-    if (!x || !w || !out || !ximg || rows < 0 || !mmq_rms_norm_image_fits(x, w, out, n))
-        return host::set_error(host::ERR_SHAPE, "mmq rms_norm: bad arguments");
-    if (rows == 0) return host::OK;
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3((unsigned) rows), dim3(256), 0, st, x, w, out, n, eps, (uint8_t *) ximg,
-                           (int64_t) mmq_i8_image_bytes(n));
-    };
-    if (n <= 2048) go(k_rms_norm_i8<1>);
-    else if (n <= 4096) go(k_rms_norm_i8<2>);
-    else go(k_rms_norm_i8<4>);
-    return host::check_launch("mmq rms_norm (int8)");
+    hipLaunchKernelGGL(k_quant_image, dim3((unsigned) ((ncols + 2047) / 2048), (unsigned) rows), dim3(256), 0, st, x,
+                       (int) ncols, form, (uint8_t *) ximg, (int64_t) mmq_form_bytes(form, ncols));
+    return host::check_launch("mmq quantize");
 }
 
-// RMSNorm of x (f32 [rows][n]) into out, its Q8_1 blocks into xq (null: none) and its split image rows into ximg, for
-// rows that mmq_rms_norm_image_fits: at most 8192 columns, 16-byte aligned arrays.
+// RMSNorm of x (f32 [rows][n]) into out, its Q8_1 blocks into xq (null: none) and its image rows into ximg, for rows
+// that mmq_rms_norm_image_fits: at most 8192 columns, 16-byte aligned arrays.
 bool mmq_rms_norm_image_fits(const float *x, const float *w, const float *out, int64_t n) {
     return n > 0 && n % 256 == 0 && n <= 8192 && (((uintptr_t) x | (uintptr_t) w | (uintptr_t) out) & 15) == 0;
 }
-int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, void *ximg,
-                       hipStream_t st) {
+int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, int form,
+                       void *ximg, hipStream_t st) {
     if (!x || !w || !out || !ximg || rows < 0 || !mmq_rms_norm_image_fits(x, w, out, n))
         return host::set_error(host::ERR_SHAPE, "mmq rms_norm: bad arguments");
     if (rows == 0) return host::OK;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned) rows), dim3(256), 0, st, x, w, out, (uint8_t *) xq, n, eps,
-                           host::q8_1_row_bytes(n), (uint8_t *) ximg, (int64_t) mmq_image_bytes(n));
+                           host::q8_1_row_bytes(n), form, (uint8_t *) ximg, (int64_t) mmq_form_bytes(form, n));
     };
     if (n <= 2048) go(k_rms_norm_image<1>);
     else if (n <= 4096) go(k_rms_norm_image<2>);
@@ -1543,12 +1556,13 @@ int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int
     return host::check_launch("mmq rms_norm");
 }
 
-int mmq_guard_image(float *act, float *escale, int64_t ncols, int64_t rows, void *img, int64_t stride, hipStream_t st) {
+int mmq_guard_image(float *act, float *escale, int64_t ncols, int64_t rows, int form, void *img, int64_t stride,
+                    hipStream_t st) {
     if (!act || !escale || !img || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
         return host::set_error(host::ERR_SHAPE, "mmq guard: bad arguments");
     if (rows == 0) return host::OK;
     hipLaunchKernelGGL(k_guard_image, dim3((unsigned) ((rows + 3) / 4)), dim3(256), 0, st, act, escale, (int) ncols,
-                       (int) rows, (uint8_t *) img, stride);
+                       (int) rows, form, (uint8_t *) img, stride);
     return host::check_launch("mmq guard");
 }
 
@@ -1573,7 +1587,7 @@ int mmq_compact(const int32_t *ids, int64_t n_tok, int64_t k, int64_t n_expert, 
 // Bytes per act image row in the prefill workspace: the image rounded up to whole 128-byte lines, so that no cache
 // line holds parts of two rows. The fused launch depends on it: rows of different groups are written and read by
 // different workgroups at different times, and a line read for one row must never carry another row's older bytes.
-int64_t act_stride(int64_t ncols) { return ((int64_t) mmq_image_bytes(ncols) + 127) / 128 * 128; }
+int64_t act_stride(int64_t ncols, int form = kImgSplit) { return ((int64_t) mmq_form_bytes(form, ncols) + 127) / 128 * 128; }
 
 // the 64-row list's upper bound for n_pairs sorted rows over n_expert experts: sum_e (n_e / 64 + (n_e % 64 > 32))
 int64_t main_groups(int64_t n_expert, int64_t n_pairs) { return n_expert + (n_pairs + kMmqTok - 1) / kMmqTok; }
@@ -1621,17 +1635,17 @@ int mmq(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, i
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
     if (!w || !x || !xq || !dst || n_tok < 0) return host::set_error(host::ERR_SHAPE, "mmq: bad arguments");
     if (n_tok == 0) return host::OK;
-    const bool i8 = type == T_Q8_0;
-    FNS_TRY(i8 ? mmq_quant_i8(x, ncols, n_tok, xq, st) : mmq_quant_image(x, ncols, n_tok, xq, st));
+    const int form = type == T_Q8_0 ? kImgI8 : kImgSplit;
+    FNS_TRY(mmq_quant_image(x, ncols, n_tok, form, xq, st));
     MmqArgs a{};
     a.w_dense = (const uint8_t *) w;
     a.ncols = (int) ncols;
     a.nrows = (int) nrows;
     a.xpack = (const uint8_t *) xq;
-    a.x_img = (int64_t) (i8 ? mmq_i8_image_bytes(ncols) : mmq_image_bytes(ncols));
+    a.x_img = (int64_t) mmq_form_bytes(form, ncols);
     a.n_rows = (int) n_tok;
     a.dst = dst;
-    return launch_mmq(type, false, a, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, i8);
+    return launch_mmq(type, false, a, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, form);
 }
 
 int mmq_experts(int type, const char *const *table, size_t off, int64_t ncols, int64_t nrows, int64_t n_expert,
@@ -1657,12 +1671,12 @@ int mmq_experts(int type, const char *const *table, size_t off, int64_t ncols, i
     const int64_t rows = n_tok * x_rows_per_tok;
     int32_t *gprefix = (int32_t *) ((uint8_t *) xq + (size_t) rows * mmq_image_bytes(ncols));
     FNS_TRY(mmq_compact(ids, n_tok, n_used, n_expert, x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, st));
-    const bool i8 = type == T_Q8_0;
-    FNS_TRY(i8 ? mmq_quant_i8(x, ncols, rows, xq, st) : mmq_quant_image(x, ncols, rows, xq, st));
+    const int form = type == T_Q8_0 ? kImgI8 : kImgSplit;
+    FNS_TRY(mmq_quant_image(x, ncols, rows, form, xq, st));
     MmqArgs a;
     FNS_TRY(expert_args(type, table, off, 0, false, ncols, nrows, n_expert, xq, ids_src1, ids_dst, bounds, gprefix, dst,
-                        nullptr, nullptr, a, i8 ? mmq_i8_image_bytes(ncols) : 0));
-    return launch_mmq(type, false, a, (int) main_groups(n_expert, n_tok * n_used), st, nullptr, i8);
+                        nullptr, nullptr, a, (int64_t) mmq_form_bytes(form, ncols)));
+    return launch_mmq(type, false, a, (int) main_groups(n_expert, n_tok * n_used), st, nullptr, form);
 }
 
 // ---- prefill MoE layer ----------------------------------------------------------------------------------------
@@ -1723,7 +1737,7 @@ int moe_prefill_workspace(const FnsMoeLayer *L, int64_t n_tok, size_t *offsets, 
 // type they ride in the routed launch (its workgroups are few: 8 at 37 tokens of the reference model's block, 25.5 +
 // 15.9 us as launches of their own, against nothing beside the routed 149 experts'), otherwise mmq_dense_shared
 // launches them.
-MmqShared shared_gate_up(const FnsMoeLayer *L, const void *ximg, int64_t n_tok, void *act_img) {
+MmqShared shared_gate_up(const FnsMoeLayer *L, const void *ximg, int x_form, int64_t n_tok, void *act_img, int act_form) {
     MmqShared g{};
     g.w = (const uint8_t *) L->shexp_gate;
     g.off_b = (const uint8_t *) L->shexp_up - (const uint8_t *) L->shexp_gate;
@@ -1731,23 +1745,24 @@ MmqShared shared_gate_up(const FnsMoeLayer *L, const void *ximg, int64_t n_tok, 
     g.nrows = L->shexp_inter;
     g.n_rows = (int) n_tok;
     g.xpack = (const uint8_t *) ximg;
-    g.x_img = (int64_t) mmq_image_bytes(L->hidden);
+    g.x_img = (int64_t) mmq_form_bytes(x_form, L->hidden);
     g.out_pack = (uint8_t *) act_img;
-    g.out_img = (int64_t) mmq_image_bytes(L->shexp_inter);
+    g.out_img = (int64_t) mmq_form_bytes(act_form, L->shexp_inter);
+    g.out_form = act_form;
     return g;
 }
-MmqShared shared_down(const FnsMoeLayer *L, const void *act_img, int64_t n_tok, float *sh) {
+MmqShared shared_down(const FnsMoeLayer *L, const void *act_img, int act_form, int64_t n_tok, float *sh) {
     MmqShared d{};
     d.w = (const uint8_t *) L->shexp_down;
     d.ncols = L->shexp_inter;
     d.nrows = L->hidden;
     d.n_rows = (int) n_tok;
     d.xpack = (const uint8_t *) act_img;
-    d.x_img = (int64_t) mmq_image_bytes(L->shexp_inter);
+    d.x_img = (int64_t) mmq_form_bytes(act_form, L->shexp_inter);
     d.dst = sh;
     return d;
 }
-int mmq_dense_shared(int type, bool glu, const MmqShared &s, hipStream_t st) {
+int mmq_dense_shared(int type, bool glu, int form, const MmqShared &s, hipStream_t st) {
     MmqArgs a{};
     a.w_dense = s.w;
     a.off_b = s.off_b;
@@ -1759,23 +1774,22 @@ int mmq_dense_shared(int type, bool glu, const MmqShared &s, hipStream_t st) {
     a.dst = s.dst;
     a.out_pack = s.out_pack;
     a.out_img = s.out_img;
-    return launch_mmq(type, glu, a, (s.n_rows + kMmqTok - 1) / kMmqTok, st);
+    a.out_form = s.out_form;
+    return launch_mmq(type, glu, a, (s.n_rows + kMmqTok - 1) / kMmqTok, st, nullptr, form);
 }
 
 // Dense GEMMs on activation images already built (the dense FFN block): gate/up in one GLU launch (SwiGLU and the
 // Q8_1 of act in the epilogue, act images out), and a plain launch whose K range may be split into ksplit parts
-// (dst then holds ksplit partial sums, part_stride floats apart). x_i8: the activations are int8 image rows and the
-// launch the int8 form; act_i8: so are the act rows written.
+// (dst then holds ksplit partial sums, part_stride floats apart). x_form, act_form: the forms of the activation image
+// read and of the act image written.
 bool mmq_tiled(int type, int64_t ncols, int64_t nrows) {
     const bool t = host::is_kquant(type) || type == T_Q8_0 || (host::is_iq(type) && (!host::iq_needs_grid(type) ||
                                                                                       host::iq_grids_ready()));
     return t && ncols > 0 && ncols % 256 == 0 && ncols <= 65536 && nrows > 0 && nrows % kMmqRows == 0;
 }
 
-bool mmq_i8(int type) { return mmq_i8_type(type); }
-
 int mmq_dense_glu(int type, const void *gate, const void *up, int64_t ncols, int64_t nrows, const void *ximg,
-                  int64_t n_tok, void *act_img, bool x_i8, bool act_i8, hipStream_t st) {
+                  int64_t n_tok, void *act_img, int x_form, int act_form, hipStream_t st) {
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
     MmqArgs g{};
     g.w_dense = (const uint8_t *) gate;
@@ -1784,28 +1798,28 @@ int mmq_dense_glu(int type, const void *gate, const void *up, int64_t ncols, int
     g.ncols = (int) ncols;
     g.nrows = (int) nrows;
     g.xpack = (const uint8_t *) ximg;
-    g.x_img = (int64_t) (x_i8 ? mmq_i8_image_bytes(ncols) : mmq_image_bytes(ncols));
+    g.x_img = (int64_t) mmq_form_bytes(x_form, ncols);
     g.n_rows = (int) n_tok;
     g.out_pack = (uint8_t *) act_img;
-    g.out_img = (int64_t) (act_i8 ? mmq_i8_image_bytes(nrows) : mmq_image_bytes(nrows));
-    g.out_i8 = act_i8;
-    return launch_mmq(type, true, g, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, x_i8);
+    g.out_img = (int64_t) mmq_form_bytes(act_form, nrows);
+    g.out_form = act_form;
+    return launch_mmq(type, true, g, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, x_form);
 }
 
 int mmq_dense_parts(int type, const void *w, int64_t ncols, int64_t nrows, const void *ximg, int64_t n_tok, float *dst,
-                    int ksplit, bool x_i8, hipStream_t st) {
+                    int ksplit, int x_form, hipStream_t st) {
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
     MmqArgs d{};
     d.w_dense = (const uint8_t *) w;
     d.ncols = (int) ncols;
     d.nrows = (int) nrows;
     d.xpack = (const uint8_t *) ximg;
-    d.x_img = (int64_t) (x_i8 ? mmq_i8_image_bytes(ncols) : mmq_image_bytes(ncols));
+    d.x_img = (int64_t) mmq_form_bytes(x_form, ncols);
     d.n_rows = (int) n_tok;
     d.dst = dst;
     d.ksplit = ksplit;
     d.part_stride = n_tok * nrows;
-    return launch_mmq(type, false, d, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, x_i8);
+    return launch_mmq(type, false, d, (int) ((n_tok + kMmqTok - 1) / kMmqTok), st, nullptr, x_form);
 }
 
 namespace {
@@ -1837,6 +1851,11 @@ int moe_prefill_status_collect(const FnsMoeLayer *L, int64_t n_tok, void *ws, ui
     return status_collect((uint32_t *) ((uint8_t *) ws + off) + words, dst, st);
 }
 
+// Whether a call's gate/up GEMM has at most 256 workgroups (its images are then in the split form).
+static bool moe_prefill_few(const FnsMoeLayer *L, int64_t n_tok) {
+    return std::min<int64_t>(L->n_expert, n_tok * L->k) * ((L->inter + 127) / 128) <= 256;
+}
+
 int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, float *out, int64_t n_tok, void *ws,
                 size_t ws_bytes, hipStream_t st) {
     if (!L || !x || !out || !ws || !L->router_w || !L->table) return host::set_error(host::ERR_SHAPE, "moe_prefill: null argument");
@@ -1863,13 +1882,27 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     const int64_t P = n_tok * L->k;
     const char *const *table = (const char *const *) L->table;
 
+    // The forms of the activation images: int8 where every matrix that reads the image has the int8 form (x: the routed
+    // and the shared gate/up).
+    const bool has_sh = L->shexp_inter > 0;
+    const int sgt = has_sh && L->shexp_gu_type ? L->shexp_gu_type : L->gu_type;
+    const int sdt = has_sh && L->shexp_down_type ? L->shexp_down_type : L->down_type;
+    // A call whose gate/up items (at most min(n_expert, pairs) groups of few rows) do not fill the GPU is bound by one
+    // workgroup's latency, where the split form's MFMAs are shorter than the int8 form's scaling (6 tokens to 4 of 32
+    // experts, 1024 -> 512: 41.7 against 43.9 us; 37 tokens to 6 of 256, 888 items: 144 against 140).
+    const bool few = moe_prefill_few(L, n_tok);
+    const int x_form = few ? kImgSplit : std::min(mmq_form(L->gu_type), mmq_form(sgt));
+    const int act_form = few ? kImgSplit : mmq_form(L->down_type), sh_form = few ? kImgSplit : mmq_form(sdt);
+    const int64_t x_img = (int64_t) mmq_form_bytes(x_form, L->hidden);
+
     // RMSNorm first when the layer has one: the router and the experts read h (reference src/engine.cu:331)
     bool have_img = false;  // the RMSNorm kernel has built the activation image
     if (L->ffn_norm) {
         float *h = (float *) sec[11];
         have_img = mmq_rms_norm_image_fits(x, L->ffn_norm, h, L->hidden);
         if (have_img)
-            FNS_TRY(mmq_rms_norm_image(x, L->ffn_norm, h, sec[12], (int) L->hidden, L->norm_eps, (int) n_tok, sec[3], st));
+            FNS_TRY(mmq_rms_norm_image(x, L->ffn_norm, h, sec[12], (int) L->hidden, L->norm_eps, (int) n_tok, x_form,
+                                       sec[3], st));
         else
             FNS_TRY(rms_norm_q8_1(x, L->ffn_norm, h, sec[12], (int) L->hidden, L->norm_eps, (int) n_tok, st));
         x = h;
@@ -1888,48 +1921,46 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
         const dim3 g((unsigned) (n_rt + n_img));
         if (bf)
             hipLaunchKernelGGL(k_router_image<true>, g, dim3(512), 0, st, L->router_w, L->router_bias, x, logits, H, NE,
-                               (int) n_tok, tiles_x, n_rt, (uint8_t *) sec[3], (int64_t) mmq_image_bytes(H), nxb);
+                               (int) n_tok, tiles_x, n_rt, x_form, (uint8_t *) sec[3], x_img, nxb);
         else
             hipLaunchKernelGGL(k_router_image<false>, g, dim3(512), 0, st, L->router_w, L->router_bias, x, logits, H,
-                               NE, (int) n_tok, tiles_x, n_rt, (uint8_t *) sec[3], (int64_t) mmq_image_bytes(H), nxb);
+                               NE, (int) n_tok, tiles_x, n_rt, x_form, (uint8_t *) sec[3], x_img, nxb);
         FNS_TRY(host::check_launch("prefill router + image"));
     } else {
         FNS_TRY(gemm_router_bias(L->router_dtype, L->router_w, L->router_bias, x, logits, L->hidden, L->n_expert,
                                  (int) n_tok, st));
-        if (!have_img) FNS_TRY(mmq_quant_image(x, L->hidden, n_tok, sec[3], st));
+        if (!have_img) FNS_TRY(mmq_quant_image(x, L->hidden, n_tok, x_form, sec[3], st));
     }
     FNS_TRY(route_topk(logits, ids, w, L->n_expert, L->k, (int) n_tok, L->gating, L->norm_w, st));
     // gate/up (SwiGLU and the Q8_1 of act fused) and down: act image rows padded to whole cache lines; one launch
     // unless the F16 guard's whole-row amax has to sit between them (or the type pair has no fused kernel)
     const int groups = (int) main_groups(L->n_expert, P);
-    const int64_t astride = act_stride(L->inter);
+    const int64_t astride = act_stride(L->inter, act_form);
     int32_t *gdone = bounds + 3 * (L->n_expert + 1);
     uint32_t *status = (uint32_t *) (gdone + groups + L->n_expert);
-    const bool fused = !L->guard && mmq_moe_kernel(L->gu_type, L->down_type) && P * astride < INT32_MAX;
+    const bool fused = !L->guard && x_form == act_form && mmq_moe_kernel(L->gu_type, L->down_type, x_form) && P * astride < INT32_MAX;
     FNS_TRY(mmq_compact(ids, n_tok, L->k, L->n_expert, 1, src1, dstr, bounds, bounds + L->n_expert + 1, st,
                         fused ? gdone : nullptr, groups + (int) L->n_expert));
     // down: one act row per (token, slot), in the same expert order as gate/up: the sorted rows are the pairs
     // themselves (activation row = output row = p), so the gate/up sort is reused with ids_dst as the source list
     MmqArgs gu, dn;
     FNS_TRY(expert_args(L->gu_type, table, L->gate_off, L->up_off, true, L->hidden, L->inter, L->n_expert, sec[3], src1,
-                        dstr, bounds, bounds + L->n_expert + 1, nullptr, sec[4], L->guard ? act : nullptr, gu, 0,
+                        dstr, bounds, bounds + L->n_expert + 1, nullptr, sec[4], L->guard ? act : nullptr, gu, x_img,
                         astride));
+    gu.out_form = act_form;
     FNS_TRY(expert_args(L->down_type, table, L->down_off, 0, false, L->inter, L->hidden, L->n_expert, sec[4], dstr,
                         dstr, bounds, bounds + L->n_expert + 1, dexp, nullptr, nullptr, dn, astride));
     // the shared expert (reference src/engine.cu:351-355): in the routed launches where the types agree
-    const bool has_sh = L->shexp_inter > 0;
-    const int sgt = has_sh && L->shexp_gu_type ? L->shexp_gu_type : L->gu_type;
-    const int sdt = has_sh && L->shexp_down_type ? L->shexp_down_type : L->down_type;
     float *sh = has_sh ? (float *) sec[14] : nullptr;
     MmqShared sgu{}, sdn{};
     if (has_sh) {
         FNS_TRY(check_mmq_shape(sgt, L->hidden, L->shexp_inter));
         FNS_TRY(check_mmq_shape(sdt, L->shexp_inter, L->hidden));
-        sgu = shared_gate_up(L, sec[3], n_tok, sec[13]);
-        sdn = shared_down(L, sec[13], n_tok, sh);
+        sgu = shared_gate_up(L, sec[3], x_form, n_tok, sec[13], sh_form);
+        sdn = shared_down(L, sec[13], sh_form, n_tok, sh);
     }
     const bool ride_gu = has_sh && !fused && sgt == L->gu_type, ride_dn = has_sh && !fused && sdt == L->down_type;
-    if (has_sh && !ride_gu) FNS_TRY(mmq_dense_shared(sgt, true, sgu, st));
+    if (has_sh && !ride_gu) FNS_TRY(mmq_dense_shared(sgt, true, x_form, sgu, st));
     if (fused) {
         MoeArgs m{};
         m.table = table;
@@ -1941,7 +1972,7 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
         m.n_expert = (int) L->n_expert;
         m.n_main = groups;
         m.ximg = sec[3];
-        m.x_img = (int64_t) mmq_image_bytes(L->hidden);
+        m.x_img = x_img;
         m.aimg = sec[4];
         m.a_img = astride;
         m.bounds = bounds;
@@ -1952,14 +1983,14 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
         m.gdone = gdone;
         m.status = status;
         moe_test_hooks(&m.spin_limit, &m.gwait);  // withheld arrivals; + the gate/up row blocks per group
-        FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, m, st));
+        FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, x_form, m, st));
     } else {
-        FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st, ride_gu ? &sgu : nullptr));
+        FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st, ride_gu ? &sgu : nullptr, x_form));
         // whole-row amax: a second pass over the f32 act rows (reference src/kernels.cu:534-552)
-        if (L->guard) FNS_TRY(mmq_guard_image(act, escale, L->inter, P, sec[4], astride, st));
-        FNS_TRY(launch_mmq(L->down_type, false, dn, groups, st, ride_dn ? &sdn : nullptr));
+        if (L->guard) FNS_TRY(mmq_guard_image(act, escale, L->inter, P, act_form, sec[4], astride, st));
+        FNS_TRY(launch_mmq(L->down_type, false, dn, groups, st, ride_dn ? &sdn : nullptr, act_form));
     }
-    if (has_sh && !ride_dn) FNS_TRY(mmq_dense_shared(sdt, false, sdn, st));
+    if (has_sh && !ride_dn) FNS_TRY(mmq_dense_shared(sdt, false, sh_form, sdn, st));
     return moe_combine(dexp, L->guard ? escale : nullptr, w, sh, x_resid, out, L->hidden, L->k, (int) n_tok, st);
 }
 

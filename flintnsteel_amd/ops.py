@@ -391,6 +391,24 @@ class MoeLayer:
 PREFILL_SECTIONS = ("logits", "ids", "w", "xpack", "apack", "dexp")
 
 
+# Types whose activations the prefill GEMM reads as int8 image rows (per 256 columns 320 bytes: int8 codes, 8 f32 block
+# scales, 32 bytes of scaled sums) in calls of more than 256 gate/up workgroups; the others read split image rows (1056).
+I8_TYPES = (Q8_0, Q4_K, Q5_K, IQ4_XS, IQ3_XXS, IQ3_S)
+
+
+def _split_of_i8(rows: torch.Tensor, ncols: int) -> torch.Tensor:
+    """The split image rows (uint8 [n][ncols / 256 * 1056]: every code times its scale as two f16 halves, then the sums)
+    that int8 image rows define: the same codes, scales and sums."""
+    n, nb = rows.shape[0], ncols // 256
+    sb = rows[:, : nb * 320].contiguous().view(n, nb, 320)
+    q = sb[:, :, :256].contiguous().view(torch.int8).float().view(n, nb, 8, 32)
+    x = q * sb[:, :, 256:288].contiguous().view(torch.float32).unsqueeze(3)  # exact in f32
+    x = x.view(n, nb, 32, 8)[..., [0, 2, 1, 3, 4, 6, 5, 7]].reshape(n, nb, 2, 128)
+    hi = x.half()
+    main = torch.cat([hi, (x - hi.float()).half()], 3).reshape(n, nb * 512).view(torch.uint8)
+    return torch.cat([main, sb[:, :, 288:].reshape(n, nb * 32)], 1)
+
+
 class MoePrefill:
     """Prefill (batched) form of a MoeLayer: fns_hip_moe_prefill over n_tok tokens."""
 
@@ -436,8 +454,8 @@ class MoePrefill:
         return off.value, size.value
 
     def trace(self, ws: torch.Tensor, n_tok: int) -> dict:
-        """Views of the intermediates a call left in its workspace: logits, ids, w, dexp, the split activation images
-        of x ("xpack", [n_tok][image bytes]) and act ("apack", [n_tok * k][image bytes], by (token, slot)), the guard
+        """The intermediates a call left in its workspace: views of logits, ids, w and dexp, the activation images of x
+        in the split form ("xpack", [n_tok][split row bytes]) and of act ("apack", [n_tok * k][split row bytes], by (token, slot)), the guard
         scales ("escale") and, with the F16 guard, the f32 act rows after the division ("act")."""
         d = self.layer.desc
         P = n_tok * d.k
@@ -450,9 +468,16 @@ class MoePrefill:
             off, n = self.section(n_tok, idx)
             if n:
                 out[name] = ws[off: off + n].view(dt).view(*shape)
-        # image rows may be padded to whole cache lines: the views hold each row's image bytes only
-        out["xpack"] = out["xpack"][:, : d.hidden // 256 * 1056]
-        out["apack"] = out["apack"][:, : d.inter // 256 * 1056]
+        # (act rows are padded to whole cache lines)
+        many = min(d.n_expert, P) * ((d.inter + 127) // 128) > 256
+        x_i8 = d.gu_type in I8_TYPES and (not d.shexp_inter or (d.shexp_gu_type or d.gu_type) in I8_TYPES)
+        for name, i8, ncols, pad in (("xpack", many and x_i8, d.hidden, 1),
+                                     ("apack", many and d.down_type in I8_TYPES, d.inter, 128)):
+            if i8:
+                stride, n = (ncols // 256 * 320 + pad - 1) // pad * pad, out[name].shape[0]
+                out[name] = _split_of_i8(out[name].reshape(-1)[: n * stride].view(n, stride), ncols)
+            else:
+                out[name] = out[name][:, : ncols // 256 * 1056]
         return out
 
 

@@ -62,3 +62,45 @@ def test_dense_prefill_int8(ops, qtype, T, H, F):
     bound = 2 * np.abs(act).max() / 127 * np.abs(down).max() + 1e-5 * np.abs(ref).max()
     l2 = rel_l2(got.cpu().numpy().astype(np.float64) - x, ref)
     assert err.max() <= bound and l2 <= CHAIN_L2_TOL, f"max err {err.max():.3e} (bound {bound:.3e}), rel L2 {l2:.3e}"
+
+
+@pytest.mark.parametrize("gu,down", [(orc.Q4_K, orc.Q4_K), (orc.Q4_K, orc.Q6_K), (orc.Q5_K, orc.IQ4_XS),
+                                     (orc.IQ3_XXS, orc.IQ3_S), (orc.Q8_0, orc.Q8_0), (orc.Q6_K, orc.Q5_K)])
+@pytest.mark.parametrize("counts", [(1, 2, 7, 8, 9), (32, 33, 40, 64, 72)])
+def test_prefill_group_sizes(ops, gu, down, counts):
+    """The prefill layer with experts of exactly these loads (a router that picks each token's expert): one tile, two
+    tiles and their remainders, in one launch or two, gate/up and down in either form of the GEMM."""
+    H, F, E = 512, 256, 8
+    owner = np.concatenate([np.full(n, e) for e, n in enumerate(counts)])
+    T = owner.size
+    rng = np.random.default_rng(T + gu)
+    router = np.zeros((E, H), np.float32)
+    x = gaussian(rng, (T, H))
+    for e in range(E):  # columns 0..7 carry the choice
+        router[e, e] = 50.0
+    x[:, :E] = 0.0
+    x[np.arange(T), owner] = 4.0
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    mats = [np.stack([weights(t, r, c, 10 * k + e).reshape(-1) for e in range(E)])
+            for k, (t, r, c) in enumerate([(gu, F, H), (gu, F, H), (down, H, F)])]
+    slots = ops.ExpertSlots.from_tensors(*(torch.from_numpy(m) for m in mats))
+    layer = ops.MoeLayer(dev(router), slots, gu, down, H, F, 1)
+    pre = ops.MoePrefill(layer)
+    ws, xd = pre.workspace(T), dev(x)
+    out = pre(xd, ws=ws).cpu().numpy().astype(np.float64)
+    tr = pre.trace(ws, T)
+    assert np.array_equal(tr["ids"].cpu().numpy()[:, 0], owner)
+    xq = orc.dequantize_q8_1(orc.quantize_q8_1(x), H)
+    w = tr["w"].cpu().numpy().astype(np.float64)
+    tight = []  # rows without a moved code: all but about one in forty (256 codes a row, one in 10^4 moves)
+    for e in range(len(counts)):
+        t = np.flatnonzero(owner == e)
+        g, u, d = (dequant(ty, m[e], r, c) for m, (ty, r, c) in zip(mats, [(gu, F, H), (gu, F, H), (down, H, F)]))
+        gate, up = xq[t] @ g.T, xq[t] @ u.T
+        act = (up * gate / (1 + np.exp(-gate))).astype(np.float32)
+        ref = orc.dequantize_q8_1(orc.quantize_q8_1(act), F) @ d.T * w[t]
+        err = np.abs(out[t] - ref).max(axis=1)
+        bound = 2 * np.abs(act).max() / 127 * np.abs(d).max() + 1e-5 * np.abs(ref).max()
+        assert err.max() <= bound, f"expert {e} ({t.size} rows): {err.max():.3e} > {bound:.3e}"
+        tight.append(err <= 1e-5 * np.abs(ref).max())
+    assert np.concatenate(tight).mean() >= 0.8
