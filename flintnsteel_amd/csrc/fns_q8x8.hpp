@@ -18,7 +18,7 @@ struct Q8x8 {
 // All four lanes of a block must be active.
 __device__ __forceinline__ Q8x8 q8_1_x8(const float (&v)[8]) {
     Q8x8 r;
-    float amax = 0.0f, s[8];
+    float amax = fabsf(v[0]), s[8];  // (not from 0: a block of NaNs keeps a NaN scale, as in the one-value form)
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         amax = fmaxf(amax, fabsf(v[k]));

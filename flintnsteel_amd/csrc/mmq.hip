@@ -210,7 +210,8 @@ __global__ __launch_bounds__(kCompactThreads) void k_mmq_compact(const int32_t *
 // superblock kb: 1024 bytes at kb * 1024, two 128-column halves of [hi 128 f16][lo 128 f16]; then at nb * 1024 + 32 kb
 // the min-term sums [S_hi 8 f16][S_lo 8 f16], S_s = d8_s * sum(q8 of sub-block s). Within every 8 columns (and every
 // 4 sums) the stored order is 0 2 1 3 4 6 5 7: the order in which the weight decoders below emit their B operand.
-// Magnitudes are those of the reference's f16 Q8_1 fields (|q8 d8| <= amax, S within the f16 sum's range).
+// Magnitudes are those of the reference's f16 Q8_1 fields (|q8 d8| <= amax, S within the f16 sum's range). A block of
+// nothing but NaNs is stored as zeros in either form of image.
 constexpr int kSbMain = 1024, kSbMin = 32;
 __host__ __device__ constexpr int64_t split_row_bytes(int64_t ncols) { return ncols / 256 * (kSbMain + kSbMin); }
 __device__ __forceinline__ int perm8(int k) { return (k & ~3) | ((k & 1) << 1) | ((k >> 1) & 1); }
@@ -255,6 +256,9 @@ enum : int { kImgSplit = 0, kImgI8 = 1 };
 constexpr int kI8Sb = 320, kI8Scale = 256, kI8Sum = 288;
 __host__ __device__ constexpr int img_sb_bytes(int form) { return form == kImgI8 ? kI8Sb : kSbMain + kSbMin; }
 
+// The scale as the images store it: rounded to f16, 0 for NaN.
+__device__ __forceinline__ float image_scale(float d) { return half_to_float(float_to_half(fmaxf(d, 0.0f))); }
+
 // The lane's part of a quantised block (8 codes at column col, a multiple of 8; all four lanes of the block active):
 // put(byte offset within the row, value); the block's first lane also stores the scale and the sums.
 template <class Put> __device__ __forceinline__ void i8_put(const Q8x8 &r, int col, Put put) {
@@ -270,7 +274,7 @@ template <class Put> __device__ __forceinline__ void i8_put(const Q8x8 &r, int c
     qsum = lanes_sum_i<4>(qsum);
     if ((col & 31) == 0) {
         const int s = (col >> 5) & 7;
-        const float dh = half_to_float(float_to_half(r.d)), sv = dh * (float) qsum;  // exact in fp32
+        const float dh = image_scale(r.d), sv = dh * (float) qsum;  // exact in fp32
         const _Float16 hi = (_Float16) sv, lo = (_Float16) (sv - (float) hi);
         put(sb + kI8Scale + 4 * s, __builtin_bit_cast(uint32_t, dh));
         put(sb + kI8Sum + 2 * perm8(s), __builtin_bit_cast(uint16_t, hi));
@@ -278,7 +282,7 @@ template <class Put> __device__ __forceinline__ void i8_put(const Q8x8 &r, int c
     }
 }
 template <class Put> __device__ __forceinline__ void split_put(const Q8x8 &q, int ncols, int col, Put put) {
-    const Q8Split r = q8_split_of(q.q, half_to_float(float_to_half(q.d)));
+    const Q8Split r = q8_split_of(q.q, image_scale(q.d));
     const uint32_t o = img_col_off(col);
     put(o, __builtin_bit_cast(uint4, r.hi));
     put(o + 256, __builtin_bit_cast(uint4, r.lo));

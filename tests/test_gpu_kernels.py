@@ -90,6 +90,28 @@ def test_rms_norm_q8_1_row_widths(ops, n):
     assert np.array_equal(host(out2), out_h) and np.array_equal(host(xq2), host(xq))
 
 
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_rms_norm_q8_1_not_finite(ops, bad):
+    """A value that is not finite: the register form's blocks are those of the loop form (an x that is not 16-byte
+    aligned), and a NaN, which makes the whole row NaN, is a NaN scale in every block of the row, not a row of zeros."""
+    rng = np.random.default_rng(75)
+    x, w = gaussian(rng, (2, 2048)), gaussian(rng, (2048,), 1.0)
+    x[1, 37] = bad
+    off = torch.empty(x.size + 1, device="cuda")[1:].view(x.shape)
+    off.copy_(dev(x))
+    blocks = []
+    for xs in (dev(x), off):
+        out, xq = ops.rms_norm_q8_1(xs, dev(w), 1e-6)
+        b = host(xq).view(np.uint8).reshape(2, -1, 36)
+        blocks.append((host(out), b[..., :4].copy().view(np.float16), b[..., 4:]))
+    for a, b in zip(*blocks):
+        assert np.array_equal(a, b, equal_nan=a.dtype != np.uint8)
+    d = blocks[0][1][..., 0]
+    assert np.isfinite(d[0]).all()
+    if np.isnan(bad):
+        assert np.isnan(d[1]).all()
+
+
 # ---- expert GEMVs -----------------------------------------------------------------------------------------------
 
 @pytest.fixture(scope="module")
