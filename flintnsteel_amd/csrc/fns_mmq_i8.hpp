@@ -324,7 +324,7 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
         __syncthreads();
         act_blocks(a, t0, t1, sh_dst, cnt, wb, wave, lane, [&](int i, int col, bool live, const float (&v)[8]) {
             if constexpr (DEV)
-                image_store_dev(kImgI8, v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img), a.nrows, col, live);
+                image_store_dev(a.out_form, v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img), a.nrows, col, live);
             else if (const Q8x8 q = q8_1_x8(v); live)
                 image_store(a.out_form, q, a.out_pack + (size_t) sh_dst[i] * a.out_img, a.nrows, col);
         });

@@ -1232,7 +1232,7 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
         act_blocks(a, (const float *) sh_a0, (const float *) sh_a1, sh_dst, cnt, wb, wave, lane,
                    [&](int i, int col, bool live, const float (&v)[8]) {
                        if constexpr (DEV)
-                           image_store_dev(kImgSplit, v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img),
+                           image_store_dev(a.out_form, v, rsrc_of(a.out_pack), (uint32_t) ((size_t) sh_dst[i] * a.out_img),
                                            a.nrows, col, live);
                        else if (const Q8x8 q = q8_1_x8(v); live)
                            image_store(a.out_form, q, a.out_pack + (size_t) sh_dst[i] * a.out_img, a.nrows, col);
@@ -1340,19 +1340,24 @@ struct MoeArgs {
     int64_t gate_off, up_off, down_off;
     int hidden, inter, n_expert, n_main;  // n_main: the 64-row list's upper bound
     int n_cb_gu, n_cb_dn, gwait, spin_limit;
-    const uint8_t *ximg;                  // x split images [n_tok][x_img]
-    uint8_t *aimg;                        // act split images [n_tok * k][a_img]
+    const uint8_t *ximg;                  // x images [n_tok][x_img]
+    uint8_t *aimg;                        // act images [n_tok * k][a_img]
     int64_t x_img, a_img;
     const int32_t *bounds, *gprefix, *src1, *dstr;
     float *dexp;
     int *gdone;
     uint32_t *status;
 };
-template <int T, bool I8>
+// Each GEMM reads the form of image that is the faster one for its type (GU8, DN8: int8), so a pair whose types take
+// different forms is one launch as well.
+template <int TGU, bool GU8, int TDN, bool DN8>
 __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mmq_moe(const MoeArgs m) {
-    __shared__ __align__(16) uint8_t sh_a0[I8 ? kI8Buf : kMmqTok * kRowA];
-    __shared__ __align__(16) uint8_t sh_a1[I8 ? kI8Buf : kMmqTok * kRowA];
-    __shared__ __align__(16) float sh_d[2][8][I8 ? kMmqTok : 4];
+    constexpr bool ANY8 = GU8 || DN8;
+    constexpr int kSplitBuf = kMmqTok * kRowA, kBuf = GU8 && DN8 ? kI8Buf : kSplitBuf;
+    static_assert(kI8Buf <= kSplitBuf, "the split form's buffers hold the int8 form's");
+    __shared__ __align__(16) uint8_t sh_a0[kBuf];
+    __shared__ __align__(16) uint8_t sh_a1[kBuf];
+    __shared__ __align__(16) float sh_d[2][8][ANY8 ? kMmqTok : 4];
     __shared__ __align__(16) uint8_t sh_s[2][kMmqTok * kRowS];
     __shared__ int sh_src[kMmqTok], sh_dst[kMmqTok], sh_grp[4];
     PF_MARK(3, 0);
@@ -1371,12 +1376,14 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
     MmqArgs a{};
     auto run = [&](auto glu) __attribute__((always_inline)) {
         constexpr bool GLU = decltype(glu)::value;
-        if constexpr (I8) {
-            const MmqI8Lds L{sh_a0, sh_a1, sh_d, sh_s, sh_src, sh_dst, sh_grp, nullptr};
+        constexpr int T = GLU ? TGU : TDN;
+        if constexpr (GLU ? GU8 : DN8) {
+            const MmqI8Lds L{(uint8_t (&)[kI8Buf]) sh_a0, (uint8_t (&)[kI8Buf]) sh_a1, (float (&)[2][8][kMmqTok]) sh_d, sh_s,
+                             sh_src, sh_dst, sh_grp, nullptr};
             if (g < m.n_main) mmq_group_i8<T, GLU, 2, true>(a, g, wb, L);
             else mmq_group_i8<T, GLU, 1, true>(a, g - m.n_main, wb, L);
         } else {
-            const MmqLds L{sh_a0, sh_a1, sh_s[0], sh_src, sh_dst, sh_grp, nullptr};
+            const MmqLds L{(uint8_t (&)[kSplitBuf]) sh_a0, (uint8_t (&)[kSplitBuf]) sh_a1, sh_s[0], sh_src, sh_dst, sh_grp, nullptr};
             if (g < m.n_main) mmq_group<T, GLU, 2, true>(a, g, wb, L);
             else mmq_group<T, GLU, 1, true>(a, g - m.n_main, wb, L);
         }
@@ -1398,6 +1405,7 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
         a.src = m.src1;
         a.out_pack = m.aimg;
         a.out_img = m.a_img;
+        a.out_form = DN8 ? kImgI8 : kImgSplit;
         run(std::true_type{});
     } else {
         a.off_a = m.down_off;
@@ -1478,18 +1486,23 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
     return host::check_launch("mmq");
 }
 
-// The fused kernel: one type for gate/up and down (Q4_K in either form, Q3_K in the split one); the other pairs take two
-// launches (the Q5_K and Q6_K decoders push the combined kernel past 256 registers).
-const void *mmq_moe_kernel(int tgu, int tdn, int form) {
-    if (tgu == T_Q4_K && tdn == T_Q4_K)
-        return form == kImgI8 ? (const void *) k_mmq_moe<T_Q4_K, true> : (const void *) k_mmq_moe<T_Q4_K, false>;
-    if (tgu == T_Q3_K && tdn == T_Q3_K && form == kImgSplit) return (const void *) k_mmq_moe<T_Q3_K, false>;
-    return nullptr;
+// The fused kernel of a pair of {Q3_K, Q4_K} and the forms of the x and act images; the other pairs take two launches (the
+// Q5_K and Q6_K decoders push the combined kernel past 256 registers).
+template <int TGU, bool GU8> const void *mmq_moe_kernel_dn(int tdn, int act_form) {
+    if (tdn == T_Q4_K)
+        return act_form == kImgI8 ? (const void *) k_mmq_moe<TGU, GU8, T_Q4_K, true>
+                                  : (const void *) k_mmq_moe<TGU, GU8, T_Q4_K, false>;
+    return tdn == T_Q3_K && act_form == kImgSplit ? (const void *) k_mmq_moe<TGU, GU8, T_Q3_K, false> : nullptr;
+}
+const void *mmq_moe_kernel(int tgu, int tdn, int x_form, int act_form) {
+    if (tgu == T_Q4_K)
+        return x_form == kImgI8 ? mmq_moe_kernel_dn<T_Q4_K, true>(tdn, act_form) : mmq_moe_kernel_dn<T_Q4_K, false>(tdn, act_form);
+    return tgu == T_Q3_K && x_form == kImgSplit ? mmq_moe_kernel_dn<T_Q3_K, false>(tdn, act_form) : nullptr;
 }
 
 // The fused launch (the arrival counters zero: the compaction kernel clears them).
-int launch_mmq_moe(int tgu, int tdn, int form, MoeArgs m, hipStream_t st) {
-    const void *fn = mmq_moe_kernel(tgu, tdn, form);
+int launch_mmq_moe(int tgu, int tdn, int x_form, int act_form, MoeArgs m, hipStream_t st) {
+    const void *fn = mmq_moe_kernel(tgu, tdn, x_form, act_form);
     if (!fn) return host::set_error(host::ERR_TYPE, "mmq: types %d / %d not supported", tgu, tdn);
     if (m.n_main <= 0) return host::OK;
     m.n_cb_gu = (m.inter + 127) / 128;
@@ -1942,7 +1955,7 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     const int64_t astride = act_stride(L->inter, act_form);
     int32_t *gdone = bounds + 3 * (L->n_expert + 1);
     uint32_t *status = (uint32_t *) (gdone + groups + L->n_expert);
-    const bool fused = !L->guard && x_form == act_form && mmq_moe_kernel(L->gu_type, L->down_type, x_form) && P * astride < INT32_MAX;
+    const bool fused = !L->guard && mmq_moe_kernel(L->gu_type, L->down_type, x_form, act_form) && P * astride < INT32_MAX;
     FNS_TRY(mmq_compact(ids, n_tok, L->k, L->n_expert, 1, src1, dstr, bounds, bounds + L->n_expert + 1, st,
                         fused ? gdone : nullptr, groups + (int) L->n_expert));
     // down: one act row per (token, slot), in the same expert order as gate/up: the sorted rows are the pairs
@@ -1987,7 +2000,7 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
         m.gdone = gdone;
         m.status = status;
         moe_test_hooks(&m.spin_limit, &m.gwait);  // withheld arrivals; + the gate/up row blocks per group
-        FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, x_form, m, st));
+        FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, x_form, act_form, m, st));
     } else {
         FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st, ride_gu ? &sgu : nullptr, x_form));
         // whole-row amax: a second pass over the f32 act rows (reference src/kernels.cu:534-552)

@@ -65,24 +65,29 @@ def test_dense_prefill_int8(ops, qtype, T, H, F):
 
 
 @pytest.mark.parametrize("gu,down", [(orc.Q4_K, orc.Q4_K), (orc.Q4_K, orc.Q6_K), (orc.Q5_K, orc.IQ4_XS),
-                                     (orc.IQ3_XXS, orc.IQ3_S), (orc.Q8_0, orc.Q8_0), (orc.Q6_K, orc.Q5_K)])
-@pytest.mark.parametrize("counts", [(1, 2, 7, 8, 9), (32, 33, 40, 64, 72)])
-def test_prefill_group_sizes(ops, gu, down, counts):
+                                     (orc.IQ3_XXS, orc.IQ3_S), (orc.Q8_0, orc.Q8_0), (orc.Q6_K, orc.Q5_K),
+                                     (orc.Q3_K, orc.Q4_K), (orc.Q4_K, orc.Q3_K)])
+@pytest.mark.parametrize("E,counts", [(8, (1, 2, 7, 8, 9)), (8, (32, 33, 40, 64, 72)),
+                                      (256, (1, 2, 7, 8, 9, 32, 33, 40, 64, 72))])
+def test_prefill_group_sizes(ops, gu, down, E, counts):
     """The prefill layer with experts of exactly these loads (a router that picks each token's expert): one tile, two
-    tiles and their remainders, in one launch or two, gate/up and down in either form of the GEMM."""
-    H, F, E = 512, 256, 8
+    tiles and their remainders, in one launch or two, gate/up and down in either form of the GEMM (8 experts: at most
+    256 gate/up workgroups, the split form; 256 experts: the int8 form for the types that have it)."""
+    H, F = 512, 256
     owner = np.concatenate([np.full(n, e) for e, n in enumerate(counts)])
     T = owner.size
     rng = np.random.default_rng(T + gu)
     router = np.zeros((E, H), np.float32)
     x = gaussian(rng, (T, H))
-    for e in range(E):  # columns 0..7 carry the choice
+    for e in range(len(counts)):  # the first columns carry the choice
         router[e, e] = 50.0
-    x[:, :E] = 0.0
+    x[:, :len(counts)] = 0.0
     x[np.arange(T), owner] = 4.0
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
-    mats = [np.stack([weights(t, r, c, 10 * k + e).reshape(-1) for e in range(E)])
-            for k, (t, r, c) in enumerate([(gu, F, H), (gu, F, H), (down, H, F)])]
+    mats = []
+    for k, (t, r, c) in enumerate([(gu, F, H), (gu, F, H), (down, H, F)]):
+        used = [weights(t, r, c, 100 * k + e).reshape(-1) for e in range(len(counts))]
+        mats.append(np.stack([used[e % len(used)] for e in range(E)]))
     slots = ops.ExpertSlots.from_tensors(*(torch.from_numpy(m) for m in mats))
     layer = ops.MoeLayer(dev(router), slots, gu, down, H, F, 1)
     pre = ops.MoePrefill(layer)
