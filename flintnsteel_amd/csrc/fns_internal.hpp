@@ -13,6 +13,9 @@
 namespace fns::impl {
 
 int quantize_q8_1(const float *x, void *xq, int64_t ncols, int64_t nrows, hipStream_t st);
+bool mmvq_f32_fits(int type, const float *x, int64_t ncols);
+int mmvq_f32_add(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, const float *resid, float *dst,
+                 hipStream_t st);
 int rms_norm_q8_1(const float *x, const float *w, float *out, void *xq, int n, float eps, int rows, hipStream_t st);
 int amax_guard(float *act, float *escale, int n, int rows, hipStream_t st);
 int amax_guard_q8_1(const float *act, float *escale, void *xq, int n, int rows, hipStream_t st);

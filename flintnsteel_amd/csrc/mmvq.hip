@@ -18,6 +18,7 @@
 #include "fns_quarter.hpp"
 #include "fns_host.hpp"
 #include "fns_internal.hpp"
+#include "fns_q8x8.hpp"
 
 namespace fns {
 
@@ -40,6 +41,7 @@ struct MmvqParams {
     int ncol_dense;  // > 0: one channel, columns j < ncol_dense read x row j and write dst row j
     float *dst;
     int ncols, nrows;
+    const float *x_f32, *resid;  // F32ADD: the f32 row to quantise (instead of xq) and the vector added to the result
 };
 
 // Channel c -> its matrices (A; B = gate for GLU), live columns, activation rows and output rows.
@@ -241,7 +243,50 @@ __device__ __forceinline__ void stage_q8_1_img(const uint8_t *__restrict__ src, 
     }
 }
 
-template <int T, int LPR, int NC, bool GLU>
+// The image of Q8_1(x) for an f32 row (ncols a multiple of 256; the columns up to npad are zeros): the blocks that
+// quantize_q8_1 writes and stage_q8_1_img reads back, quantised by every workgroup for itself. Bound by the latency of
+// the row's loads: four 2048-column pieces are in flight at a time (one at a time the layer took 0.9 us more). Asking for
+// the workgroup's weights ahead of it, a byte of every line, made it slower (7.4 -> 7.5 us at 6144 -> 2048).
+__device__ __forceinline__ void stage_f32_img(const float *__restrict__ x, int ncols, int npad, uint8_t *img, int tid) {
+    constexpr int U = 4;
+    float *d = (float *) (img + img_q_bytes(npad)), *s16 = d + npad / 32, *s32 = s16 + npad / 16;
+    for (int c0 = 8 * tid; c0 < npad; c0 += U * 2048) {
+        float4 a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int c = min(c0 + 2048 * u, ncols - 8);
+            a[u] = *(const float4 *) (x + c);
+            b[u] = *(const float4 *) (x + c + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int c = c0 + 2048 * u;
+            if (c >= npad) break;  // (a block's four lanes are all in or all out)
+            const bool in = c < ncols;
+            const float v[8] = {in ? a[u].x : 0.0f, in ? a[u].y : 0.0f, in ? a[u].z : 0.0f, in ? a[u].w : 0.0f,
+                                in ? b[u].x : 0.0f, in ? b[u].y : 0.0f, in ? b[u].z : 0.0f, in ? b[u].w : 0.0f};
+            const Q8x8 q = q8_1_x8(v);
+            const float dh = half_to_float(float_to_half(q.d));
+            uint32_t w[2] = {0, 0};
+            int sum = 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                w[k / 4] |= (uint32_t) (uint8_t) (int8_t) q.q[k] << (8 * (k % 4));
+                sum += q.q[k];
+            }
+            *(uint2 *) (img + img_q_index(c)) = make_uint2(w[0], w[1]);
+            const int s2 = sum + xor_lane_i<1>(sum), s4 = s2 + xor_lane_i<2>(s2);
+            if (c % 16 == 0) s16[c / 16] = dh * (float) s2;
+            if (c % 32 == 0) {
+                d[c / 32] = dh;
+                s32[c / 32] = dh * (float) s4;
+            }
+        }
+    }
+}
+
+// F32ADD: the activation row is p.x_f32, quantised here, and p.resid is added to the result.
+template <int T, int LPR, int NC, bool GLU, bool F32ADD>
 __global__ __launch_bounds__(256) void k_mmvq_q(const MmvqParams p) {
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int BB = Traits<T>::bytes;
@@ -256,7 +301,8 @@ __global__ __launch_bounds__(256) void k_mmvq_q(const MmvqParams p) {
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
         img[j] = act_img(smem + j * ib, npad);
-        if (j < ncol) stage_q8_1_img(p.xq + (int64_t) xrow[j] * p.xq_row_bytes, npad, smem + j * ib, tid, 256);
+        if constexpr (F32ADD) stage_f32_img(p.x_f32, p.ncols, npad, smem, tid);
+        else if (j < ncol) stage_q8_1_img(p.xq + (int64_t) xrow[j] * p.xq_row_bytes, npad, smem + j * ib, tid, 256);
     }
     iq_grids_to_lds<T>(tid, 256);  // (visible after the barrier)
     __syncthreads();
@@ -287,7 +333,7 @@ __global__ __launch_bounds__(256) void k_mmvq_q(const MmvqParams p) {
             v += 0.0f;  // fused-GLU epilogue with zero biases (reference src/ggml/ggml_mmvq.cu:240-247)
             v *= silu(gsum + 0.0f);
         }
-        if (lane == 0 && j < ncol && row < p.nrows) out[j][row] = v;
+        if (lane == 0 && j < ncol && row < p.nrows) out[j][row] = F32ADD ? p.resid[row] + v : v;
     }
 }
 
@@ -295,13 +341,17 @@ template <int T, int NC, bool GLU> int launch_q(const MmvqParams &p, int n_chan,
     const int npad = (int) host::pad512(p.ncols);
     const size_t lds = (size_t) NC * img_bytes(npad);
     if (lds > 160 * 1024) return host::set_error(host::ERR_SHAPE, "mmvq: ncols %d too large for LDS staging", p.ncols);
-    if (p.ncols / 256 * 4 <= 16) {
-        hipLaunchKernelGGL((k_mmvq_q<T, 16, NC, GLU>), dim3((unsigned) ((p.nrows + 15) / 16), (unsigned) n_chan),
-                           dim3(256), lds, st, p);
-    } else {
-        hipLaunchKernelGGL((k_mmvq_q<T, 32, NC, GLU>), dim3((unsigned) ((p.nrows + 7) / 8), (unsigned) n_chan),
-                           dim3(256), lds, st, p);
-    }
+    auto go = [&](auto lpr) {
+        constexpr int LPR = decltype(lpr)::value, RPB = 256 / LPR;
+        const dim3 grid((unsigned) ((p.nrows + RPB - 1) / RPB), (unsigned) n_chan);
+        auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p); };
+        if constexpr (NC == 1 && !GLU) {
+            if (p.x_f32) return launch(k_mmvq_q<T, LPR, NC, GLU, true>);
+        }
+        launch(k_mmvq_q<T, LPR, NC, GLU, false>);
+    };
+    if (p.ncols / 256 * 4 <= 16) go(std::integral_constant<int, 16>{});
+    else go(std::integral_constant<int, 32>{});
     return host::check_launch("mmvq (quarters)");
 }
 
@@ -352,6 +402,30 @@ int mmvq(int type, const void *w, int64_t ncols, int64_t nrows, const void *xq, 
         FNS_TRY(n == 1 ? launch_type<1, false>(type, p, 1, st) : launch_type<4, false>(type, p, 1, st));
     }
     return host::OK;
+}
+
+// out = resid + W . Q8_1(x) for one f32 row x (16-byte aligned), types of the quarter form: the Q8_1 blocks, the GEMV and
+// the addition of quantize_q8_1, mmvq and add, bit for bit, in one launch.
+bool mmvq_f32_fits(int type, const float *x, int64_t ncols) {
+    return host::is_supported(type) && !host::is_kquant(type) && ((uintptr_t) x & 15) == 0 && ncols > 0 && ncols % 256 == 0 &&
+           img_bytes((int) host::pad512(ncols)) <= 64 * 1024;
+}
+int mmvq_f32_add(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, const float *resid, float *dst,
+                 hipStream_t st) {
+    FNS_TRY(check_shape(type, ncols, nrows));
+    if (!w || !x || !resid || !dst || !mmvq_f32_fits(type, x, ncols))
+        return host::set_error(host::ERR_SHAPE, "mmvq_f32_add: bad arguments");
+    MmvqParams p{};
+    p.base = (const uint8_t *) w;
+    p.x_f32 = x;
+    p.resid = resid;
+    p.n_xq = 1;
+    p.x_div = 1;
+    p.ncol_dense = 1;
+    p.dst = dst;
+    p.ncols = (int) ncols;
+    p.nrows = (int) nrows;
+    return launch_type<1, false>(type, p, 1, st);
 }
 
 int mmvq_ids(int type, const void *w, int64_t ncols, int64_t nrows, int64_t n_mats, const void *xq, int64_t n_xq,

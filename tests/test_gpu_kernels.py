@@ -364,3 +364,27 @@ def test_add(ops, n, off):
     assert np.array_equal(got, (x[off:] + y[off:]).astype(np.float32))
     ops.add(xd[off:], yd[off:], out=xd[off:])
     assert np.array_equal(host(xd)[off:], got)
+
+
+@pytest.mark.parametrize("qtype", [orc.Q8_0, orc.IQ4_XS, orc.IQ3_XXS, orc.IQ2_S])
+@pytest.mark.parametrize("H,F", [(256, 256), (512, 768), (264 * 32, 1280), (256, 16384)])
+def test_dense_ffn_one_token_down_launch(ops, qtype, H, F):
+    """One token's down GEMV quantises act and adds the residual in its own launch (types of the quarter form): the
+    same bits as the separate launches, which two tokens take, at widths below, off and above the 512-column padding
+    and on both sides of the 16-lane rows' limit; in place too; a NaN in x reaches every output."""
+    from tests.iq_data import random_blocks, register_grids, register_grids_in_library
+    register_grids_in_library(register_grids())
+    rng = np.random.default_rng(H + F)
+    gate, up = (orc.quantize(orc.Q8_0, gaussian(rng, (F, H), 0.05)) for _ in range(2))
+    down = orc.quantize(qtype, gaussian(rng, (H, F), 0.05)) if qtype == orc.Q8_0 else random_blocks(qtype, H, F, 3)
+    norm = dev(gaussian(rng, (H,), 1.0))
+    ffn = ops.DenseFfn(dev(gate), dev(up), dev(down), orc.Q8_0, orc.Q8_0, qtype, H, F, ffn_norm=norm)
+    x = gaussian(rng, (2, H))
+    two = host(ffn(dev(x)))
+    for t in range(2):
+        one = dev(x[t:t + 1])
+        assert np.array_equal(host(ffn(one))[0], two[t])
+        ffn(one, out=one)
+        assert np.array_equal(host(one)[0], two[t])
+    x[0, 5] = np.nan
+    assert np.isnan(host(ffn(dev(x[:1])))).all()
