@@ -5,9 +5,11 @@
 // (token, slot) pairs by expert, the activations are quantised once per source row, the GEMM writes each row back to
 // its (token, slot) position), include/fns/ggml_kernels.h:50-69. This is a new CDNA4 design, not ggml's mmq.cuh:
 //
-//   * The K-quant scales change every 32 (Q4_K, Q5_K) or 16 (Q6_K, Q3_K) columns and the Q8_1 scale d8 every 32, so an
-//     int8 MFMA per sub-block needs a convert + scale + add per output element per sub-block: VALU-bound. Here the
-//     scales are folded into the operands instead, exactly: A = q8 * d8 as two f16 halves (hi + lo, see the image
+//   * Two forms of the GEMM. Types whose scales change every 32 columns (Q4_K, Q5_K, Q8_0, IQ4_XS, IQ3_XXS, IQ3_S) run on
+//     int8 MFMA, one exact integer dot per sub-block and a convert + scale + fma per output (fns_mmq_i8.hpp). The others
+//     (Q6_K and Q3_K scale every 16 columns, IQ2_S every 16), and calls of at most 256 gate/up workgroups, run the split
+//     form of this file, to which the points below apply:
+//   * In the split form the scales are folded into the operands instead, exactly: A = q8 * d8 as two f16 halves (hi + lo, see the image
 //     layout below), B = integer code * integer sub-block scale as f16 (|B| <= 2048: exact; Q6_K's 8-bit scales are
 //     split in two operands). v_mfma_f32_32x32x16_f16 then accumulates a whole 256-column superblock, and only the
 //     superblock's float scales d (and dmin times one more MFMA of the min term) touch the accumulators.

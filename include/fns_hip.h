@@ -204,7 +204,8 @@ int fns_hip_moe_layer_stage(const FnsMoeLayer *layer, int stage, const float *x,
 
 /* --- prefill / batched expert GEMM (MMQ) ---
  * Q8_1 activation rows for the MMQ path are kept as "split images" (q8 * d8 as two f16 halves per value, then the
- * per-32 scaled sums as f16 halves: 4.125 bytes per value): fns_hip_mmq_q8_1_bytes(ncols, nrows) bytes hold nrows
+ * per-32 scaled sums as f16 halves: 4.125 bytes per value; Q8_0, and the layers below for the types scaled every 32
+ * columns, use int8 codes, scales and sums, 1.25 bytes per value, in the same room): fns_hip_mmq_q8_1_bytes(ncols, nrows) bytes hold nrows
  * of them plus 4096 bytes of slack (mmq_experts keeps its group lists there). */
 /* include/fns/ggml_kernels.h:53-54 mmq_q8_1_bytes */
 size_t fns_hip_mmq_q8_1_bytes(int64_t ncols, int64_t nrows);
@@ -212,9 +213,9 @@ size_t fns_hip_mmq_q8_1_bytes(int64_t ncols, int64_t nrows);
 size_t fns_hip_mmq_bounds_bytes(int64_t n_expert);
 /* include/fns/ggml_kernels.h:56-58 mmq: dst[t][nrows] = W . q8_1(x[t]), x f32 [n_tok][ncols]; xq scratch of
  * fns_hip_mmq_q8_1_bytes(ncols, n_tok) bytes. ncols a multiple of 256, nrows of 64. Types (the reference's MMQ set,
- * src/ggml/ggml_mmq.cu:59-66, plus Q3_K): the K-quants and IQ4_XS / IQ3_XXS / IQ3_S / IQ2_S (the last three once
- * their codebooks are registered) on the tiled MFMA GEMM; Q8_0 (any nrows) on the GEMV kernels, a few token columns
- * per weight pass. */
+ * src/ggml/ggml_mmq.cu:59-66, plus Q3_K): the K-quants, Q8_0 and IQ4_XS / IQ3_XXS / IQ3_S / IQ2_S (the last three once
+ * their codebooks are registered) on the tiled MFMA GEMM; Q8_0 takes any nrows: one that is not a multiple of 64 runs on
+ * the GEMV kernels, a few token columns per weight pass. */
 int fns_hip_mmq(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, int64_t n_tok, void *xq,
                 float *dst, void *stream);
 /* include/fns/ggml_kernels.h:60-69 MmqIdsScratch + mmq_experts: dst[t][j][nrows] = W_e . q8_1(x[t][j % x_rows_per_tok]),
@@ -246,7 +247,7 @@ int fns_hip_moe_prefill_section(const FnsMoeLayer *layer, int64_t n_tok, int sec
 int fns_hip_moe_prefill(const FnsMoeLayer *layer, const float *x, const float *x_resid, float *out, int64_t n_tok,
                         void *workspace, size_t workspace_bytes, void *stream);
 /* No counterpart in the reference. Without the F16 guard and for gate/up and down types from {Q3_K, Q4_K}, gate/up
- * and down run as one launch whose down workgroups wait (bounded) for their row group's gate/up
+ * and down (each on the image form of its type) run as one launch whose down workgroups wait (bounded) for their row group's gate/up
  * workgroups; one that gives up writes NaN to its output rows and sets FNS_STATUS_EXCHANGE_TIMEOUT in the workspace's
  * status word (section 8, which the workspace must hold zeroed when first used). As fns_hip_moe_layer_status: waits
  * for the stream's work so far, stores the word in *status and, with clear = 1, zeroes it. The poll limit and
