@@ -359,7 +359,7 @@ __global__ __launch_bounds__(256) void k_guard_image(float *__restrict__ act, fl
 // Router GEMM tiles and the split activation image of the same rows in one launch (the two only read x): workgroups
 // [0, n_rt) are router tiles (tile (id % tiles_x, id / tiles_x)), the rest quantise two 2048-column pieces of x each,
 // as k_quant_image does, so the image is built on the CUs the router tiles leave free.
-template <bool BF16>
+template <bool BF16, bool TILE32>
 __global__ __launch_bounds__(512) void k_router_image(const void *__restrict__ w, const float *__restrict__ bias,
                                                       const float *__restrict__ x, float *__restrict__ y, int ncols,
                                                       int nrows, int n_tok, int tiles_x, int n_rt,
@@ -368,7 +368,8 @@ __global__ __launch_bounds__(512) void k_router_image(const void *__restrict__ w
     PF_MARK(0, 0);
     const int id = blockIdx.x;
     if (id < n_rt) {
-        router_gemm_tile<BF16, true>(w, bias, x, y, ncols, nrows, n_tok, id % tiles_x, id / tiles_x);
+        if constexpr (TILE32) router_gemm_tile32<BF16>(w, bias, x, y, ncols, nrows, n_tok, id % tiles_x, id / tiles_x);
+        else router_gemm_tile<BF16, true>(w, bias, x, y, ncols, nrows, n_tok, id % tiles_x, id / tiles_x);
         PF_MARK(0, 1);
         return;
     }
@@ -1933,17 +1934,18 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     const bool one = (bf || L->router_dtype == 0) && H % 64 == 0 && (int64_t) H * std::max<int64_t>(n_tok, NE) < INT32_MAX &&
                      ((uintptr_t) x & 15) == 0 && ((uintptr_t) L->router_w & (bf ? 7 : 15)) == 0;
     if (one) {
-        const int tiles_x = (int) ((n_tok + 15) / 16), n_rt = tiles_x * ((NE + 15) / 16);
+        const bool t32 = (n_tok + 31) / 32 * ((NE + 31) / 32) >= kRouterTile32Min;
+        const int side = t32 ? 32 : 16, tiles_x = (int) ((n_tok + side - 1) / side), n_rt = tiles_x * ((NE + side - 1) / side);
         const int nxb = (H + 2047) / 2048;
         const int64_t n_img = have_img ? 0 : (nxb * n_tok + 1) / 2;
         if (n_rt + n_img > INT32_MAX) return host::set_error(host::ERR_SHAPE, "prefill: grid too large");
         const dim3 g((unsigned) (n_rt + n_img));
-        if (bf)
-            hipLaunchKernelGGL(k_router_image<true>, g, dim3(512), 0, st, L->router_w, L->router_bias, x, logits, H, NE,
-                               (int) n_tok, tiles_x, n_rt, x_form, (uint8_t *) sec[3], x_img, nxb);
-        else
-            hipLaunchKernelGGL(k_router_image<false>, g, dim3(512), 0, st, L->router_w, L->router_bias, x, logits, H,
-                               NE, (int) n_tok, tiles_x, n_rt, x_form, (uint8_t *) sec[3], x_img, nxb);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, g, dim3(512), 0, st, L->router_w, L->router_bias, x, logits, H, NE, (int) n_tok, tiles_x,
+                               n_rt, x_form, (uint8_t *) sec[3], x_img, nxb);
+        };
+        if (bf) t32 ? go(k_router_image<true, true>) : go(k_router_image<true, false>);
+        else t32 ? go(k_router_image<false, true>) : go(k_router_image<false, false>);
         FNS_TRY(host::check_launch("prefill router + image"));
     } else {
         FNS_TRY(gemm_router_bias(L->router_dtype, L->router_w, L->router_bias, x, logits, L->hidden, L->n_expert,

@@ -109,3 +109,33 @@ def test_prefill_group_sizes(ops, gu, down, E, counts):
         assert err.max() <= bound, f"expert {e} ({t.size} rows): {err.max():.3e} > {bound:.3e}"
         tight.append(err <= 1e-5 * np.abs(ref).max())
     assert np.concatenate(tight).mean() >= 0.8
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("H,E,T", [(256, 256, 993), (576 * 4, 250, 1025), (512, 33, 4097)])
+def test_prefill_router_tiles(ops, bf16, H, E, T):
+    """The router GEMM's 32 x 32 tiles (at least 256 of them) give every token the logits of the 16 x 16 tiles, which a
+    call of fewer tokens takes, bit for bit: ragged token and expert counts, fewer column chunks than waves and more."""
+    rng = np.random.default_rng(T)
+    F = 256
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    router = dev(gaussian(rng, (E, H)))
+    x = dev(gaussian(rng, (T, H)))
+    mats = [np.repeat(weights(orc.Q4_K, r, c, k).reshape(1, -1), E, axis=0)
+            for k, (r, c) in enumerate([(F, H), (F, H), (H, F)])]
+    slots = ops.ExpertSlots.from_tensors(*(torch.from_numpy(m) for m in mats))
+    layer = ops.MoeLayer(router.bfloat16() if bf16 else router, slots, orc.Q4_K, orc.Q4_K, H, F, 1)
+    pre = ops.MoePrefill(layer)
+
+    def logits(xs):
+        ws = pre.workspace(xs.shape[0])
+        pre(xs, ws=ws)
+        return pre.trace(ws, xs.shape[0])["logits"].cpu().numpy()
+
+    whole = logits(x)
+    w64, x64 = (t.bfloat16().double() if bf16 else t.double() for t in (router, x))
+    ref = (x64 @ w64.T).cpu().numpy()
+    assert np.abs(whole - ref).max() <= 1e-5 * np.abs(ref).max()  # fp32 sums of at most 2304 products
+    step = 300
+    for t in range(0, T, step):
+        assert np.array_equal(logits(x[t:t + step].contiguous()), whole[t:t + step]), f"tokens from {t}"
