@@ -392,7 +392,7 @@ struct MmqArgs {
     const int32_t *gprefix;    // [2][n_expert + 1] group prefixes: 64-row groups, then the <= 32-row remainders
     int n_main;                // launch: groups of the 64-row list (then the remainder list up to n_groups)
     int n_groups, n_cb;        // launch: groups in both lists; weight row blocks per group
-    const int32_t *src;        // sorted position -> activation image row (null: identity)
+    const int32_t *src;        // sorted position -> activation image row (null: identity, dense only)
     const int32_t *dst_rows;   // sorted position -> output row (null: identity)
     int n_rows;                // dense: number of activation rows
     int dense_small;           // dense: 1 = groups of 32 activation rows (one tile), 0 = of 64
@@ -447,9 +447,17 @@ template <> struct WFrag<T_IQ2_S> { uint32_t d; uint2 qh, sc; uint4 idx[2], sg[2
 
 // Buffer loads: a uniform base in a resource (SGPRs), a 32-bit per-lane offset and a uniform offset - no 64-bit
 // address arithmetic per load. (Unaligned dword access is enabled on the platform, as for the plain global loads.)
+// A resource reaches kRsrcBytes from its base (a read past that gives zeros), so one launch's scattered image rows lie
+// within that many bytes (image_tokens), and rows in order are read from their group's first.
 typedef __amdgpu_buffer_rsrc_t Rsrc;
+constexpr int64_t kRsrcBytes = 0x7FFFFFFF;
 __device__ __forceinline__ Rsrc rsrc_of(const void *base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0x7FFFFFFF, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int) kRsrcBytes, 0x00020000);
+}
+// Activation image rows of a group whose first sorted row is seg: a.src names them from the image's start; without it they
+// are rows seg, seg + 1, ... and are counted from seg.
+__device__ __forceinline__ Rsrc image_rsrc(const uint8_t *img, int64_t row_bytes, bool listed, int seg) {
+    return rsrc_of(listed ? img : img + seg * row_bytes);
 }
 __device__ __forceinline__ uint4 bload16(Rsrc r, uint32_t vo, uint32_t so) {
     const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
@@ -974,7 +982,7 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
     MMQ_NOTE(NT * 1000 + cnt);
     for (int i = tid; i < ROWS; i += kMmqThreads) {
         const int q = seg + min(i, cnt - 1);
-        sh_src[i] = a.src ? a.src[q] : q;
+        sh_src[i] = a.src ? a.src[q] : q - seg;
         sh_dst[i] = a.dst_rows ? a.dst_rows[q] : q;
     }
 
@@ -984,7 +992,7 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
     // weight rows past nrows (nrows % WROWS != 0) are computed from the last row and not stored
     const int row0 = wb * WROWS + wave * 32 + jl;
     const int ra = min(row0, a.nrows - 1), rb = GLU ? ra : min(row0 + 128, a.nrows - 1);
-    const Rsrc r0 = rsrc_of(wbase + a.off_a), r1 = rsrc_of(wbase + (GLU ? a.off_b : a.off_a)), rx = rsrc_of(a.xpack);
+    const Rsrc r0 = rsrc_of(wbase + a.off_a), r1 = rsrc_of(wbase + (GLU ? a.off_b : a.off_a)), rx = image_rsrc(a.xpack, a.x_img, a.src, seg);
     const uint32_t v0 = (uint32_t) (ra * row_bytes), v1 = (uint32_t) (rb * row_bytes);
     const uint32_t c0 = v0 + 16 * hh, c1 = v1 + 16 * hh;
     __syncthreads();  // sh_src / sh_dst
@@ -1609,6 +1617,12 @@ int mmq_compact(const int32_t *ids, int64_t n_tok, int64_t k, int64_t n_expert, 
 // different workgroups at different times, and a line read for one row must never carry another row's older bytes.
 int64_t act_stride(int64_t ncols, int form = kImgSplit) { return ((int64_t) mmq_form_bytes(form, ncols) + 127) / 128 * 128; }
 
+// Tokens of one expert launch, whose tokens' image rows (row_bytes a token) a buffer resource has to reach: all of a call
+// whose images are below 2 GiB, otherwise ranges of tokens one after another.
+int64_t image_tokens(int64_t n_tok, int64_t row_bytes) {
+    return std::min(n_tok, std::max<int64_t>(1, kRsrcBytes / std::max<int64_t>(1, row_bytes)));
+}
+
 // the 64-row list's upper bound for n_pairs sorted rows over n_expert experts: sum_e (n_e / 64 + (n_e % 64 > 32))
 int64_t main_groups(int64_t n_expert, int64_t n_pairs) { return n_expert + (n_pairs + kMmqTok - 1) / kMmqTok; }
 
@@ -1690,13 +1704,24 @@ int mmq_experts(int type, const char *const *table, size_t off, int64_t ncols, i
     // the slack that mmq_q8_1_bytes adds after the activation images (4096 bytes >= 257 ints)
     const int64_t rows = n_tok * x_rows_per_tok;
     int32_t *gprefix = (int32_t *) ((uint8_t *) xq + (size_t) rows * mmq_image_bytes(ncols));
-    FNS_TRY(mmq_compact(ids, n_tok, n_used, n_expert, x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, st));
     const int form = type == T_Q8_0 ? kImgI8 : kImgSplit;
+    const int64_t img = (int64_t) mmq_form_bytes(form, ncols);
+    FNS_TRY(mmq_compact(ids, n_tok, n_used, n_expert, x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, st));
     FNS_TRY(mmq_quant_image(x, ncols, rows, form, xq, st));
-    MmqArgs a;
-    FNS_TRY(expert_args(type, table, off, 0, false, ncols, nrows, n_expert, xq, ids_src1, ids_dst, bounds, gprefix, dst,
-                        nullptr, nullptr, a, (int64_t) mmq_form_bytes(form, ncols)));
-    return launch_mmq(type, false, a, (int) main_groups(n_expert, n_tok * n_used), st, nullptr, form);
+    const int64_t step = image_tokens(n_tok, x_rows_per_tok * img);
+    for (int64_t t = 0; t < n_tok; t += step) {
+        const int64_t n = std::min(step, n_tok - t);
+        if (step < n_tok)
+            FNS_TRY(mmq_compact(ids + t * n_used, n, n_used, n_expert, x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, st));
+        MmqArgs a;
+        FNS_TRY(expert_args(type, table, off, 0, false, ncols, nrows, n_expert, (uint8_t *) xq + t * x_rows_per_tok * img,
+                            ids_src1, ids_dst, bounds, gprefix, dst + t * n_used * nrows, nullptr, nullptr, a, img));
+        FNS_TRY(launch_mmq(type, false, a, (int) main_groups(n_expert, n * n_used), st, nullptr, form));
+    }
+    // the sort that the caller's arrays are left with is the whole call's
+    if (step < n_tok)
+        FNS_TRY(mmq_compact(ids, n_tok, n_used, n_expert, x_rows_per_tok, ids_src1, ids_dst, bounds, gprefix, st));
+    return host::OK;
 }
 
 // ---- prefill MoE layer ----------------------------------------------------------------------------------------
@@ -1955,63 +1980,74 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     FNS_TRY(route_topk(logits, ids, w, L->n_expert, L->k, (int) n_tok, L->gating, L->norm_w, st));
     // gate/up (SwiGLU and the Q8_1 of act fused) and down: act image rows padded to whole cache lines; one launch
     // unless the F16 guard's whole-row amax has to sit between them (or the type pair has no fused kernel)
-    const int groups = (int) main_groups(L->n_expert, P);
     const int64_t astride = act_stride(L->inter, act_form);
-    int32_t *gdone = bounds + 3 * (L->n_expert + 1);
-    uint32_t *status = (uint32_t *) (gdone + groups + L->n_expert);
-    const bool fused = !L->guard && mmq_moe_kernel(L->gu_type, L->down_type, x_form, act_form) && P * astride < INT32_MAX;
-    FNS_TRY(mmq_compact(ids, n_tok, L->k, L->n_expert, 1, src1, dstr, bounds, bounds + L->n_expert + 1, st,
-                        fused ? gdone : nullptr, groups + (int) L->n_expert));
-    // down: one act row per (token, slot), in the same expert order as gate/up: the sorted rows are the pairs
-    // themselves (activation row = output row = p), so the gate/up sort is reused with ids_dst as the source list
-    MmqArgs gu, dn;
-    FNS_TRY(expert_args(L->gu_type, table, L->gate_off, L->up_off, true, L->hidden, L->inter, L->n_expert, sec[3], src1,
-                        dstr, bounds, bounds + L->n_expert + 1, nullptr, sec[4], L->guard ? act : nullptr, gu, x_img,
-                        astride));
-    gu.out_form = act_form;
-    FNS_TRY(expert_args(L->down_type, table, L->down_off, 0, false, L->inter, L->hidden, L->n_expert, sec[4], dstr,
-                        dstr, bounds, bounds + L->n_expert + 1, dexp, nullptr, nullptr, dn, astride));
-    // the shared expert (reference src/engine.cu:351-355): in the routed launches where the types agree
-    float *sh = has_sh ? (float *) sec[14] : nullptr;
-    MmqShared sgu{}, sdn{};
+    int32_t *gprefix = bounds + L->n_expert + 1, *gdone = bounds + 3 * (L->n_expert + 1);
+    uint32_t *status = (uint32_t *) (gdone + main_groups(L->n_expert, P) + L->n_expert);
+    const bool fused = !L->guard && mmq_moe_kernel(L->gu_type, L->down_type, x_form, act_form);
     if (has_sh) {
         FNS_TRY(check_mmq_shape(sgt, L->hidden, L->shexp_inter));
         FNS_TRY(check_mmq_shape(sdt, L->shexp_inter, L->hidden));
-        sgu = shared_gate_up(L, sec[3], x_form, n_tok, sec[13], sh_form);
-        sdn = shared_down(L, sec[13], sh_form, n_tok, sh);
     }
-    const bool ride_gu = has_sh && !fused && sgt == L->gu_type, ride_dn = has_sh && !fused && sdt == L->down_type;
-    if (has_sh && !ride_gu) FNS_TRY(mmq_dense_shared(sgt, true, x_form, sgu, st));
-    if (fused) {
-        MoeArgs m{};
-        m.table = table;
-        m.gate_off = (int64_t) L->gate_off;
-        m.up_off = (int64_t) L->up_off;
-        m.down_off = (int64_t) L->down_off;
-        m.hidden = (int) L->hidden;
-        m.inter = (int) L->inter;
-        m.n_expert = (int) L->n_expert;
-        m.n_main = groups;
-        m.ximg = sec[3];
-        m.x_img = x_img;
-        m.aimg = sec[4];
-        m.a_img = astride;
-        m.bounds = bounds;
-        m.gprefix = bounds + L->n_expert + 1;
-        m.src1 = src1;
-        m.dstr = dstr;
-        m.dexp = dexp;
-        m.gdone = gdone;
-        m.status = status;
-        moe_test_hooks(&m.spin_limit, &m.gwait);  // withheld arrivals; + the gate/up row blocks per group
-        FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, x_form, act_form, m, st));
-    } else {
-        FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st, ride_gu ? &sgu : nullptr, x_form));
-        // whole-row amax: a second pass over the f32 act rows (reference src/kernels.cu:534-552)
-        if (L->guard) FNS_TRY(mmq_guard_image(act, escale, L->inter, P, act_form, sec[4], astride, st));
-        FNS_TRY(launch_mmq(L->down_type, false, dn, groups, st, ride_dn ? &sdn : nullptr, act_form));
+    const int64_t sh_img = has_sh ? (int64_t) mmq_form_bytes(sh_form, L->shexp_inter) : 0;
+    float *sh = has_sh ? (float *) sec[14] : nullptr;
+    // tokens [t, t + n): all of them unless an image has 2 GiB or more (image_tokens)
+    const int64_t step = image_tokens(n_tok, std::max(x_img, L->k * astride));
+    for (int64_t t = 0; t < n_tok; t += step) {
+        const int64_t n = std::min(step, n_tok - t), p0 = t * L->k, np = n * L->k;
+        const int groups = (int) main_groups(L->n_expert, np);
+        const uint8_t *ximg = sec[3] + t * x_img;
+        uint8_t *aimg = sec[4] + p0 * astride, *shimg = has_sh ? sec[13] + t * sh_img : nullptr;
+        FNS_TRY(mmq_compact(ids + p0, n, L->k, L->n_expert, 1, src1 + p0, dstr + p0, bounds, gprefix, st,
+                            fused ? gdone : nullptr, groups + (int) L->n_expert));
+        // down: one act row per (token, slot), in the same expert order as gate/up: the sorted rows are the pairs
+        // themselves (activation row = output row = p), so the gate/up sort is reused with ids_dst as the source list
+        MmqArgs gu, dn;
+        FNS_TRY(expert_args(L->gu_type, table, L->gate_off, L->up_off, true, L->hidden, L->inter, L->n_expert, ximg,
+                            src1 + p0, dstr + p0, bounds, gprefix, nullptr, aimg,
+                            L->guard ? act + p0 * L->inter : nullptr, gu, x_img, astride));
+        gu.out_form = act_form;
+        FNS_TRY(expert_args(L->down_type, table, L->down_off, 0, false, L->inter, L->hidden, L->n_expert, aimg, dstr + p0,
+                            dstr + p0, bounds, gprefix, dexp + p0 * L->hidden, nullptr, nullptr, dn, astride));
+        // the shared expert (reference src/engine.cu:351-355): in the routed launches where the types agree
+        MmqShared sgu{}, sdn{};
+        if (has_sh) {
+            sgu = shared_gate_up(L, ximg, x_form, n, shimg, sh_form);
+            sdn = shared_down(L, shimg, sh_form, n, sh + t * L->hidden);
+        }
+        const bool ride_gu = has_sh && !fused && sgt == L->gu_type, ride_dn = has_sh && !fused && sdt == L->down_type;
+        if (has_sh && !ride_gu) FNS_TRY(mmq_dense_shared(sgt, true, x_form, sgu, st));
+        if (fused) {
+            MoeArgs m{};
+            m.table = table;
+            m.gate_off = (int64_t) L->gate_off;
+            m.up_off = (int64_t) L->up_off;
+            m.down_off = (int64_t) L->down_off;
+            m.hidden = (int) L->hidden;
+            m.inter = (int) L->inter;
+            m.n_expert = (int) L->n_expert;
+            m.n_main = groups;
+            m.ximg = ximg;
+            m.x_img = x_img;
+            m.aimg = aimg;
+            m.a_img = astride;
+            m.bounds = bounds;
+            m.gprefix = gprefix;
+            m.src1 = src1 + p0;
+            m.dstr = dstr + p0;
+            m.dexp = dexp + p0 * L->hidden;
+            m.gdone = gdone;
+            m.status = status;
+            moe_test_hooks(&m.spin_limit, &m.gwait);  // withheld arrivals; + the gate/up row blocks per group
+            FNS_TRY(launch_mmq_moe(L->gu_type, L->down_type, x_form, act_form, m, st));
+        } else {
+            FNS_TRY(launch_mmq(L->gu_type, true, gu, groups, st, ride_gu ? &sgu : nullptr, x_form));
+            // whole-row amax: a second pass over the f32 act rows (reference src/kernels.cu:534-552)
+            if (L->guard)
+                FNS_TRY(mmq_guard_image(act + p0 * L->inter, escale + p0, L->inter, np, act_form, aimg, astride, st));
+            FNS_TRY(launch_mmq(L->down_type, false, dn, groups, st, ride_dn ? &sdn : nullptr, act_form));
+        }
+        if (has_sh && !ride_dn) FNS_TRY(mmq_dense_shared(sdt, false, sh_form, sdn, st));
     }
-    if (has_sh && !ride_dn) FNS_TRY(mmq_dense_shared(sdt, false, sh_form, sdn, st));
     return moe_combine(dexp, L->guard ? escale : nullptr, w, sh, x_resid, out, L->hidden, L->k, (int) n_tok, st);
 }
 

@@ -238,7 +238,8 @@ int fns_hip_mmq_compact(const int32_t *ids, int64_t n_tok, int64_t n_used, int64
  * workspace: fns_hip_moe_prefill_workspace() bytes; sections (byte offsets in offsets[6]): 0 logits f32 [n_tok][n_expert],
  * 1 ids i32 [n_tok][k], 2 w f32 [n_tok][k], 3 x images, 4 act images [n_tok * k], 5 down outputs f32 [n_tok][k][hidden]. */
 int fns_hip_moe_prefill_workspace(const FnsMoeLayer *layer, int64_t n_tok, size_t *offsets, size_t *total_bytes);
-/* Byte offset and size of any workspace section of fns_hip_moe_prefill (the six above, then 6 ids_src1, 7 ids_dst,
+/* Byte offset and size of any workspace section of fns_hip_moe_prefill (the six above, then 6 ids_src1, 7 ids_dst
+ * (a call whose x or act images have 2 GiB or more runs ranges of tokens in turn; 6 to 8 are then each range's own),
  * 8 expert bounds, group prefix, arrival counters and the status word, 9 f32 act [n_tok * k][inter] (F16 guard
  * only, after the division), 10 guard scales [n_tok * k],
  * 11 RMSNorm output, 12 its Q8_1 blocks, 13 shared-expert act images, 14 shared-expert output). Inspection and tests;

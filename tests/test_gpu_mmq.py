@@ -611,3 +611,71 @@ def test_moe_prefill_fused_launch_with_shared_expert_in_place(ops):
     assert fused.status(ws_f, T) == 0
     rows = np.flatnonzero((a != b).any(axis=1))
     assert np.isfinite(a).all() and rows.size == 0, f"rows {rows[:16].tolist()} of {rows.size} differ"
+
+
+# ---- activation images of 2 GiB and more --------------------------------------------------------------------------
+# (a buffer resource reaches 2 GiB: rows in order are read from their group's first, the experts' scattered rows in
+# ranges of tokens; every token equals the same token in a small call, bit for bit)
+
+@pytest.mark.parametrize("gu,dn,F", [(orc.Q4_K, orc.Q6_K, 14336), (orc.Q4_K, orc.Q4_K, 28672)])
+def test_moe_prefill_images_past_2gib(ops, gu, dn, F):
+    """65536 act rows of 3.9 GB (split, two launches) and of 2.3 GB (int8, one launch)."""
+    from flintnsteel_amd import synth
+    H, NE, K, T = 256, 4, 2, 32768
+    layer = synth.build_layer(H, F, NE, K, gu, dn, seed=8, layer=9)
+    pre = ops.MoePrefill(layer)
+    x = synth.activations(T, H, seed=8, layer=10)
+    ws = pre.workspace(T)
+    out = pre(x, ws=ws)
+    assert pre.status(ws, T) == 0
+    for t in (0, T // 2 - 32, T - 64):
+        xt = x[t:t + 64].contiguous()
+        assert np.array_equal(host(pre(xt)), host(out[t:t + 64])), f"tokens from {t}"
+
+
+@pytest.mark.parametrize("qtype,ncols,n_tok", [(orc.Q6_K, 14336, 37000), (orc.Q8_0, 32768, 53000)])
+def test_mmq_images_past_2gib(ops, qtype, ncols, n_tok):
+    """mmq over an image of 2.2 GB in either form."""
+    nrows = 64
+    w = dev(orc.quantize(qtype, gaussian(np.random.default_rng(1), (nrows, ncols), 0.02)))
+    x = torch.randn(n_tok, ncols, device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    out = ops.mmq(qtype, w, ncols, nrows, x)
+    for t in (0, n_tok - 80):
+        assert np.array_equal(host(ops.mmq(qtype, w, ncols, nrows, x[t:t + 80].contiguous())), host(out[t:t + 80]))
+
+
+def test_mmq_experts_images_past_2gib(ops):
+    """mmq_experts, one activation row per (token, slot), over a 2.2 GB image; the sort that is left is the whole call's."""
+    from flintnsteel_amd.ops import _p, _s, call
+    ncols, nrows, NE, K, T = 14336, 64, 4, 2, 18500
+    mats = dev(make_expert_mats(orc.Q6_K, NE, nrows, ncols, 3))
+    ids_h = distinct_ids(np.random.default_rng(4), T, K, NE)
+    ids, table = dev(ids_h), table_of(mats)
+    x = torch.randn(T * K, ncols, device="cuda", generator=torch.Generator("cuda").manual_seed(5))
+    src, dst = (torch.empty(T * K, dtype=torch.int32, device="cuda") for _ in range(2))
+    bounds = torch.empty(NE + 1, dtype=torch.int32, device="cuda")
+    xq = torch.empty(ops.mmq_q8_1_bytes(ncols, T * K), dtype=torch.uint8, device="cuda")
+    out = torch.empty(T, K, nrows, device="cuda")
+    call("fns_hip_mmq_experts", orc.Q6_K, _p(table), 0, ncols, nrows, NE, _p(x), K, T, _p(ids), K, _p(src), _p(dst),
+         _p(bounds), _p(xq), _p(out), _s())
+    for t in (0, T - 50):
+        small = ops.mmq_experts(orc.Q6_K, table, 0, ncols, nrows, NE, x[t * K:(t + 50) * K].contiguous(), K,
+                                ids[t:t + 50].contiguous())
+        assert np.array_equal(host(small), host(out[t:t + 50])), f"tokens from {t}"
+    want = np.argsort(ids_h.ravel(), kind="stable")
+    assert np.array_equal(host(dst), want) and np.array_equal(host(src), want)
+    assert np.array_equal(host(bounds), np.concatenate([[0], np.cumsum(np.bincount(ids_h.ravel(), minlength=NE))]))
+
+
+def test_dense_ffn_act_image_past_2gib(ops):
+    """The dense FFN block's prefill over an act image of 2.2 GB. A small call splits down's columns in four parts, the
+    large one in none: 32-bit sums of the same products in another order."""
+    H, F, T = 256, 14336, 37000
+    rng = np.random.default_rng(6)
+    g, u, d = (dev(orc.quantize(orc.Q6_K, gaussian(rng, s, 0.02))) for s in ((F, H), (F, H), (H, F)))
+    ffn = ops.DenseFfn(g, u, d, orc.Q6_K, orc.Q6_K, orc.Q6_K, H, F)
+    x = torch.randn(T, H, device="cuda", generator=torch.Generator("cuda").manual_seed(7))
+    out = ffn(x, prefill=True)
+    for t in (0, T - 64):
+        xt = x[t:t + 64].contiguous()
+        assert_close(host(out[t:t + 64] - xt), host(ffn(xt, prefill=True) - xt), f"tokens from {t}", 1e-5, 1e-5)
