@@ -300,7 +300,7 @@ __device__ __forceinline__ void image_store(int form, const Q8x8 &q, uint8_t *ro
     else split_put(q, ncols, col, put);
 }
 
-// x [rows][ncols] f32 -> image rows with the reference's Q8_1 arithmetic; grid (ceil(ncols / 2048), rows), 256 threads
+// x [rows][ncols] f32 -> image rows with the reference's Q8_1 arithmetic; grid (rows, ceil(ncols / 2048)), 256 threads
 // of 8 columns each (ncols % 256 == 0, so a block's 4 lanes are all in or all out).
 __device__ __forceinline__ void quant_image8(const float *__restrict__ x, int ncols, int row, int col, int form,
                                              uint8_t *__restrict__ out, int64_t img_row_bytes) {
@@ -311,7 +311,7 @@ __device__ __forceinline__ void quant_image8(const float *__restrict__ x, int nc
 }
 __global__ __launch_bounds__(256) void k_quant_image(const float *__restrict__ x, int ncols, int form,
                                                      uint8_t *__restrict__ out, int64_t img_row_bytes) {
-    const int row = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * 8;
+    const int row = blockIdx.x, col = (blockIdx.y * 256 + threadIdx.x) * 8;
     if (col < ncols) quant_image8(x, ncols, row, col, form, out, img_row_bytes);
 }
 
@@ -1556,10 +1556,10 @@ size_t mmq_form_bytes(int form, int64_t ncols) { return (size_t) (ncols / 256) *
 int mmq_form(int type) { return mmq_i8_kernel<false>(type) ? kImgI8 : kImgSplit; }
 
 int mmq_quant_image(const float *x, int64_t ncols, int64_t rows, int form, void *ximg, hipStream_t st) {
-    if (!x || !ximg || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
+    if (!x || !ximg || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > INT32_MAX)
         return host::set_error(host::ERR_SHAPE, "mmq quantize: bad arguments");
     if (rows == 0) return host::OK;
-    hipLaunchKernelGGL(k_quant_image, dim3((unsigned) ((ncols + 2047) / 2048), (unsigned) rows), dim3(256), 0, st, x,
+    hipLaunchKernelGGL(k_quant_image, dim3((unsigned) rows, (unsigned) ((ncols + 2047) / 2048)), dim3(256), 0, st, x,
                        (int) ncols, form, (uint8_t *) ximg, (int64_t) mmq_form_bytes(form, ncols));
     return host::check_launch("mmq quantize");
 }
@@ -1586,7 +1586,7 @@ int mmq_rms_norm_image(const float *x, const float *w, float *out, void *xq, int
 
 int mmq_guard_image(float *act, float *escale, int64_t ncols, int64_t rows, int form, void *img, int64_t stride,
                     hipStream_t st) {
-    if (!act || !escale || !img || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > 65535)
+    if (!act || !escale || !img || ncols <= 0 || ncols % 256 || ncols > 65536 || rows < 0 || rows > INT32_MAX - 3)
         return host::set_error(host::ERR_SHAPE, "mmq guard: bad arguments");
     if (rows == 0) return host::OK;
     hipLaunchKernelGGL(k_guard_image, dim3((unsigned) ((rows + 3) / 4)), dim3(256), 0, st, act, escale, (int) ncols,
@@ -1667,7 +1667,7 @@ int mmq(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, i
         return mmvq(type, w, ncols, nrows, xq, dst, n_tok, st);
     }
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
-    if (!w || !x || !xq || !dst || n_tok < 0) return host::set_error(host::ERR_SHAPE, "mmq: bad arguments");
+    if (!w || !x || !xq || !dst || n_tok < 0 || n_tok > 65535) return host::set_error(host::ERR_SHAPE, "mmq: bad arguments");
     if (n_tok == 0) return host::OK;
     const int form = type == T_Q8_0 ? kImgI8 : kImgSplit;
     FNS_TRY(mmq_quant_image(x, ncols, n_tok, form, xq, st));
@@ -1698,7 +1698,8 @@ int mmq_experts(int type, const char *const *table, size_t off, int64_t ncols, i
                                 n_tok * n_used, dst, st);
     }
     FNS_TRY(check_mmq_shape(type, ncols, nrows));
-    if (!x || !xq || n_used < 1 || n_tok < 0) return host::set_error(host::ERR_SHAPE, "mmq_experts: bad arguments");
+    if (!x || !xq || n_used < 1 || n_tok < 0 || n_tok * x_rows_per_tok > 65535)
+        return host::set_error(host::ERR_SHAPE, "mmq_experts: bad arguments");
     if (n_tok == 0) return host::OK;
     // bounds holds n_expert + 1 ints (the reference's MmqIdsScratch sizing); the tile-group prefix of the GEMM goes in
     // the slack that mmq_q8_1_bytes adds after the activation images (4096 bytes >= 257 ints)

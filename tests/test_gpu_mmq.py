@@ -613,6 +613,27 @@ def test_moe_prefill_fused_launch_with_shared_expert_in_place(ops):
     assert np.isfinite(a).all() and rows.size == 0, f"rows {rows[:16].tolist()} of {rows.size} differ"
 
 
+@pytest.mark.parametrize("T,K,aligned", [(8192, 8, True), (65536, 1, True), (65536, 1, False)])
+def test_moe_prefill_guard_largest_call(ops, T, K, aligned):
+    """n_tok * k = 65536 (token, slot) rows with the F16 guard active, the most that the layer takes, at both ends of k and
+    with a router matrix off its 16-byte alignment (the activation image is then a launch of its own): every token
+    equals the same token in a small call, bit for bit."""
+    from flintnsteel_amd import synth
+    H, F, NE = 256, 256, 16
+    base = synth.build_layer(H, F, NE, K, orc.Q4_K, orc.Q6_K, seed=5, layer=80, std=0.5)
+    router = base.router_w
+    if not aligned:
+        router = torch.empty(NE * H + 1, device="cuda")[1:].view(NE, H).copy_(base.router_w)
+    layer = ops.MoeLayer(router, base.slots, orc.Q4_K, orc.Q6_K, H, F, K, guard=True)
+    pre = ops.MoePrefill(layer)
+    x = synth.activations(T, H, seed=5, layer=81) * 40.0
+    ws = pre.workspace(T)
+    out = pre(x, ws=ws)
+    assert (host(pre.trace(ws, T)["escale"]) > 1.0).mean() > 0.5
+    for t in (0, T - 40):
+        assert np.array_equal(host(pre(x[t:t + 40].contiguous())), host(out[t:t + 40])), f"tokens from {t}"
+
+
 # ---- activation images of 2 GiB and more --------------------------------------------------------------------------
 # (a buffer resource reaches 2 GiB: rows in order are read from their group's first, the experts' scattered rows in
 # ranges of tokens; every token equals the same token in a small call, bit for bit)
