@@ -153,14 +153,14 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
         sh_src[i] = a.src ? a.src[q] : q - seg;
         sh_dst[i] = a.dst_rows ? a.dst_rows[q] : q;
     }
-    const uint8_t *wbase = expert_base(a, e);
     const int nb = a.ncols / 256;
     const int64_t row_bytes = (int64_t) nb * BB;
+    const uint8_t *wbase = expert_base(a, e) + wb * WROWS * row_bytes;  // the workgroup's first weight row
     // weight rows past nrows (nrows % WROWS != 0) are computed from the last row and not stored
     const int row0 = wb * WROWS + wave * 32 + jl;
     const int ra = min(row0, a.nrows - 1), rb = GLU ? ra : min(row0 + 128, a.nrows - 1);
     const Rsrc r0 = rsrc_of(wbase + a.off_a), r1 = rsrc_of(wbase + (GLU ? a.off_b : a.off_a)), rx = image_rsrc(a.xpack, a.x_img, a.src, seg);
-    const uint32_t v0 = (uint32_t) (ra * row_bytes), v1 = (uint32_t) (rb * row_bytes);
+    const uint32_t v0 = (uint32_t) ((ra - wb * WROWS) * row_bytes), v1 = (uint32_t) ((rb - wb * WROWS) * row_bytes);
     const uint32_t c0 = v0 + 16 * hh, c1 = v1 + 16 * hh;
     __syncthreads();  // sh_src / sh_dst
 

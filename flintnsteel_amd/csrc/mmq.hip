@@ -448,7 +448,8 @@ template <> struct WFrag<T_IQ2_S> { uint32_t d; uint2 qh, sc; uint4 idx[2], sg[2
 // Buffer loads: a uniform base in a resource (SGPRs), a 32-bit per-lane offset and a uniform offset - no 64-bit
 // address arithmetic per load. (Unaligned dword access is enabled on the platform, as for the plain global loads.)
 // A resource reaches kRsrcBytes from its base (a read past that gives zeros), so one launch's scattered image rows lie
-// within that many bytes (image_tokens), and rows in order are read from their group's first.
+// within that many bytes (image_tokens), image rows in order are read from their group's first and weight rows from the
+// workgroup's first.
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 constexpr int64_t kRsrcBytes = 0x7FFFFFFF;
 __device__ __forceinline__ Rsrc rsrc_of(const void *base) {
@@ -986,14 +987,14 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
         sh_dst[i] = a.dst_rows ? a.dst_rows[q] : q;
     }
 
-    const uint8_t *wbase = expert_base(a, e);
     const int nb = a.ncols / 256;
     const int64_t row_bytes = (int64_t) nb * BB;
+    const uint8_t *wbase = expert_base(a, e) + wb * WROWS * row_bytes;  // the workgroup's first weight row
     // weight rows past nrows (nrows % WROWS != 0) are computed from the last row and not stored
     const int row0 = wb * WROWS + wave * 32 + jl;
     const int ra = min(row0, a.nrows - 1), rb = GLU ? ra : min(row0 + 128, a.nrows - 1);
     const Rsrc r0 = rsrc_of(wbase + a.off_a), r1 = rsrc_of(wbase + (GLU ? a.off_b : a.off_a)), rx = image_rsrc(a.xpack, a.x_img, a.src, seg);
-    const uint32_t v0 = (uint32_t) (ra * row_bytes), v1 = (uint32_t) (rb * row_bytes);
+    const uint32_t v0 = (uint32_t) ((ra - wb * WROWS) * row_bytes), v1 = (uint32_t) ((rb - wb * WROWS) * row_bytes);
     const uint32_t c0 = v0 + 16 * hh, c1 = v1 + 16 * hh;
     __syncthreads();  // sh_src / sh_dst
 

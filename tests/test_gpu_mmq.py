@@ -700,3 +700,20 @@ def test_dense_ffn_act_image_past_2gib(ops):
     for t in (0, T - 64):
         xt = x[t:t + 64].contiguous()
         assert_close(host(out[t:t + 64] - xt), host(ffn(xt, prefill=True) - xt), f"tokens from {t}", 1e-5, 1e-5)
+
+
+@pytest.mark.parametrize("qtype,nrows,block,d_at", [(orc.Q8_0, 248064, 34, 0), (orc.Q6_K, 320000, 210, 208)])
+def test_mmq_weights_past_2gib(ops, qtype, nrows, block, d_at):
+    """A matrix of 2.2 GB (8192 columns; an output head's) in either form: its last rows' results equal those of the same
+    64 rows as a matrix of their own, bit for bit."""
+    ncols, T = 8192, 3
+    row = orc.row_bytes(qtype, ncols)
+    w = torch.randint(0, 256, (nrows * row // block, block), dtype=torch.uint8, device="cuda",
+                      generator=torch.Generator("cuda").manual_seed(1))
+    w[:, d_at:d_at + 2] = torch.tensor([0.001], dtype=torch.float16, device="cuda").view(torch.uint8)
+    w = w.view(nrows, row)
+    x = torch.randn(T, ncols, device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    out = ops.mmq(qtype, w, ncols, nrows, x)
+    for r in (0, nrows - 64):
+        part = host(ops.mmq(qtype, w[r:r + 64], ncols, 64, x))
+        assert np.array_equal(part, host(out[:, r:r + 64])) and np.abs(part).max() > 0.1, f"rows from {r}"
