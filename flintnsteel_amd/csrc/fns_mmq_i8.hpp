@@ -136,17 +136,15 @@ template <int T> __device__ __forceinline__ void grid_to_lds(const MmqI8Lds &L) 
         for (int i = threadIdx.x; i < kGridWords<T> / 4; i += kMmqThreads) ((uint4 *) L.grid)[i] = src[i];
     }
 }
-// Group g, weight row block wb: as mmq_group (4 waves, two 32-row weight streams each, 32 NT activation rows; DEV: an item
-// of the fused launch).
-template <int T, bool GLU, int NT, bool DEV>
-__device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, const MmqI8Lds &L) {
+// Rows seg .. seg + cnt - 1 of expert e, weight row block wb: as mmq_group (4 waves, two 32-row weight streams each, 32 NT
+// activation rows; DEV: an item of the fused launch). LIVE: the rows of a tile whose products are scaled, all 32 or
+// (NT = 1, see mmq_group_i8) as many as the group has; the others are not stored.
+template <int T, bool GLU, int NT, int LIVE, bool DEV>
+__device__ __forceinline__ void mmq_rows_i8(const MmqArgs &a, int slot, int wb, int e, int seg, int cnt, const MmqI8Lds &L) {
     constexpr int ROWS = 32 * NT, WROWS = GLU ? 128 : 256, BB = Traits<T>::bytes;
     constexpr bool MIN = T == T_Q4_K || T == T_Q5_K;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
     const int hh = lane / 32, jl = lane % 32;
-    grid_to_lds<T>(L);
-    int e, seg, cnt;
-    if (!group_rows<NT>(a, g, L.grp, e, seg, cnt)) return;
     int *const sh_src = L.src, *const sh_dst = L.dst;
     for (int i = tid; i < ROWS; i += kMmqThreads) {
         const int q = seg + min(i, cnt - 1);
@@ -210,7 +208,7 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
     if constexpr (DEV && !GLU) {  // the first weights in flight, then the wait for the group's act rows
         i8frag_load<T, 0>(r0, v0, c0, 0, f0);
         i8frag_load<T, 0>(r1, v1, c1, 0, f1);
-        failed = wait_group(a, NT == 2 ? g : a.n_main + g, &L.grp[3]);
+        failed = wait_group(a, slot, &L.grp[3]);
         dma_sb(L.q0, 0, 0);
         store_d(0, load_d(0));
     } else {
@@ -244,7 +242,7 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
     };
     auto load_scales = [&](int sb, int i, float (&d)[16]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < LIVE / 8; ++q) {
             const float4 v = *(const float4 *) &L.d[sb][i / NT][(i % NT) * 32 + 8 * q + 4 * hh];
             d[4 * q] = v.x, d[4 * q + 1] = v.y, d[4 * q + 2] = v.z, d[4 * q + 3] = v.w;
         }
@@ -272,7 +270,7 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
             const v16i i0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur, b0, z, 0, 0, 0);
             const v16i i1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur, b1, z, 0, 0, 0);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
+            for (int q = 0; q < LIVE / 2; ++q) {
                 acc[t][0][q] = fmaf_((float) i0[q], d8[q] * w0, acc[t][0][q]);
                 acc[t][1][q] = fmaf_((float) i1[q], d8[q] * w1, acc[t][1][q]);
             }
@@ -337,10 +335,26 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
             dma_wait();
             __syncthreads();
             if (tid == 0)
-                __hip_atomic_fetch_add(a.gdone + (NT == 2 ? g : a.n_main + g), 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(a.gdone + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+}
+
+// Group g, weight row block wb. The scaling of a tile is what bounds a group, so one of at most 8 or 16 rows leaves out that of
+// the rows it does not have: 1 token to 8 of 128 experts (Q4_K, 2048 / 768) 51.0 -> 40.8 us, 12 tokens through a dense
+// Q4_K block (2048 / 6144) 49.5 -> 40.1; a 37-token block (256 experts, one or two rows each) 135 -> 124. (The same as a
+// branch per 8 rows inside the tile: 24 rows a group 252 -> 266 us; as two copies inside a superblock: Q5_K and IQ spill.)
+template <int T, bool GLU, int NT, bool DEV>
+__device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, const MmqI8Lds &L) {
+    grid_to_lds<T>(L);
+    int e, seg, cnt;
+    if (!group_rows<NT>(a, g, L.grp, e, seg, cnt)) return;
+    const int slot = NT == 2 ? g : a.n_main + g;  // the group's arrival count (fused launch)
+    if constexpr (NT == 1) {
+        if (cnt <= 8) return mmq_rows_i8<T, GLU, 1, 8, DEV>(a, slot, wb, e, seg, cnt, L);
+        if (cnt <= 16) return mmq_rows_i8<T, GLU, 1, 16, DEV>(a, slot, wb, e, seg, cnt, L);
+    }
+    mmq_rows_i8<T, GLU, NT, 32, DEV>(a, slot, wb, e, seg, cnt, L);
 }
 
 // Grid as k_mmq's for the expert lists and the shared expert. Dense: the row blocks go to the XCDs in turn and an XCD

@@ -68,7 +68,7 @@ def test_dense_prefill_int8(ops, qtype, T, H, F):
                                      (orc.IQ3_XXS, orc.IQ3_S), (orc.Q8_0, orc.Q8_0), (orc.Q6_K, orc.Q5_K),
                                      (orc.Q3_K, orc.Q4_K), (orc.Q4_K, orc.Q3_K)])
 @pytest.mark.parametrize("E,counts", [(8, (1, 2, 7, 8, 9)), (8, (32, 33, 40, 64, 72)),
-                                      (256, (1, 2, 7, 8, 9, 32, 33, 40, 64, 72))])
+                                      (256, (1, 2, 7, 8, 9, 32, 33, 40, 64, 72)), (256, (15, 16, 17, 24, 31, 48, 80, 81))])
 def test_prefill_group_sizes(ops, gu, down, E, counts):
     """The prefill layer with experts of exactly these loads (a router that picks each token's expert): one tile, two
     tiles and their remainders, in one launch or two, gate/up and down in either form of the GEMM (8 experts: at most
