@@ -140,7 +140,7 @@ template <int T> __device__ __forceinline__ void grid_to_lds(const MmqI8Lds &L) 
 // activation rows; DEV: an item of the fused launch). LIVE: the rows of a tile whose products are scaled, all 32 or
 // (NT = 1, see mmq_group_i8) as many as the group has; the others are not stored.
 template <int T, bool GLU, int NT, int LIVE, bool DEV>
-__device__ __forceinline__ void mmq_rows_i8(const MmqArgs &a, int slot, int wb, int e, int seg, int cnt, const MmqI8Lds &L) {
+__device__ __forceinline__ void mmq_rows_i8(const MmqArgs &a, int wb, int e, int seg, int cnt, const MmqI8Lds &L) {
     constexpr int ROWS = 32 * NT, WROWS = GLU ? 128 : 256, BB = Traits<T>::bytes;
     constexpr bool MIN = T == T_Q4_K || T == T_Q5_K;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -208,7 +208,7 @@ __device__ __forceinline__ void mmq_rows_i8(const MmqArgs &a, int slot, int wb, 
     if constexpr (DEV && !GLU) {  // the first weights in flight, then the wait for the group's act rows
         i8frag_load<T, 0>(r0, v0, c0, 0, f0);
         i8frag_load<T, 0>(r1, v1, c1, 0, f1);
-        failed = wait_group(a, slot, &L.grp[3]);
+        failed = wait_group(a, a.slot, &L.grp[3]);
         dma_sb(L.q0, 0, 0);
         store_d(0, load_d(0));
     } else {
@@ -335,7 +335,7 @@ __device__ __forceinline__ void mmq_rows_i8(const MmqArgs &a, int slot, int wb, 
             dma_wait();
             __syncthreads();
             if (tid == 0)
-                __hip_atomic_fetch_add(a.gdone + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(a.gdone + a.slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -349,12 +349,11 @@ __device__ __forceinline__ void mmq_group_i8(const MmqArgs &a, int g, int wb, co
     grid_to_lds<T>(L);
     int e, seg, cnt;
     if (!group_rows<NT>(a, g, L.grp, e, seg, cnt)) return;
-    const int slot = NT == 2 ? g : a.n_main + g;  // the group's arrival count (fused launch)
     if constexpr (NT == 1) {
-        if (cnt <= 8) return mmq_rows_i8<T, GLU, 1, 8, DEV>(a, slot, wb, e, seg, cnt, L);
-        if (cnt <= 16) return mmq_rows_i8<T, GLU, 1, 16, DEV>(a, slot, wb, e, seg, cnt, L);
+        if (cnt <= 8) return mmq_rows_i8<T, GLU, 1, 8, DEV>(a, wb, e, seg, cnt, L);
+        if (cnt <= 16) return mmq_rows_i8<T, GLU, 1, 16, DEV>(a, wb, e, seg, cnt, L);
     }
-    mmq_rows_i8<T, GLU, NT, 32, DEV>(a, slot, wb, e, seg, cnt, L);
+    mmq_rows_i8<T, GLU, NT, 32, DEV>(a, wb, e, seg, cnt, L);
 }
 
 // Grid as k_mmq's for the expert lists and the shared expert. Dense: the row blocks go to the XCDs in turn and an XCD
@@ -373,7 +372,7 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
     MmqArgs a;
     int g, wb;
     bool one;
-    if (!mmq_item(m, sh, a, g, wb, one)) return;
+    if (!mmq_item<true>(m, sh, a, g, wb, one)) return;
     if (one) mmq_group_i8<T, GLU, 1, false>(a, g, wb, L);
     else mmq_group_i8<T, GLU, 2, false>(a, g, wb, L);
 }

@@ -390,10 +390,10 @@ struct MmqArgs {
     int64_t x_img;             // bytes per activation image row
     const int32_t *bounds;     // [n_expert + 1] (null: dense)
     const int32_t *gprefix;    // [2][n_expert + 1] group prefixes: 64-row groups, then the <= 32-row remainders
-    int n_main;                // launch: groups of the 64-row list (then the remainder list up to n_groups)
-    int n_groups, n_cb;        // launch: groups in both lists; weight row blocks per group
+    int n_groups, n_cb;        // launch: groups (dense); weight row blocks per group
     const int32_t *src;        // sorted position -> activation image row (null: identity, dense only)
     const int32_t *dst_rows;   // sorted position -> output row (null: identity)
+    int half;                  // item: 0 / 1 = that 32-row half of a 64-row group of the list, -1: the whole group
     int n_rows;                // dense: number of activation rows
     int dense_small;           // dense: 1 = groups of 32 activation rows (one tile), 0 = of 64
     int rows_first;            // dense: 1 = row blocks over the XCDs, all groups of a block in turn; 0 = groups over them
@@ -405,6 +405,7 @@ struct MmqArgs {
     int out_form;              // GLU: the form of the act image rows (kImg*)
     float *act_out;            // GLU: optional f32 act [out row][nrows]
     int *gdone;                // fused launch: per-group arrival counts (zeroed by the compaction kernel)
+    int slot;                  // fused launch: the item's group's count
     int gwait;                 // fused launch: arrivals a down item waits for (its group's gate/up items)
     int spin_limit;            // fused launch: polls before a down item gives up (its outputs are then NaN)
     uint32_t *status;          // fused launch: sticky status word, kStatusTimeout once a wait gave up
@@ -862,18 +863,19 @@ __device__ __forceinline__ bool group_rows(const MmqArgs &a, int g, int (&grp)[4
     // gp[t + 1]); all the prefix loads are independent, one round trip, and the one match publishes through LDS
     e = seg = cnt = 0;
     if (a.bounds) {
-        const int32_t *gp = NT == 2 ? a.gprefix : a.gprefix + a.n_expert + 1;
+        const bool rest = NT == 1 && a.half < 0;  // the list of the <= 32-row remainders
+        const int32_t *gp = rest ? a.gprefix + a.n_expert + 1 : a.gprefix;
         if (g >= gp[a.n_expert]) return false;
         if (tid < a.n_expert) {
             const int g0 = gp[tid], g1 = gp[tid + 1], b0 = a.bounds[tid], b1 = a.bounds[tid + 1];
             if (g0 <= g && g < g1) {
                 int c, sg;
-                if constexpr (NT == 1) {  // the expert's last rows: n_e % 64 of them
+                if (rest) {  // the expert's last rows: n_e % 64 of them
                     c = (b1 - b0) % kMmqTok;
                     sg = b1 - c;
-                } else {
-                    sg = b0 + (g - g0) * kMmqTok;
-                    c = min(kMmqTok, b1 - sg);
+                } else {  // a group, or 32 rows of it
+                    sg = b0 + (g - g0) * kMmqTok + (NT == 1 ? 32 * a.half : 0);
+                    c = min(32 * NT, b1 - sg);
                 }
                 grp[0] = tid;
                 grp[1] = sg;
@@ -1036,7 +1038,7 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
     if constexpr (DEV && !GLU) {  // the first weights in flight, then the wait for the group's act rows
         wfrag_load<T, 0>(r0, v0, c0, 0, f0);
         wfrag_load<T, 0>(r1, v1, c1, 0, f1);
-        failed = wait_group(a, NT == 2 ? g : a.n_main + g, &L.grp[3]);
+        failed = wait_group(a, a.slot, &L.grp[3]);
         dma_chunk(sh_a0, 0, 0);
         dma_sums(0);
     } else {
@@ -1253,8 +1255,7 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
             dma_wait();
             __syncthreads();
             if (tid == 0)
-                __hip_atomic_fetch_add(a.gdone + (NT == 2 ? g : a.n_main + g), 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(a.gdone + a.slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     MMQ_MARK(12);
@@ -1267,12 +1268,46 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
 // row block; groups go to the XCDs in turn (group u on XCD u % 8) in increasing order.
 // (SPX mode: one partition of all 8 XCDs. In a partitioned mode the mapping is a performance assumption only.)
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
+// A launch of the int8 form whose items leave CUs idle runs its 64-row groups as two items of 32 rows: its time is that of
+// one item, which is half, for the same sums (200 tokens to 4 of 16 experts, Q4_K, 2048 / 768: 81 -> 64 us, where the
+// split form takes 70). The rule: at most one item per CU, the groups counted as halves and the shared expert's too.
+constexpr int kHalvesMax = 256;
+__host__ __device__ constexpr int xcd_items(int groups, int n_cb) { return n_cb * kXcds * ((groups + kXcds - 1) / kXcds); }
+__host__ __device__ constexpr int groups32(int rows) { return (rows + 31) / 32; }
+
+// Item j of the two lists (nm 64-row groups, then the remainders): its group g, half, and whether it is one token tile.
+__device__ __forceinline__ void list_item(int j, int nm, bool halves, int &g, int &half, bool &one) {
+    half = -1;
+    one = true;
+    if (halves && j < 2 * nm) {
+        g = j >> 1;
+        half = j & 1;
+    } else {
+        g = halves ? j - nm : j;
+        one = g >= nm;
+        if (one) g -= nm;
+    }
+}
+
 // Workgroup -> its arguments, group g, weight row block wb and whether the group is one token tile (at most 32 rows);
-// false: nothing to do.
+// false: nothing to do. I8: a launch of the int8 form.
+template <bool I8>
 __device__ __forceinline__ bool mmq_item(const MmqArgs &m, const MmqShared &sh, MmqArgs &a, int &g, int &wb, bool &one) {
     a = m;
-    const bool shared = (int) blockIdx.x < sh.items;
-    const int lid = shared ? (int) blockIdx.x : (int) blockIdx.x - sh.items, r = lid / kXcds;
+    a.half = -1;
+    int nm = 0, nr = 0, sh_items = sh.items;
+    bool halves = false;
+    if (m.bounds) {
+        // expert path: the groups that exist in this call (the device-side counts of the 64-row list and of the
+        // remainder list) take the first workgroups; the rest of the grid (sized for the upper bound) returns at once
+        nm = m.gprefix[m.n_expert], nr = m.gprefix[2 * (m.n_expert + 1) - 1];
+        if constexpr (I8) {
+            halves = (2 * nm + nr) * m.n_cb + groups32(sh.n_rows) * sh.n_cb <= kHalvesMax;
+            if (halves) sh_items = xcd_items(groups32(sh.n_rows), sh.n_cb);
+        }
+    }
+    const bool shared = (int) blockIdx.x < sh_items;
+    const int lid = shared ? (int) blockIdx.x : (int) blockIdx.x - sh_items, r = lid / kXcds;
     const int n_cb = shared ? sh.n_cb : m.n_cb;
     const int j = (r / n_cb) * kXcds + lid % kXcds, wbj = r % n_cb;
     one = false;
@@ -1294,16 +1329,16 @@ __device__ __forceinline__ bool mmq_item(const MmqArgs &m, const MmqShared &sh, 
         a.out_img = sh.out_img;
         a.out_form = sh.out_form;
         a.act_out = nullptr;
+        if (halves) {
+            one = true;
+            return 32 * j < sh.n_rows;
+        }
         if (kMmqTok * j >= sh.n_rows) return false;
         one = sh.n_rows - kMmqTok * j <= kMmqTok / 2;
         if (one) g = 2 * j;
     } else if (m.bounds) {
-        // expert path: the groups that exist in this call (the device-side counts of the 64-row list and of the
-        // remainder list) take the first workgroups; the rest of the grid (sized for the upper bound) returns at once
-        const int nm = m.gprefix[m.n_expert], nr = m.gprefix[2 * (m.n_expert + 1) - 1];
-        if (j >= nm + nr) return false;
-        one = j >= nm;
-        if (one) g = j - nm;
+        if (j >= (halves ? 2 * nm : nm) + nr) return false;
+        list_item(j, nm, halves, g, a.half, one);
     } else {
         if (m.rows_first) {
             wb = (r / m.n_groups) * kXcds + lid % kXcds;
@@ -1329,7 +1364,7 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
     MmqArgs a;
     int g, wb;
     bool one;
-    if (!mmq_item(m, sh, a, g, wb, one)) return;
+    if (!mmq_item<false>(m, sh, a, g, wb, one)) return;
     if (one) mmq_group<T, GLU, 1, false>(a, g, wb, L);
     else mmq_group<T, GLU, 2, false>(a, g, wb, L);
 }
@@ -1377,34 +1412,37 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
     // remainders) are numbered j = 0 .. R - 1 and take the first workgroups of the grid; the workgroups past them (the
     // grid is sized for the upper bound) return at once, after every real item has been dispatched.
     const int nm = m.gprefix[m.n_expert], nr = m.gprefix[2 * (m.n_expert + 1) - 1];
-    const int R = nm + nr, rounds = (R + kXcds - 1) / kXcds;
-    const int items_gu = m.n_cb_gu * kXcds * rounds;  // a multiple of kXcds
-    const bool is_gu = (int) blockIdx.x < items_gu;
+    const bool halves_gu = GU8 && (2 * nm + nr) * m.n_cb_gu <= kHalvesMax, halves_dn = DN8 && (2 * nm + nr) * m.n_cb_dn <= kHalvesMax;
+    const int items_gu = xcd_items((halves_gu ? 2 * nm : nm) + nr, m.n_cb_gu);  // a multiple of kXcds
+    const bool is_gu = (int) blockIdx.x < items_gu, halves = is_gu ? halves_gu : halves_dn;
     const int cb = is_gu ? m.n_cb_gu : m.n_cb_dn;
     const int lid = is_gu ? (int) blockIdx.x : (int) blockIdx.x - items_gu, r = lid / kXcds;
     const int j = (r / cb) * kXcds + lid % kXcds, wb = r % cb;
-    if (j >= R) return;
-    const int g = j < nm ? j : m.n_main + (j - nm);
+    if (j >= (halves ? 2 * nm : nm) + nr) return;
     MmqArgs a{};
+    int g;
+    bool one;
+    list_item(j, nm, halves, g, a.half, one);
+    const bool rest = one && a.half < 0;
+    a.slot = rest ? m.n_main + g : g;
     auto run = [&](auto glu) __attribute__((always_inline)) {
         constexpr bool GLU = decltype(glu)::value;
         constexpr int T = GLU ? TGU : TDN;
         if constexpr (GLU ? GU8 : DN8) {
             const MmqI8Lds L{(uint8_t (&)[kI8Buf]) sh_a0, (uint8_t (&)[kI8Buf]) sh_a1, (float (&)[2][8][kMmqTok]) sh_d, sh_s,
                              sh_src, sh_dst, sh_grp, nullptr};
-            if (g < m.n_main) mmq_group_i8<T, GLU, 2, true>(a, g, wb, L);
-            else mmq_group_i8<T, GLU, 1, true>(a, g - m.n_main, wb, L);
+            if (one) mmq_group_i8<T, GLU, 1, true>(a, g, wb, L);
+            else mmq_group_i8<T, GLU, 2, true>(a, g, wb, L);
         } else {
             const MmqLds L{(uint8_t (&)[kSplitBuf]) sh_a0, (uint8_t (&)[kSplitBuf]) sh_a1, sh_s[0], sh_src, sh_dst, sh_grp, nullptr};
-            if (g < m.n_main) mmq_group<T, GLU, 2, true>(a, g, wb, L);
-            else mmq_group<T, GLU, 1, true>(a, g - m.n_main, wb, L);
+            if (one) mmq_group<T, GLU, 1, true>(a, g, wb, L);
+            else mmq_group<T, GLU, 2, true>(a, g, wb, L);
         }
     };
     a.table = m.table;
     a.n_expert = m.n_expert;
     a.bounds = m.bounds;
     a.gprefix = m.gprefix;
-    a.n_main = m.n_main;
     a.dst_rows = m.dstr;
     a.gdone = m.gdone;
     if (is_gu) {
@@ -1427,7 +1465,7 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
         a.x_img = m.a_img;
         a.src = m.dstr;
         a.dst = m.dexp;
-        a.gwait = m.gwait;
+        a.gwait = m.gwait + (halves_gu && !rest ? m.n_cb_gu : 0);  // both halves of a group arrive at its count
         a.spin_limit = m.spin_limit;
         a.status = m.status;
         run(std::false_type{});
@@ -1452,6 +1490,9 @@ const void *mmq_kernel(int type, bool glu) {
     return nullptr;
 }
 
+// the most items that n_cb row blocks of halves take, where 64-row groups and remainders are at most total
+int64_t halves_items(int total, int n_cb) { return xcd_items(std::min(2 * total, kHalvesMax / n_cb), n_cb); }
+
 // groups: upper bound of the 64-row list; expert path: of the 64-row list and the <= 32-row remainders together (the
 // workgroups past the device-side counts return at once)
 // sh: a dense matrix of the same type whose groups come first in the grid (expert path only); form: of the activations
@@ -1461,7 +1502,6 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
     if (!fn) return host::set_error(host::ERR_TYPE, "mmq: type %d not supported", type);
     if (groups <= 0) return host::OK;
     MmqArgs arg = a;
-    arg.n_main = groups;
     // expert path: n_expert + ceil(pairs / 64) (the 64-row list's bound) bounds both lists together, as expert e
     // has ceil(n_e / 64) groups in all
     int total = groups;
@@ -1472,8 +1512,7 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
     if (sh && a.bounds) {
         shared = *sh;
         shared.n_cb = (sh->nrows + rows - 1) / rows;
-        const int sg = (sh->n_rows + kMmqTok - 1) / kMmqTok;
-        sh_items = (int64_t) shared.n_cb * kXcds * ((sg + kXcds - 1) / kXcds);
+        sh_items = xcd_items((sh->n_rows + kMmqTok - 1) / kMmqTok, shared.n_cb);
     }
     arg.n_cb = (a.nrows + rows - 1) / rows;
     // dense: when even twice the workgroups of the 64-row groups fit one per CU, groups of 32 rows (one token tile:
@@ -1489,8 +1528,11 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
     }
     arg.n_groups = total;
     arg.rows_first = form != kImgSplit && !a.bounds && (arg.n_cb % kXcds == 0 || arg.n_cb >= 4 * kXcds);
-    const int64_t items = sh_items + (arg.rows_first ? (int64_t) total * kXcds * ((arg.n_cb + kXcds - 1) / kXcds)
-                                                     : (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds));
+    int64_t items = sh_items + (arg.rows_first ? (int64_t) total * kXcds * ((arg.n_cb + kXcds - 1) / kXcds)
+                                               : (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds));
+    const int sh32 = groups32(shared.n_rows);
+    if (form == kImgI8 && a.bounds && sh32 * shared.n_cb <= kHalvesMax)  // room for the halves
+        items = std::max<int64_t>(items, xcd_items(sh32, shared.n_cb) + halves_items(total, arg.n_cb));
     if (items > INT32_MAX) return host::set_error(host::ERR_SHAPE, "mmq: grid too large");
     shared.items = (int) sh_items;
     const hipError_t e = hipLaunchKernel(fn, dim3((unsigned) items, (unsigned) ks), dim3(kMmqThreads), args, 0, st);
@@ -1521,8 +1563,12 @@ int launch_mmq_moe(int tgu, int tdn, int x_form, int act_form, MoeArgs m, hipStr
     m.n_cb_dn = (m.hidden + 255) / 256;
     m.gwait += m.n_cb_gu;
     // n_main = n_expert + ceil(pairs / 64) bounds both lists together: expert e has ceil(n_e / 64) groups in all
-    const int64_t total = m.n_main;
-    const int64_t items = (int64_t) (m.n_cb_gu + m.n_cb_dn) * kXcds * ((total + kXcds - 1) / kXcds);
+    const int total = m.n_main;
+    auto part = [&](int n_cb, bool i8) {
+        const int64_t whole = (int64_t) n_cb * kXcds * ((total + kXcds - 1) / kXcds);
+        return i8 ? std::max(whole, halves_items(total, n_cb)) : whole;
+    };
+    const int64_t items = part(m.n_cb_gu, x_form == kImgI8) + part(m.n_cb_dn, act_form == kImgI8);
     if (items > INT32_MAX) return host::set_error(host::ERR_SHAPE, "mmq: grid too large");
     void *args[] = {&m};
     const hipError_t e = hipLaunchKernel(fn, dim3((unsigned) items), dim3(kMmqThreads), args, 0, st);
