@@ -64,6 +64,7 @@ SIGNATURES: dict[str, list] = {
     "fns_hip_mmq_compact": [_P, _I64, _I64, _I64, _I64, _P, _P, _P, _P],
     "fns_hip_moe_prefill_workspace": [_P, _I64, _P, _P],
     "fns_hip_moe_prefill_section": [_P, _I64, _I, _P, _P],
+    "fns_hip_moe_prefill_image": [_P, _I, _P, _P],
     "fns_hip_moe_prefill": [_P, _P, _P, _P, _I64, _P, _SZ, _P],
     "fns_hip_moe_prefill_status": [_P, _I64, _P, _I, _P, _P],
     "fns_hip_moe_prefill_status_collect": [_P, _I64, _P, _P, _P],

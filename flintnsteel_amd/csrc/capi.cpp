@@ -231,6 +231,10 @@ int fns_hip_dense_ffn_prefill(const FnsDenseFfn *ffn, const float *x, float *out
     return impl::dense_ffn(ffn, x, out, n_tok, workspace, workspace_bytes, true, S(stream));
 }
 
+int fns_hip_moe_prefill_image(const FnsMoeLayer *layer, int section, int *form, size_t *row_stride) {
+    return impl::moe_prefill_image(layer, section, form, row_stride);
+}
+
 int fns_hip_moe_prefill_status(const FnsMoeLayer *layer, int64_t n_tok, void *workspace, int clear, uint32_t *status,
                                void *stream) {
     return impl::moe_prefill_status(layer, n_tok, workspace, clear, status, S(stream));

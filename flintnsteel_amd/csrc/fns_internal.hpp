@@ -95,6 +95,7 @@ int moe_layer_status(const FnsMoeLayer *L, int n_tok, void *ws, int clear, uint3
 int moe_layer_status_collect(const FnsMoeLayer *L, int n_tok, void *ws, uint32_t *dst, hipStream_t st);
 int status_collect(uint32_t *word, uint32_t *dst, hipStream_t st);
 int moe_prefill_workspace(const FnsMoeLayer *L, int64_t n_tok, size_t *offsets, size_t *total);
+int moe_prefill_image(const FnsMoeLayer *L, int section, int *form, size_t *row_stride);
 int moe_prefill_section(const FnsMoeLayer *L, int64_t n_tok, int section, size_t *offset, size_t *bytes);
 int moe_prefill_status(const FnsMoeLayer *L, int64_t n_tok, void *ws, int clear, uint32_t *status, hipStream_t st);
 int moe_prefill_status_collect(const FnsMoeLayer *L, int64_t n_tok, void *ws, uint32_t *dst, hipStream_t st);

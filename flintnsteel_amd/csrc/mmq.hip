@@ -7,8 +7,8 @@
 //
 //   * Two forms of the GEMM. Types whose scales change every 32 columns (Q4_K, Q5_K, Q8_0, IQ4_XS, IQ3_XXS, IQ3_S) run on
 //     int8 MFMA, one exact integer dot per sub-block and a convert + scale + fma per output (fns_mmq_i8.hpp). The others
-//     (Q6_K and Q3_K scale every 16 columns, IQ2_S every 16), and calls of at most 256 gate/up workgroups, run the split
-//     form of this file, to which the points below apply:
+//     (Q6_K and Q3_K scale every 16 columns, IQ2_S every 16) run the split form of this file, to which the points below
+//     apply:
 //   * In the split form the scales are folded into the operands instead, exactly: A = q8 * d8 as two f16 halves (hi + lo, see the image
 //     layout below), B = integer code * integer sub-block scale as f16 (|B| <= 2048: exact; Q6_K's 8-bit scales are
 //     split in two operands). v_mfma_f32_32x32x16_f16 then accumulates a whole 256-column superblock, and only the
@@ -1473,8 +1473,8 @@ __global__ __launch_bounds__(kMmqThreads) __attribute__((amdgpu_waves_per_eu(2, 
     PF_MARK(3, 1);
 }
 
-// the split form: mmq and mmq_experts over the caller's split image (Q8_0 takes the int8 form there), the types without an
-// int8 form, and calls of few workgroups
+// the split form: the types without an int8 form, mmq and mmq_experts over the caller's split image (Q8_0 takes the int8
+// form there), and gate/up beside a shared expert that reads the split image of x
 const void *mmq_kernel(int type, bool glu) {
     switch (type) {
         case T_Q3_K: return glu ? (const void *) k_mmq<T_Q3_K, true> : (const void *) k_mmq<T_Q3_K, false>;
@@ -1485,7 +1485,7 @@ const void *mmq_kernel(int type, bool glu) {
         case T_IQ4_XS: return glu ? (const void *) k_mmq<T_IQ4_XS, true> : (const void *) k_mmq<T_IQ4_XS, false>;
         case T_IQ3_XXS: return glu ? (const void *) k_mmq<T_IQ3_XXS, true> : (const void *) k_mmq<T_IQ3_XXS, false>;
         case T_IQ3_S: return glu ? (const void *) k_mmq<T_IQ3_S, true> : (const void *) k_mmq<T_IQ3_S, false>;
-        case T_Q8_0: return glu ? (const void *) k_mmq<T_Q8_0, true> : (const void *) k_mmq<T_Q8_0, false>;
+        case T_Q8_0: return glu ? (const void *) k_mmq<T_Q8_0, true> : nullptr;
     }
     return nullptr;
 }
@@ -1543,9 +1543,7 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
 // The fused kernel of a pair of {Q3_K, Q4_K} and the forms of the x and act images; the other pairs take two launches (the
 // Q5_K and Q6_K decoders push the combined kernel past 256 registers).
 template <int TGU, bool GU8> const void *mmq_moe_kernel_dn(int tdn, int act_form) {
-    if (tdn == T_Q4_K)
-        return act_form == kImgI8 ? (const void *) k_mmq_moe<TGU, GU8, T_Q4_K, true>
-                                  : (const void *) k_mmq_moe<TGU, GU8, T_Q4_K, false>;
+    if (tdn == T_Q4_K) return act_form == kImgI8 ? (const void *) k_mmq_moe<TGU, GU8, T_Q4_K, true> : nullptr;
     return tdn == T_Q3_K && act_form == kImgSplit ? (const void *) k_mmq_moe<TGU, GU8, T_Q3_K, false> : nullptr;
 }
 const void *mmq_moe_kernel(int tgu, int tdn, int x_form, int act_form) {
@@ -1944,9 +1942,29 @@ int moe_prefill_status_collect(const FnsMoeLayer *L, int64_t n_tok, void *ws, ui
     return status_collect((uint32_t *) ((uint8_t *) ws + off) + words, dst, st);
 }
 
-// Whether a call's gate/up GEMM has at most 256 workgroups (its images are then in the split form).
-static bool moe_prefill_few(const FnsMoeLayer *L, int64_t n_tok) {
-    return std::min<int64_t>(L->n_expert, n_tok * L->k) * ((L->inter + 127) / 128) <= 256;
+// The forms of a layer's activation images: int8 where every matrix that reads the image has the int8 form (x: the routed
+// and the shared gate/up). They follow from the types alone, so a token's result has the same bits in a call of any
+// length. (In calls whose items leave CUs idle the split form was the faster one for Q4_K and Q5_K, 70 against 81 us for
+// 200 tokens to 4 of 16 experts; the int8 form's halves and its groups of few rows made up for that: 64.)
+namespace {
+struct PrefillForms { int x, act, sh; };
+PrefillForms prefill_forms(const FnsMoeLayer *L) {
+    const bool has_sh = L->shexp_inter > 0;
+    const int sgt = has_sh && L->shexp_gu_type ? L->shexp_gu_type : L->gu_type;
+    const int sdt = has_sh && L->shexp_down_type ? L->shexp_down_type : L->down_type;
+    return {std::min(mmq_form(L->gu_type), mmq_form(sgt)), mmq_form(L->down_type), mmq_form(sdt)};
+}
+}  // namespace
+
+int moe_prefill_image(const FnsMoeLayer *L, int section, int *form, size_t *row_stride) {
+    if (!L || !form || !row_stride) return host::set_error(host::ERR_SHAPE, "moe_prefill_image: null argument");
+    const PrefillForms f = prefill_forms(L);
+    switch (section) {
+        case 3: *form = f.x, *row_stride = mmq_form_bytes(f.x, L->hidden); return host::OK;
+        case 4: *form = f.act, *row_stride = (size_t) act_stride(L->inter, f.act); return host::OK;
+        case 13: *form = f.sh, *row_stride = mmq_form_bytes(f.sh, L->shexp_inter); return host::OK;
+    }
+    return host::set_error(host::ERR_SHAPE, "moe_prefill_image: section %d holds no image", section);
 }
 
 int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, float *out, int64_t n_tok, void *ws,
@@ -1975,17 +1993,11 @@ int moe_prefill(const FnsMoeLayer *L, const float *x, const float *x_resid, floa
     const int64_t P = n_tok * L->k;
     const char *const *table = (const char *const *) L->table;
 
-    // The forms of the activation images: int8 where every matrix that reads the image has the int8 form (x: the routed
-    // and the shared gate/up).
     const bool has_sh = L->shexp_inter > 0;
     const int sgt = has_sh && L->shexp_gu_type ? L->shexp_gu_type : L->gu_type;
     const int sdt = has_sh && L->shexp_down_type ? L->shexp_down_type : L->down_type;
-    // A call whose gate/up items (at most min(n_expert, pairs) groups of few rows) do not fill the GPU is bound by one
-    // workgroup's latency, where the split form's MFMAs are shorter than the int8 form's scaling (6 tokens to 4 of 32
-    // experts, 1024 -> 512: 41.7 against 43.9 us; 37 tokens to 6 of 256, 888 items: 144 against 140).
-    const bool few = moe_prefill_few(L, n_tok);
-    const int x_form = few ? kImgSplit : std::min(mmq_form(L->gu_type), mmq_form(sgt));
-    const int act_form = few ? kImgSplit : mmq_form(L->down_type), sh_form = few ? kImgSplit : mmq_form(sdt);
+    const PrefillForms forms = prefill_forms(L);
+    const int x_form = forms.x, act_form = forms.act, sh_form = forms.sh;
     const int64_t x_img = (int64_t) mmq_form_bytes(x_form, L->hidden);
 
     // RMSNorm first when the layer has one: the router and the experts read h (reference src/engine.cu:331)

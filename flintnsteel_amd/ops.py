@@ -391,14 +391,10 @@ class MoeLayer:
 PREFILL_SECTIONS = ("logits", "ids", "w", "xpack", "apack", "dexp")
 
 
-# Types whose activations the prefill GEMM reads as int8 image rows (per 256 columns 320 bytes: int8 codes, 8 f32 block
-# scales, 32 bytes of scaled sums) in calls of more than 256 gate/up workgroups; the others read split image rows (1056).
-I8_TYPES = (Q8_0, Q4_K, Q5_K, IQ4_XS, IQ3_XXS, IQ3_S)
-
-
 def _split_of_i8(rows: torch.Tensor, ncols: int) -> torch.Tensor:
     """The split image rows (uint8 [n][ncols / 256 * 1056]: every code times its scale as two f16 halves, then the sums)
-    that int8 image rows define: the same codes, scales and sums."""
+    that int8 image rows (per 256 columns 320 bytes: int8 codes, 8 f32 block scales, 32 bytes of scaled sums) define: the
+    same codes, scales and sums."""
     n, nb = rows.shape[0], ncols // 256
     sb = rows[:, : nb * 320].contiguous().view(n, nb, 320)
     q = sb[:, :, :256].contiguous().view(torch.int8).float().view(n, nb, 8, 32)
@@ -468,16 +464,12 @@ class MoePrefill:
             off, n = self.section(n_tok, idx)
             if n:
                 out[name] = ws[off: off + n].view(dt).view(*shape)
-        # (act rows are padded to whole cache lines)
-        many = min(d.n_expert, P) * ((d.inter + 127) // 128) > 256
-        x_i8 = d.gu_type in I8_TYPES and (not d.shexp_inter or (d.shexp_gu_type or d.gu_type) in I8_TYPES)
-        for name, i8, ncols, pad in (("xpack", many and x_i8, d.hidden, 1),
-                                     ("apack", many and d.down_type in I8_TYPES, d.inter, 128)):
-            if i8:
-                stride, n = (ncols // 256 * 320 + pad - 1) // pad * pad, out[name].shape[0]
-                out[name] = _split_of_i8(out[name].reshape(-1)[: n * stride].view(n, stride), ncols)
-            else:
-                out[name] = out[name][:, : ncols // 256 * 1056]
+        form, stride = ctypes.c_int(), ctypes.c_size_t()
+        for name, idx, ncols in (("xpack", 3, d.hidden), ("apack", 4, d.inter)):
+            call("fns_hip_moe_prefill_image", ctypes.byref(d), idx, ctypes.byref(form), ctypes.byref(stride))
+            n = out[name].shape[0]
+            rows = out[name].reshape(-1)[: n * stride.value].view(n, stride.value)
+            out[name] = _split_of_i8(rows, ncols) if form.value else rows[:, : ncols // 256 * 1056]
         return out
 
 

@@ -245,6 +245,9 @@ int fns_hip_moe_prefill_workspace(const FnsMoeLayer *layer, int64_t n_tok, size_
  * 11 RMSNorm output, 12 its Q8_1 blocks, 13 shared-expert act images, 14 shared-expert output). Inspection and tests;
  * the image layouts are internal. */
 int fns_hip_moe_prefill_section(const FnsMoeLayer *layer, int64_t n_tok, int section, size_t *offset, size_t *bytes);
+/* The form (0: split, 1: int8) and the row stride in bytes of the images in section 3, 4 or 13. They follow from the
+ * layer's types alone: a token's result has the same bits in a call of any length. */
+int fns_hip_moe_prefill_image(const FnsMoeLayer *layer, int section, int *form, size_t *row_stride);
 int fns_hip_moe_prefill(const FnsMoeLayer *layer, const float *x, const float *x_resid, float *out, int64_t n_tok,
                         void *workspace, size_t workspace_bytes, void *stream);
 /* No counterpart in the reference. Without the F16 guard and for gate/up and down types from {Q3_K, Q4_K}, gate/up

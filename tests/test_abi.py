@@ -39,6 +39,30 @@ def _buf():
     return ctypes.c_void_p(0x1000)  # never dereferenced: validation fails first
 
 
+def test_prefill_image_forms():
+    """The forms of a prefill layer's activation images follow from its types: int8 (320 bytes per 256 columns) where every
+    matrix that reads the image has the int8 form of the GEMM, otherwise split (1056); act rows are whole 128-byte lines."""
+    from flintnsteel_amd.ops import MoeLayerDesc
+    form, stride = ctypes.c_int(), ctypes.c_size_t()
+
+    def image(section, **kw):
+        d = MoeLayerDesc(hidden=1024, inter=768, n_expert=16, k=4, **kw)
+        _lib.call("fns_hip_moe_prefill_image", ctypes.byref(d), section, ctypes.byref(form), ctypes.byref(stride))
+        return form.value, stride.value
+
+    q8_0, q3_k, q4_k, q6_k, iq2_s, iq4_xs = 8, 11, 12, 14, 22, 23
+    assert image(3, gu_type=q4_k, down_type=q6_k) == (1, 1280)
+    assert image(4, gu_type=q4_k, down_type=q6_k) == (0, 3200)      # 3168 to whole lines
+    assert image(3, gu_type=q3_k, down_type=iq4_xs) == (0, 4224)
+    assert image(4, gu_type=iq2_s, down_type=iq4_xs) == (1, 1024)   # 960 to whole lines
+    sh = {"shexp_inter": 512, "gu_type": q4_k, "down_type": q8_0}
+    assert image(3, **sh) == (1, 1280) and image(13, **sh) == (1, 640)
+    assert image(3, shexp_gu_type=q6_k, **sh) == (0, 4224)           # the shared gate/up reads x too
+    assert image(13, shexp_down_type=q6_k, **sh) == (0, 2112)
+    with pytest.raises(_lib.FnsError, match="no image"):
+        image(5, gu_type=q4_k, down_type=q4_k)
+
+
 def test_unsupported_type_is_rejected():
     L = _lib.lib()
     rc = L.fns_hip_mmvq(10, _buf(), 2048, 16, _buf(), _buf(), 1, None)  # Q2_K: not accepted

@@ -111,6 +111,37 @@ def test_prefill_group_sizes(ops, gu, down, E, counts):
     assert np.concatenate(tight).mean() >= 0.8
 
 
+@pytest.mark.parametrize("gu,down,guard,shared", [
+    (orc.Q4_K, orc.Q4_K, False, None), (orc.Q4_K, orc.Q3_K, False, None), (orc.Q3_K, orc.Q4_K, False, None),
+    (orc.Q4_K, orc.Q5_K, False, None), (orc.Q5_K, orc.Q6_K, True, None), (orc.IQ3_XXS, orc.IQ4_XS, False, None),
+    (orc.IQ3_S, orc.IQ4_XS, True, (orc.IQ3_S, orc.IQ4_XS)), (orc.Q8_0, orc.Q8_0, False, (orc.Q8_0, orc.Q8_0)),
+    (orc.Q4_K, orc.Q4_K, False, (orc.Q6_K, orc.Q4_K)), (orc.Q4_K, orc.Q5_K, False, (orc.Q4_K, orc.Q5_K))])
+def test_prefill_token_alone_and_in_a_chunk(ops, gu, down, guard, shared):
+    """A token's result does not depend on the call's length: 1000 tokens (64-row groups), their first 150 (64-row groups as
+    two items where that fills no more than the GPU), 33 of them and single tokens give the same bits, for every type of
+    the int8 form, one launch and two, each pair of image forms, and a shared expert of the routed types or others."""
+    E, K, H, F, T = 16, 4, 1024, 768, 1000
+    rng = np.random.default_rng(gu * 100 + down)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    mats = [np.stack([weights(t, r, c, 10 * k + e % 4).reshape(-1) for e in range(E)])
+            for k, (t, r, c) in enumerate([(gu, F, H), (gu, F, H), (down, H, F)])]
+    slots = ops.ExpertSlots.from_tensors(*(torch.from_numpy(m) for m in mats))
+    shexp = None
+    if shared:
+        g, d = shared
+        shexp = {"gate": dev(weights(g, 512, H, 91)), "up": dev(weights(g, 512, H, 92)), "down": dev(weights(d, H, 512, 93)),
+                 "inter": 512, "gu_type": g, "down_type": d}
+    layer = ops.MoeLayer(dev(gaussian(rng, (E, H), 0.05)), slots, gu, down, H, F, K, guard=guard, shexp=shexp,
+                         ffn_norm=dev(gaussian(rng, (H,), 1.0)))
+    pre = ops.MoePrefill(layer)
+    x = dev(gaussian(rng, (T, H)))
+    whole = pre(x).cpu().numpy()
+    assert np.isfinite(whole).all() and np.abs(whole).max() > 0
+    for t0, n in ((0, 150), (400, 33), (0, 1), (T - 1, 1)):
+        part = pre(x[t0:t0 + n].contiguous()).cpu().numpy()
+        assert np.array_equal(part, whole[t0:t0 + n]), f"{n} tokens from {t0}"
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("H,E,T", [(256, 256, 993), (576 * 4, 250, 1025), (512, 33, 4097)])
 def test_prefill_router_tiles(ops, bf16, H, E, T):
