@@ -499,6 +499,26 @@ def test_moe_prefill_guard_bf16_sigmoid_residual(ops):
                          "guarded bf16 sigmoid prefill", resid=host(resid))
 
 
+@pytest.mark.parametrize("gu,dn,T", [(orc.Q4_K, orc.Q5_K, 33), (orc.Q5_K, orc.Q4_K, 77)])
+def test_moe_prefill_guard_int8_images(ops, gu, dn, T):
+    """The F16 guard active on int8 act images (rows divided in place and their images made again): the images against the
+    oracle's Q8_1 of the divided rows, byte for byte, and the layer against the float64 chains."""
+    from flintnsteel_amd import synth
+    H, F, NE, K = 512, 512, 32, 6
+    base = synth.build_layer(H, F, NE, K, gu, dn, seed=6, layer=82, std=0.5)
+    layer = ops.MoeLayer(base.router_w, base.slots, gu, dn, H, F, K, guard=True)
+    pre = ops.MoePrefill(layer)
+    x = synth.activations(T, H, seed=6, layer=83) * 40.0
+    ws = pre.workspace(T)
+    out = host(pre(x, ws=ws))
+    tr = {k: host(v) for k, v in pre.trace(ws, T).items()}
+    assert (tr["escale"] > 1.0).any()
+    assert np.array_equal(tr["apack"], split_image(orc.quantize_q8_1(tr["act"]), F)), "act image"
+    slots = {k: base.slots.view(k).cpu().numpy() for k in ("gate", "up", "down")}
+    tr["out"] = out
+    check_prefill_chains(tr, layer, slots, host(x), list(range(0, T, 3)), tr["ids"], gu, dn, H, F, "guard, int8 images")
+
+
 def test_moe_prefill_unaligned_inputs_take_the_two_launch_router(ops):
     """x 4 bytes off a 16-byte boundary: the prefill takes the separate router GEMM (guarded loads) and activation
     quantiser instead of the one-launch router + image kernel. Same chunk order, products and Q8_1 arithmetic, so the

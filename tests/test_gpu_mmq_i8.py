@@ -42,8 +42,13 @@ def dequant(qtype: int, w: np.ndarray, nrows: int, ncols: int) -> np.ndarray:
     return np.asarray(orc.dequantize(qtype, w.reshape(nrows, -1), ncols), np.float64).reshape(nrows, ncols)
 
 
-@pytest.mark.parametrize("T,H,F", [(1, 512, 768), (33, 512, 768), (65, 512, 768), (130, 2048, 1024)])
-@pytest.mark.parametrize("qtype", TYPES)
+# (T <= 130: every launch takes groups of 32 rows, 1 to 5 of them. 449: 64-row groups, the last of one row; gate/up with 34
+# weight row blocks over the XCDs, not a multiple of 8; down with its columns split in four.)
+SHAPES = [(1, 512, 768), (33, 512, 768), (65, 512, 768), (130, 2048, 1024)]
+
+
+@pytest.mark.parametrize("qtype,T,H,F", [(t, *s) for t in TYPES for s in SHAPES] +
+                         [(t, 449, 2048, 4352) for t in (orc.Q8_0, orc.Q4_K, orc.IQ4_XS)])
 def test_dense_prefill_int8(ops, qtype, T, H, F):
     rng = np.random.default_rng(T + H)
     g, u, d = weights(qtype, F, H, 1), weights(qtype, F, H, 2), weights(qtype, H, F, 3)
@@ -140,6 +145,28 @@ def test_prefill_token_alone_and_in_a_chunk(ops, gu, down, guard, shared):
     for t0, n in ((0, 150), (400, 33), (0, 1), (T - 1, 1)):
         part = pre(x[t0:t0 + n].contiguous()).cpu().numpy()
         assert np.array_equal(part, whole[t0:t0 + n]), f"{n} tokens from {t0}"
+
+
+@pytest.mark.parametrize("T", [5, 70])
+def test_prefill_split_x_int8_act(ops, T):
+    """Q4_K experts beside a Q6_K shared gate/up: x in the split form, act in the int8 form, gate/up and down in one launch.
+    Against the decode path of the same layer (other sums of the same products: the chain bounds)."""
+    from tests.helpers import assert_close_chain
+    E, K, H, F = 16, 4, 512, 768
+    rng = np.random.default_rng(40 + T)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    mats = [np.stack([weights(orc.Q4_K, r, c, 10 * k + e).reshape(-1) for e in range(E)])
+            for k, (r, c) in enumerate([(F, H), (F, H), (H, F)])]
+    shexp = {"gate": dev(weights(orc.Q6_K, 256, H, 91)), "up": dev(weights(orc.Q6_K, 256, H, 92)),
+             "down": dev(weights(orc.Q4_K, H, 256, 93)), "inter": 256, "gu_type": orc.Q6_K, "down_type": orc.Q4_K}
+    layer = ops.MoeLayer(dev(gaussian(rng, (E, H), 0.05)), ops.ExpertSlots.from_tensors(*(torch.from_numpy(m) for m in mats)),
+                         orc.Q4_K, orc.Q4_K, H, F, K, shexp=shexp)
+    pre, x = ops.MoePrefill(layer), dev(gaussian(rng, (T, H)))
+    ws, ws1 = pre.workspace(T), layer.workspace(1)
+    out = pre(x, ws=ws).cpu().numpy()
+    assert pre.status(ws, T) == 0
+    one = np.stack([layer(x[t:t + 1].contiguous(), ws=ws1).cpu().numpy()[0] for t in range(T)])
+    assert_close_chain(out, one, f"{T} tokens")
 
 
 @pytest.mark.parametrize("bf16", [False, True])
