@@ -20,7 +20,7 @@ The JSON line also carries:
   cpu_baseline - the oracle's OpenMP CPU restatement of the same layer (int8 x K-quant dot products, not ggml), timed
                  on this host's cores on a bounded sample.
   extra        - configs 1 (Q3_K/Q5_K mix), 2 (4-token speculative verify), 3 (48-layer Q4_K/Q6_K stack) and 4
-                 (512-token prefill through the f16-MFMA split-operand grouped GEMM, Dirichlet(0.3)-skewed router bias; MFMA
+                 (512-token prefill through the grouped GEMM on int8 MFMA, Dirichlet(0.3)-skewed router bias; MFMA
                  utilisation = 38.65 G int8 ops per layer / time / 5.0 POP/s dense int8 peak), the reference
                  model's whole MoE block (RMSNorm, 256 experts top-6 sigmoid, width 512, shared expert) at decode with
                  K-quant and with IQ3_XXS / IQ3_S gate/up + IQ4_XS down experts, and its dense FFN block (2048 ->
@@ -311,9 +311,7 @@ def run_prefill(torch, synth, n_layers: int = 4, T: int = 512, replays: int = 10
             "max_expert_load": max_load, "row_groups": groups, "tile_fill": round(T * K_TOP / (32 * tiles), 3),
             "weight_gbs": round(touched * expert_bytes(Q4_K, Q4_K) / (us * 1e-6) / 1e9, 1),
             "int8_tops": round(ops_per_layer / (us * 1e-6) / 1e12, 2),
-            "mfma_util": round(ops_per_layer / (us * 1e-6) / 5.0e15, 4),
-            # the split-operand GEMM issues every product twice (hi and lo halves) on the 2.5 PFLOP/s f16 pipe
-            "f16_pipe_util": round(2 * ops_per_layer / (us * 1e-6) / 2.5e15, 4)}
+            "mfma_util": round(ops_per_layer / (us * 1e-6) / 5.0e15, 4)}
 
 
 def run_dropin(torch, layers, replays: int = 40) -> dict:

@@ -3,16 +3,18 @@
 // epilogues and weight fragments it shares.
 //
 // Per sub-block s the MFMA gives the exact integer dot I of 32 codes; the output takes I * (d8[token] * dw[row]) with
-// dw = the row's sub-block scale (block d times the integer scale, exact in fp32 for a 6-bit scale): convert, scale
-// product and fma, 48 VALU instructions per 32x32x32 step against one 32-cycle MFMA, so the kernel is bound by VALU
-// issue, 192 cycles a step. The f16 form spends four MFMAs (128 cycles; eight for Q8_0 and IQ4_XS, whose operands are
+// dw = the row's sub-block scale (block d times the integer scale, exact in fp32). The scale product d8 dw is rounded to fp32
+// once per sub-block (relative 2^-24; exact for Q8_0). Convert, scale product and fma are 48 VALU instructions per 32x32x32
+// step against one 32-cycle MFMA, decode, addresses and waits about 6 more, so the kernel is bound by VALU issue: at 4096
+// tokens (Q4_K gate/up) 54.5 instructions of 4 cycles in 234 cycles a step, 93 % of the launch, the matrix pipe busy for
+// 14 %. The f16 form spends four MFMAs (128 cycles; eight for Q8_0 and IQ4_XS, whose operands are
 // split in two) plus the B decode on the same step, and its activations are 4.125 bytes a value against 1.25 here: less
 // than a third of the LDS-DMA traffic, one barrier instead of two, and no f16 decode of the codes.
 // Measured against the f16 form (us): Q8_0 dense block (2048 / 6144) of 512 tokens 251 -> 140, of 40 tokens 173 -> 62; Q4_K
 // gate/up of 4096 tokens to 8 of 128 experts 452 -> 400; Q4_K dense block of 2048 tokens 343 -> 275. Tried and slower:
 // scales fetched a sub-block ahead (spills: a Q8_0 block 140 -> 167), v_dot4 for groups of at most 8 rows (512 tokens
 // 150 -> 175, an LDS round trip per row and sub-block), the f16 codes with d8 applied after each sub-block (418-449
-// against 400).
+// against 400). Registers: 216 to 252, Q8_0 256 with 6 (GLU) and 14 (plain) spilled.
 #pragma once
 
 namespace fns {
@@ -116,7 +118,8 @@ template <int T> __device__ __forceinline__ float i8_scale(const I8Frag<T> &f, i
 
 // ---- one group ----------------------------------------------------------------------------------------------------
 // LDS: the superblock's codes [rows][256] and scales [8][rows], double-buffered (the 16-byte pieces of row r at piece
-// p ^ (r % 16), so an operand read touches distinct banks), and its min-term sums. 40 KB for 64 rows.
+// p ^ (r % 16), so an operand read touches distinct banks), and its min-term sums. 43.5 KB for 64 rows (39.4 without the
+// sums, 1 or 2 KB more with a codebook); the registers allow two workgroups per CU.
 constexpr int kI8Buf = kMmqTok * kActRow * 4;  // a code buffer, sized for the GLU epilogue's act tile (17 KB)
 struct MmqI8Lds {
     uint8_t (&q0)[kI8Buf];

@@ -1261,7 +1261,7 @@ __device__ __forceinline__ void mmq_group(const MmqArgs &a, int g, int wb, const
     MMQ_MARK(12);
 }
 
-// One launch runs both lists, the 64-row groups first (g < n_main) and then the experts' <= 32-row remainders, so the
+// One launch runs both lists, the 64-row groups first and then the experts' <= 32-row remainders, so the
 // smaller workgroups fill the machine while the last large ones finish. The grid is one-dimensional and XCD-aware:
 // workgroup L runs on XCD L % 8 (the hardware's round-robin dispatch), and the n_cb weight row blocks of a group are
 // consecutive items of one XCD, so the group's activation rows are fetched into that XCD's L2 once, not once per
@@ -1701,7 +1701,8 @@ int expert_args(int type, const char *const *table, size_t off_a, size_t off_b, 
 
 // Q8_0 (the reference's dense and output-head type, src/ggml/ggml_mmq.cu:59) takes the int8 form of the GEMM, and for
 // row counts that are not a multiple of 64 the GEMV kernels, a few token columns per weight pass. The K-quants and IQ
-// types keep the split image in the caller's scratch.
+// types read the split image here and in mmq_experts; nothing in these calls forbids the int8 form, which has not been
+// measured for them.
 int mmq(int type, const void *w, int64_t ncols, int64_t nrows, const float *x, int64_t n_tok, void *xq, float *dst,
         hipStream_t st) {
     if (type == T_Q8_0 && nrows % kMmqRows) {  // the GEMV kernels (any row count), a few token columns per pass
@@ -1793,7 +1794,7 @@ void prefill_sizes(const FnsMoeLayer *L, int64_t T, size_t *sz) {
     sz[10] = (size_t) P * 4;                              // escale
     const int64_t fs = L->shexp_inter > 0 ? L->shexp_inter : 0;
     sz[11] = L->ffn_norm ? (size_t) T * L->hidden * 4 : 0;                         // RMSNorm output h
-    sz[12] = L->ffn_norm ? (size_t) T * host::q8_1_row_bytes(L->hidden) : 0;      // its Q8_1 blocks (unused)
+    sz[12] = L->ffn_norm ? (size_t) T * host::q8_1_row_bytes(L->hidden) : 0;      // its Q8_1 blocks (for inspection)
     sz[13] = fs ? (size_t) T * mmq_image_bytes(fs) : 0;                            // shared-expert act images
     sz[14] = fs ? (size_t) T * L->hidden * 4 : 0;                                  // shared-expert output
 }
