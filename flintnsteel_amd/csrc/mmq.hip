@@ -424,6 +424,7 @@ struct MmqShared {
     int64_t out_img;
     int out_form;
     int n_cb, items;           // launch: row blocks per group; workgroups of the grid it takes (a multiple of kXcds)
+    int may_halve;             // launch (with or without such a matrix): the device looks whether it runs in halves
 };
 
 // Weight fragments of one 256-value block for one lane: the header (scales, d) and the codes of column groups
@@ -1295,16 +1296,15 @@ template <bool I8>
 __device__ __forceinline__ bool mmq_item(const MmqArgs &m, const MmqShared &sh, MmqArgs &a, int &g, int &wb, bool &one) {
     a = m;
     a.half = -1;
-    int nm = 0, nr = 0, sh_items = sh.items;
+    int nm, nr, sh_items = sh.items;
     bool halves = false;
-    if (m.bounds) {
-        // expert path: the groups that exist in this call (the device-side counts of the 64-row list and of the
-        // remainder list) take the first workgroups; the rest of the grid (sized for the upper bound) returns at once
-        nm = m.gprefix[m.n_expert], nr = m.gprefix[2 * (m.n_expert + 1) - 1];
-        if constexpr (I8) {
-            halves = (2 * nm + nr) * m.n_cb + groups32(sh.n_rows) * sh.n_cb <= kHalvesMax;
-            if (halves) sh_items = xcd_items(groups32(sh.n_rows), sh.n_cb);
-        }
+    // expert path: the groups that exist in this call (the device-side counts of the 64-row list and of the remainder
+    // list) take the first workgroups; the rest of the grid (sized for the upper bound) returns at once
+    auto counts = [&] { nm = m.gprefix[m.n_expert], nr = m.gprefix[2 * (m.n_expert + 1) - 1]; };
+    if (I8 && sh.may_halve) {
+        counts();
+        halves = (2 * nm + nr) * m.n_cb + groups32(sh.n_rows) * sh.n_cb <= kHalvesMax;
+        if (halves) sh_items = xcd_items(groups32(sh.n_rows), sh.n_cb);
     }
     const bool shared = (int) blockIdx.x < sh_items;
     const int lid = shared ? (int) blockIdx.x : (int) blockIdx.x - sh_items, r = lid / kXcds;
@@ -1337,6 +1337,7 @@ __device__ __forceinline__ bool mmq_item(const MmqArgs &m, const MmqShared &sh, 
         one = sh.n_rows - kMmqTok * j <= kMmqTok / 2;
         if (one) g = 2 * j;
     } else if (m.bounds) {
+        if (!(I8 && sh.may_halve)) counts();
         if (j >= (halves ? 2 * nm : nm) + nr) return false;
         list_item(j, nm, halves, g, a.half, one);
     } else {
@@ -1530,8 +1531,12 @@ int launch_mmq(int type, bool glu, const MmqArgs &a, int groups, hipStream_t st,
     arg.rows_first = form != kImgSplit && !a.bounds && (arg.n_cb % kXcds == 0 || arg.n_cb >= 4 * kXcds);
     int64_t items = sh_items + (arg.rows_first ? (int64_t) total * kXcds * ((arg.n_cb + kXcds - 1) / kXcds)
                                                : (int64_t) arg.n_cb * kXcds * ((total + kXcds - 1) / kXcds));
+    // Halves where the rows allow them (an item takes at most 32 of the more than 64 (groups - n_expert - 1) rows), so that
+    // the first workgroups of a larger launch, the shared expert's, need not wait for the counts (1021-token block: 1 us).
     const int sh32 = groups32(shared.n_rows);
-    if (form == kImgI8 && a.bounds && sh32 * shared.n_cb <= kHalvesMax)  // room for the halves
+    shared.may_halve = form == kImgI8 && a.bounds &&
+                       (int64_t) std::max(1, 2 * (groups - a.n_expert) - 1) * arg.n_cb + sh32 * shared.n_cb <= kHalvesMax;
+    if (shared.may_halve)
         items = std::max<int64_t>(items, xcd_items(sh32, shared.n_cb) + halves_items(total, arg.n_cb));
     if (items > INT32_MAX) return host::set_error(host::ERR_SHAPE, "mmq: grid too large");
     shared.items = (int) sh_items;
